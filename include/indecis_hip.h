@@ -184,7 +184,10 @@ int ixh_model_set_rope(ixh_model *m, int is_global, const float *cos_t,
 /* Kernel and pass choices of a model handle (no counterpart in the
  * reference, whose only knob is the worker count, linalg.SetWorkers).
  * Results never depend on them (the tests check every choice against the
- * oracle); they only move time. Each call reads the handle's values once. */
+ * oracle); they only move time. Each call reads the handle's values once.
+ * Setting a kernel option (any but PARTS and PASS_TOKENS, to any value)
+ * fixes the options' kernels for every batch size; until then batches of
+ * few rows take kernels of their own. */
 enum {
   IXH_OPT_PARTS = 0,       /* streams a large batch is split over: 0 auto (default), 1..4 */
   IXH_OPT_PASS_TOKENS = 1, /* most tokens of one pass, 1..131072 (default): larger

@@ -30,10 +30,12 @@ int set_tuning(Tuning &t, int option, int64_t v, bool model_opts) {
   case IXH_OPT_GEMM:
     if (v < 0 || v > 2) return bad();
     t.gemm = (int)v;
+    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_GEMM_TILE:
     if (v < 0 || v > 2) return bad();
     t.gemm_tile = (int)v;
+    t.fixed = true;
     return IXH_OK;
   default: break;
   }
@@ -50,26 +52,32 @@ int set_tuning(Tuning &t, int option, int64_t v, bool model_opts) {
   case IXH_OPT_QKV_FUSED:
     if (v != 0 && v != 1) return bad();
     t.qkv_fused = (int)v;
+    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_QKV_HEADS:
     if (v != 1 && v != 2) return bad();
     t.qkv_heads = (int)v;
+    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_LN_SEG:
     if (v != 0 && v != 1) return bad();
     t.ln_seg = (int)v;
+    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_FUSE_RES:
     if (v < 0 || v > 4) return bad();
     t.fuse_res = (int)v;
+    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_FUSE_MLP:
     if (v < 0 || v > 2) return bad();
     t.fuse_mlp = (int)v;
+    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_QKV_KBLOCK:
     if (v != 0 && v != 1) return bad();
     t.qkv_kblock = (int)v;
+    t.fixed = true;
     return IXH_OK;
   default: return fail(IXH_EINVAL, "indecis: unknown option %d", option);
   }

@@ -35,6 +35,9 @@ struct Tuning {
   int fuse_mlp = 2;       // the MLP block (Wi, GeGLU, quantizeA, WoMLP, next LN) as one kernel:
                           // 2 mlp_block (64 rows, transposed), 1 mlp_res (32 rows), 0 separate
   int qkv_kblock = 1;     // the fused QKV kernel reads its input rows K-blocked (1) or row-major (0)
+  // a kernel option was set: the options' kernels at every batch size
+  // (unset, batches of few rows take kernels of their own)
+  bool fixed = false;
 };
 
 // Upper bound of Tuning::pass_tokens.

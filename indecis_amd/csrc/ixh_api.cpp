@@ -511,6 +511,14 @@ int split_parts(const Tuning &t, int N, int B, int H) {
   return 2;
 }
 
+// Most rows of a pass whose Wo and MLP run cut by output channel
+// (split_rows.hip). Past it each tile's workgroups read the float32 input
+// rows too many times over: sequences of 128 tokens, a pass on the whole-row
+// kernels over one on these, measured 2.05 at 128 rows, 1.45 at 1,024, 1.14
+// at 1,536, 0.93 at 2,048 (hidden 768; hidden 384: 1.81, 1.39, 1.18, 1.01;
+// hidden 256: 1.26, 1.16, 1.12, 1.10).
+constexpr int kSplitRowsMax = 1536;
+
 // What a forward pass issued but has not waited for: its profiling records
 // and the RoPE tables its kernels read.
 struct Pending {
@@ -575,10 +583,13 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
                          mlp_block_supported(H, I, KpH, KpI, m->layers[0].i.np);
   const bool fuse_mlp = mlp_block || (mlp_common && fuse_res && tune.fuse_mlp != 0 &&
                                       mlp_res_supported(H, I, KpH, KpI, m->layers[0].i.np));
+  // few rows: Wo and the MLP cut by output channel (split_rows.hip)
+  const bool split = !tune.fixed && N <= kSplitRowsMax && split_rows_supported(H, I, KpH, KpI) &&
+                     m->layers[0].o.qk.p && mlp_common;
   // the fused QKV kernel's input rows K-blocked (the weight rows then stay
   // in LDS): written so by the embedding LayerNorm and by the MLP kernel of
   // each layer
-  const bool kblock = fused && fuse_mlp && tune.qkv_kblock != 0 && qkv_kblock_supported(KpH) &&
+  const bool kblock = fused && (fuse_mlp || split) && tune.qkv_kblock != 0 && qkv_kblock_supported(KpH) &&
                       m->layers[0].qkv.qk.p;
 
   int rc;
@@ -586,14 +597,14 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   if ((rc = w->tabs.ensure(4 * ntab)) || (rc = w->pos.ensure(4 * (size_t)N)) ||
       (rc = w->x.ensure(4 * (size_t)N * H)) || (rc = w->xn.ensure(4 * (size_t)N * H)) ||
       (!fused && (rc = w->qkv.ensure(4 * (size_t)N * 3 * H))) || (rc = w->xq.ensure((size_t)N * ldq)) ||
-      (kblock && (rc = w->xqk.ensure((size_t)N * KpH))) ||
+      ((kblock || split) && (rc = w->xqk.ensure((size_t)N * KpH))) ||
       (rc = w->sa.ensure(4 * (size_t)N)) || (rc = w->qq.ensure((size_t)N * H)) ||
       (rc = w->sq.ensure(4 * (size_t)N * nh)) || (rc = w->kp.ensure((size_t)nh * Npad * D)) ||
       (rc = w->ks.ensure(4 * (size_t)nh * Npad)) || (rc = w->vt.ensure((size_t)nh * D * Npad)) ||
       (rc = w->vs.ensure(3 * 4 * (size_t)B * nh * D)) || (rc = w->ctx.ensure(4 * (size_t)N * H)) ||
-      (!fuse_mlp && (rc = w->g.ensure(4 * (size_t)N * I))) ||
-      (stream_ctx && (rc = w->cmax.ensure(4 * (size_t)N * nh))) ||
-      (stream_ctx && (rc = w->gmax.ensure(4 * (size_t)N * (I / 32)))))
+      ((!fuse_mlp || split) && (rc = w->g.ensure(4 * (size_t)N * I))) ||
+      ((stream_ctx || split) && (rc = w->cmax.ensure(4 * (size_t)N * nh))) ||
+      ((stream_ctx || split) && (rc = w->gmax.ensure(4 * (size_t)N * (I / 32)))))
     return rc;
 
   // small host-built tables through pinned memory, one copy
@@ -747,7 +758,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   ln.seg = tune.ln_seg;
   const double ln_bytes = dN * (4 * dH + dH + 4);
 
-  float *const cmax = stream_ctx ? w->cmax.as<float>() : nullptr;
+  float *const cmax = stream_ctx || split ? w->cmax.as<float>() : nullptr;
   aa.rmax = cmax;
   // the GeGLU maxima exist only where Wi runs on gemm_as (which writes them)
   float *gmax = nullptr;
@@ -823,6 +834,57 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
     const double pairs = global ? keys_global : keys_local;
     RUN(global ? "attn_global" : "attn_local", 4.0 * D * nh * pairs,
         dN * 3 * dH + 8 * dN * nh + dN * dH * 4, launch_attn_main(aa, st));
+    if (split) {
+      // x += ctx . Wo^T (infer.go:403), mlp_norm (infer.go:404-407), Wi +
+      // GeGLU, x += g . WoMLP^T (infer.go:408-424), the next attn_norm
+      auto product = [&](const Mat &M, const float *A, int K, float *rmax, int P, float *C, int ldc, int n) {
+        SplitArgs r{};
+        r.A = A;
+        r.lda = K;
+        r.Ak = w->xqk.as<int8_t>();
+        r.ak_rows = N;
+        r.sa = w->sa.as<float>();
+        r.Bk = M.qk.as<int8_t>();
+        r.Np = M.np;
+        r.n = n;
+        r.K = K;
+        r.sb = M.sb.as<float>();
+        r.zc = M.zc.as<float>();
+        r.c128 = M.c128.as<int32_t>();
+        r.small = M.small;
+        r.C = C;
+        r.ldc = ldc;
+        r.rmax = rmax;
+        r.P = P;
+        r.M = N;
+        return r;
+      };
+      LnRowsArgs lr{};
+      lr.x = w->x.as<float>();
+      lr.M = N;
+      lr.H = H;
+      lr.gamma = L.mlp_norm.as<float>();
+      lr.eps = c.norm_eps;
+      lr.qk = w->xqk.as<int8_t>();
+      lr.sa = w->sa.as<float>();
+      RUN("gemm_wo", 2 * dN * dH * dH, res_bytes(dH, false),
+          launch_res_split(product(L.o, w->ctx.as<float>(), H, cmax, nh, w->x.as<float>(), H, H), st));
+      RUN("ln_quant", 0, ln_bytes, launch_ln_rows(lr, c.lanes, st));
+      float *const gm = w->gmax.as<float>();
+      RUN("gemm_wi", 2 * dN * 2 * dI * dH, gemm_bytes(dH, 2 * dI, dI, false),
+          launch_wi_split(product(L.i, nullptr, H, gm, I / 32, w->g.as<float>(), I, 2 * I), st));
+      RUN("gemm_womlp", 2 * dN * dH * dI, res_bytes(dI, false),
+          launch_res_split(product(L.omlp, w->g.as<float>(), I, gm, I / 32, w->x.as<float>(), H, H), st));
+      if (l + 1 < c.layers) {
+        lr.gamma = m->layers[l + 1].attn_norm.as<float>();
+        lr.qk = kblock ? w->xqk.as<int8_t>() : nullptr;
+        lr.q = kblock ? nullptr : w->xq.as<int8_t>();
+        lr.ldq = KpH;
+        RUN("ln_quant", 0, ln_bytes, launch_ln_rows(lr, c.lanes, st));
+        ln_done = true;
+      }
+      continue;
+    }
     // x += ctx . Wo^T (infer.go:403), then mlp_norm (infer.go:404-407)
     if (wo8) {
       MlpArgs wa{};

@@ -170,6 +170,44 @@ bool launch_mlp_block(const MlpArgs &a, int lanes, hipStream_t s);
 bool wo_res_supported(int H, int KpH, int Np);
 bool launch_wo_res(const MlpArgs &a, int lanes, hipStream_t s);
 
+// The Wo and MLP products of batches of few rows (split_rows.hip): cut into
+// 32-channel tiles over many workgroups, A float32 with the maxima of its
+// rows' parts (res) or int8 K-blocked (wi).
+struct SplitArgs {
+  const float *A;        // res: [M][lda] float32 input rows, K columns
+  int lda;
+  const int8_t *Ak;      // wi: [K/32][ak_rows][32] quantised rows
+  int ak_rows;
+  const float *sa;       // wi: [M] their scales
+  const int8_t *Bk;      // weights K-blocked [K/32][Np][32] (wi: rows interleaved by 32)
+  int Np, n, K;          // its rows a K-block, those of the product, the depth
+  const float *sb, *zc;  // [Np]
+  const int32_t *c128;   // [Np]
+  int small;             // the weights' dequantisation bound holds (GemmArgs::small)
+  float *C;              // wi: g [M][ldc] out; res: x [M][ldc], added to
+  int ldc;
+  float *rmax;           // [M][P] max |A| (res, in) or |g| (wi, out: P = n/64) of the row's parts
+  int P;
+  int M;
+};
+// (H, I) one of (768, 1152), (384, 1152), (256, 512), unpadded
+bool split_rows_supported(int H, int I, int KpH, int KpI);
+void launch_wi_split(const SplitArgs &a, hipStream_t s);
+void launch_res_split(const SplitArgs &a, hipStream_t s);
+// LayerNorm + quantizeA of the rows of x [M][H]: sa [M], and q [M][ldq] or
+// K-blocked qk [H/32][M][32], whichever is not null.
+struct LnRowsArgs {
+  const float *x;
+  int M, H;
+  const float *gamma;
+  double eps;
+  int8_t *q;
+  int ldq;
+  int8_t *qk;
+  float *sa;
+};
+void launch_ln_rows(const LnRowsArgs &a, int lanes, hipStream_t s);
+
 // ---- host helpers (ixh_api.cpp) ---------------------------------------------
 // Sets the calling thread's ixh_last_error message; returns code.
 int set_error(int code, const char *msg);

@@ -1,0 +1,339 @@
+// split_rows.hip — the encoder's Wo and MLP products for batches of few
+// rows: every product cut into 32-channel tiles over many workgroups, its
+// depth over the waves of a workgroup.
+//
+// Replaces, for such batches, the whole-row kernels of gemm_res.hip and
+// mlp_block.hip (infer.go:401-424: MatMul8N of ctx into x, mlp_norm, Wi +
+// GeluMul, MatMul8N of g into x, the next attn_norm), with the same
+// arithmetic: quantizeA of the input rows (int8.go:160-191), q*w summed in
+// int32 by v_mfma_i32_32x32x32_i8, the reference tile's dequantisation
+// ((f32(tile) - zc) * sb) * sa, GELU in the FMA form, the LayerNorm's V
+// float32 lane chains in column order combined in float64 in lane order.
+//
+// Why: a whole-row kernel gives 32 or 64 rows to one workgroup, which then
+// streams every weight of the block through one CU; one row costs it as
+// much as 64, and a batch of 24 rows ran on one CU of 256. Cut by output
+// channel, a weight byte is read by one workgroup per 32 rows, and the
+// chip's CUs read different weights.
+//
+//  res_split_kernel  x[:, tile] += quantizeA(A) . W^T tile: one workgroup
+//      per (32 rows, 32 output channels), 4 waves, each a quarter of the
+//      depth. A (ctx or g, float32) is quantised into an LDS panel from the
+//      row maxima its producer wrote (attention per head, wi_split per 32
+//      columns), so no pass over the row comes before the product.
+//  wi_split_kernel   g tile = GeGLU(xn . Wi^T): one workgroup per (32 rows,
+//      gated tile of 32 columns), 4 waves over the depth; also max |g| of
+//      each row's 32 columns.
+//  ln_rows_kernel    LayerNorm + quantizeA of 8 rows a workgroup.
+//
+// What bounds them: latency. At 24 rows of hidden 768 (36 and 24 workgroups)
+// a launch takes 4.9 us (Wi), 5.1 us (Wo) and 6.4 us (WoMLP), LayerNorm 4.8
+// us: against 25 us (Wo + LayerNorm) and 50 us (the MLP block) on the
+// whole-row kernels, and 2.05 -> 0.93 ms a pass of 22 layers. Every global
+// load of a wave is in flight before its first use.
+//
+// The products are transposed as in mlp_block.hip (weights the A operand,
+// rows the B operand): a lane holds one row and 16 consecutive channels,
+// so results leave as float4.
+#include <type_traits>
+
+#include "ixh_device.h"
+#include "ixh_internal.h"
+
+namespace ixh {
+
+namespace {
+
+constexpr int NXCD = 8;
+constexpr int WAVES = 4;  // of a workgroup, sharing a tile's depth
+
+// the weight row that lane row i loads, so that accumulator r of a lane is
+// channel 16*(lane/32) + r of the tile (mlp_block.hip)
+__device__ __forceinline__ int perm32(int i) { return 16 * ((i >> 2) & 1) + 4 * (i >> 3) + (i & 3); }
+
+__device__ __forceinline__ int pack4(const float4 v, float inv) {
+  return (q8(v.x, inv) & 0xff) | ((q8(v.y, inv) & 0xff) << 8) | ((q8(v.z, inv) & 0xff) << 16) | (q8(v.w, inv) << 24);
+}
+
+// Workgroup -> (tile, row block): workgroup L runs on XCD L % 8, and the
+// row blocks of one tile go to one XCD, so that its L2 reads the tile's
+// weights once. False past the last tile.
+__device__ __forceinline__ bool tile_of(int ntiles, int nblk, int *tile, int *blk) {
+  const int i = blockIdx.x / NXCD;
+  *tile = (int)(blockIdx.x % NXCD) + NXCD * (i / nblk);
+  *blk = i % nblk;
+  return *tile < ntiles;
+}
+int tile_grid(int ntiles, int nblk) { return NXCD * ((ntiles + NXCD - 1) / NXCD) * nblk; }
+
+// The waves' partial sums meet in LDS: wave w gets accumulators 4w .. 4w+3
+// of the whole depth. part: [WAVES][4][64] int4, acc's 4 accumulator groups.
+__device__ __forceinline__ int4 gather_sums(const int4 *part, int wave, int lane) {
+  int4 s = part[(0 * 4 + wave) * 64 + lane];
+#pragma unroll
+  for (int w = 1; w < WAVES; w++) {
+    const int4 t = part[(w * 4 + wave) * 64 + lane];
+    s = int4{s.x + t.x, s.y + t.y, s.z + t.z, s.w + t.w};
+  }
+  return s;
+}
+__device__ __forceinline__ void put_sums(int4 *part, int wave, int lane, const v16i &acc) {
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    part[(wave * 4 + q) * 64 + lane] = int4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+}
+
+// ((f32(acc + 128 colsum) - zc) * sb) * sa of four channels; small: the
+// weights' bound holds and f32(acc + 128 colsum) - zc is f32(acc)
+__device__ __forceinline__ float4 deq4(int4 t, bool small, const int32_t *c128, const float *zc, float4 sb, float sa) {
+  if (small)
+    return make_float4(((float)t.x * sb.x) * sa, ((float)t.y * sb.y) * sa, ((float)t.z * sb.z) * sa,
+                       ((float)t.w * sb.w) * sa);
+  const int4 c = *(const int4 *)c128;
+  const float4 z = *(const float4 *)zc;
+  return make_float4(deq(t.x + c.x, z.x, sb.x, sa), deq(t.y + c.y, z.y, sb.y, sa), deq(t.z + c.z, z.z, sb.z, sa),
+                     deq(t.w + c.w, z.w, sb.w, sa));
+}
+
+template <int KT>
+__global__ __launch_bounds__(256) void wi_split_kernel(SplitArgs a) {
+  constexpr int KW = KT / WAVES;  // K steps of a wave
+  static_assert(KT % WAVES == 0, "depth over the waves");
+  __shared__ int4 part[2][WAVES * 4 * 64];
+  __shared__ float mx_s[WAVES][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 31, fh = lane >> 5;
+  int t, blk;
+  if (!tile_of(a.n / 64, (a.M + 31) / 32, &t, &blk)) return;
+  const int m0 = 32 * blk, row = min(m0 + fr, a.M - 1);  // rows past M: row M-1, never stored
+  // every load of the wave in flight at once
+  v4i w[KW][2], x[KW];
+  const int8_t *wp = a.Bk + ((size_t)(wave * KW) * a.Np + 64 * t + perm32(fr)) * 32 + 16 * fh;
+  const int8_t *xp = a.Ak + ((size_t)(wave * KW) * a.ak_rows + row) * 32 + 16 * fh;
+#pragma unroll
+  for (int k = 0; k < KW; k++) {
+    x[k] = *(const v4i *)(xp + (size_t)k * a.ak_rows * 32);
+    w[k][0] = *(const v4i *)(wp + (size_t)k * a.Np * 32);
+    w[k][1] = *(const v4i *)(wp + (size_t)k * a.Np * 32 + 1024);
+  }
+  const float sa = a.sa[row];
+  const int ch = 64 * t + 16 * fh + 4 * wave;  // this lane's GELU-input channels (the multiplier's: + 32)
+  const float4 sba = *(const float4 *)(a.sb + ch), sbb = *(const float4 *)(a.sb + ch + 32);
+  v16i acc[2] = {};
+#pragma unroll
+  for (int k = 0; k < KW; k++) {
+    acc[0] = mfma32(w[k][0], x[k], acc[0]);
+    acc[1] = mfma32(w[k][1], x[k], acc[1]);
+  }
+  put_sums(part[0], wave, lane, acc[0]);
+  put_sums(part[1], wave, lane, acc[1]);
+  __syncthreads();
+  const float4 za = deq4(gather_sums(part[0], wave, lane), a.small, a.c128 + ch, a.zc + ch, sba, sa);
+  const float4 zb = deq4(gather_sums(part[1], wave, lane), a.small, a.c128 + ch + 32, a.zc + ch + 32, sbb, sa);
+  const float4 g = make_float4(gelu_fma(za.x) * zb.x, gelu_fma(za.y) * zb.y, gelu_fma(za.z) * zb.z, gelu_fma(za.w) * zb.w);
+  if (m0 + fr < a.M) *(float4 *)(a.C + (size_t)(m0 + fr) * a.ldc + 32 * t + 16 * fh + 4 * wave) = g;
+  mx_s[wave][lane] = amax(amax(amax(amax(0.f, g.x), g.y), g.z), g.w);
+  __syncthreads();
+  if (tid < 32 && m0 + tid < a.M) {
+    float m = 0.f;
+#pragma unroll
+    for (int q = 0; q < WAVES; q++) m = __builtin_fmaxf(__builtin_fmaxf(m, mx_s[q][tid]), mx_s[q][32 + tid]);
+    a.rmax[(size_t)(m0 + tid) * a.P + t] = m;
+  }
+}
+
+template <int KT>
+__global__ __launch_bounds__(256) void res_split_kernel(SplitArgs a) {
+  constexpr int KW = KT / WAVES;
+  static_assert(KT % WAVES == 0, "depth over the waves");
+  __shared__ __attribute__((aligned(16))) int8_t panel[KT * 1024];  // [KT][64 lanes][16]
+  __shared__ int4 part[WAVES * 4 * 64];
+  __shared__ float sa_s[32];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 31, fh = lane >> 5;
+  int t, blk;
+  if (!tile_of(a.n / 32, (a.M + 31) / 32, &t, &blk)) return;
+  const int m0 = 32 * blk;
+  // the row's maxima and its values: 8 threads a row, 32 columns a step
+  const int tr = tid >> 3, j = tid & 7;
+  const int arow = min(m0 + tr, a.M - 1);  // rows past M: row M-1, never stored
+  float mx = 0.f;
+  for (int p = j; p < a.P; p += 8) mx = __builtin_fmaxf(mx, a.rmax[(size_t)arow * a.P + p]);
+  float4 v[KT];
+  const float *ap = a.A + (size_t)arow * a.lda + 4 * j;
+#pragma unroll
+  for (int k = 0; k < KT; k++) v[k] = *(const float4 *)(ap + 32 * k);
+  v4i w[KW];
+  const int8_t *wp = a.Bk + ((size_t)(wave * KW) * a.Np + 32 * t + perm32(fr)) * 32 + 16 * fh;
+#pragma unroll
+  for (int k = 0; k < KW; k++) w[k] = *(const v4i *)(wp + (size_t)k * a.Np * 32);
+  const int ch = 32 * t + 16 * fh + 4 * wave;
+  const float4 sb = *(const float4 *)(a.sb + ch);
+  float *const xp = a.C + (size_t)min(m0 + fr, a.M - 1) * a.ldc + ch;
+  float4 x = *(const float4 *)xp;
+#pragma unroll
+  for (int o = 1; o < 8; o <<= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, o));
+  float s = 0.f, inv = 0.f;
+  if (mx != 0.f) {  // quantizeA: s = max/127, inv = 1/s (int8.go:175-183)
+    s = mx / 127.0f;
+    inv = 1.0f / s;
+  }
+  if (j == 0) sa_s[tr] = s;
+  int8_t *pp = panel + (tr + 32 * (j >> 2)) * 16 + 4 * (j & 3);
+#pragma unroll
+  for (int k = 0; k < KT; k++) *(int *)(pp + 1024 * k) = pack4(v[k], inv);
+  __syncthreads();
+  v16i acc = {};
+#pragma unroll
+  for (int k = 0; k < KW; k++) acc = mfma32(w[k], *(const v4i *)(panel + 1024 * (wave * KW + k) + 16 * lane), acc);
+  put_sums(part, wave, lane, acc);
+  __syncthreads();
+  const float4 d = deq4(gather_sums(part, wave, lane), a.small, a.c128 + ch, a.zc + ch, sb, sa_s[fr]);
+  x = make_float4(x.x + d.x, x.y + d.y, x.z + d.z, x.w + d.w);
+  if (m0 + fr < a.M) *(float4 *)xp = x;
+}
+
+// LayerNorm (vec_simd.go:285-327) and quantizeA of ROWS rows a workgroup:
+// 32 threads a row hold its values in registers, the lane chains run over
+// a copy in LDS.
+template <int H, int V>
+__global__ __launch_bounds__(256) void ln_rows_kernel(LnRowsArgs a) {
+  constexpr int ROWS = 8, LD = H + 8;  // floats a row in LDS
+  constexpr int C4 = H / 128;          // float4 a thread
+  __shared__ __attribute__((aligned(16))) float xs[ROWS * LD];
+  __shared__ float mean_s[ROWS], rstd_s[ROWS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int r = tid >> 5, c = tid & 31, m0 = ROWS * blockIdx.x;
+  const int row = min(m0 + r, a.M - 1);
+  float4 v[C4], g[C4];
+#pragma unroll
+  for (int u = 0; u < C4; u++) v[u] = *(const float4 *)(a.x + (size_t)row * H + 4 * (c + 32 * u));
+#pragma unroll
+  for (int u = 0; u < C4; u++) g[u] = *(const float4 *)(a.gamma + 4 * (c + 32 * u));
+#pragma unroll
+  for (int u = 0; u < C4; u++) *(float4 *)&xs[r * LD + 4 * (c + 32 * u)] = v[u];
+  __syncthreads();
+  // chain ch: lane partial ch % V of row ch / V (V 0: one float64 chain a row)
+  constexpr int NCH = V > 0 ? ROWS * V : ROWS;
+  if (tid < (NCH + 63) / 64 * 64) {
+    const int ch = min(tid, NCH - 1), cr = V > 0 ? ch / (V > 0 ? V : 1) : ch;
+    float mean = 0.f;
+#pragma unroll
+    for (int pass = 0; pass < 2; pass++) {
+      double sum = 0.0;
+      if constexpr (V > 0) {
+        const float *xr = xs + cr * LD + ch % V;
+        constexpr int NE = H / V, NB = NE < 16 ? NE : 16;
+        float p = 0.f, b[NB], n[NB];
+#pragma unroll
+        for (int e = 0; e < NB; e++) b[e] = xr[V * e];
+#pragma unroll
+        for (int e0 = 0; e0 < NE; e0 += NB) {
+          if (e0 + NB < NE) {
+#pragma unroll
+            for (int e = 0; e < NB; e++) n[e] = xr[V * (e0 + NB + e)];
+          }
+#pragma unroll
+          for (int e = 0; e < NB; e++) {
+            if (pass == 0) {
+              p = p + b[e];
+            } else {
+              const float d = b[e] - mean;
+              p = __builtin_fmaf(d, d, p);
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < NB; e++) b[e] = n[e];
+        }
+        const int base = lane & ~(V - 1);
+#pragma unroll
+        for (int q = 0; q < V; q++) sum += (double)__shfl(p, base + q);
+      } else {
+        const float *xr = xs + cr * LD;
+        for (int e = 0; e < H; e++) {
+          if (pass == 0) {
+            sum += (double)xr[e];
+          } else {
+            const double d = (double)(xr[e] - mean);
+            sum += d * d;
+          }
+        }
+      }
+      if (pass == 0) {
+        mean = (float)(sum / (double)H);
+      } else if (tid < NCH && (V == 0 || tid % (V > 0 ? V : 1) == 0)) {
+        mean_s[cr] = mean;
+        rstd_s[cr] = (float)(1.0 / __builtin_sqrt(sum / (double)H + a.eps));
+      }
+    }
+  }
+  __syncthreads();
+  const float mean = mean_s[r], rstd = rstd_s[r];
+  float mx = 0.f;
+#pragma unroll
+  for (int u = 0; u < C4; u++) {
+    v[u] = make_float4(((v[u].x - mean) * rstd) * g[u].x, ((v[u].y - mean) * rstd) * g[u].y,
+                       ((v[u].z - mean) * rstd) * g[u].z, ((v[u].w - mean) * rstd) * g[u].w);
+    mx = amax(amax(amax(amax(mx, v[u].x), v[u].y), v[u].z), v[u].w);
+  }
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, o));
+  float s = 0.f, inv = 0.f;
+  if (mx != 0.f) {
+    s = mx / 127.0f;
+    inv = 1.0f / s;
+  }
+  if (m0 + r >= a.M) return;
+  if (c == 0) a.sa[row] = s;
+#pragma unroll
+  for (int u = 0; u < C4; u++) {
+    const int col = 4 * (c + 32 * u), w = pack4(v[u], inv);
+    if (a.qk) *(int *)(a.qk + ((size_t)(col >> 5) * a.M + row) * 32 + (col & 31)) = w;
+    if (a.q) *(int *)(a.q + (size_t)row * a.ldq + col) = w;
+  }
+}
+
+template <int H>
+void launch_ln(const LnRowsArgs &a, int lanes, hipStream_t s) {
+  const int grid = (a.M + 7) / 8;
+  switch (lanes) {
+  case 0: ln_rows_kernel<H, 0><<<grid, 256, 0, s>>>(a); break;
+  case 4: ln_rows_kernel<H, 4><<<grid, 256, 0, s>>>(a); break;
+  case 8: ln_rows_kernel<H, 8><<<grid, 256, 0, s>>>(a); break;
+  default: ln_rows_kernel<H, 16><<<grid, 256, 0, s>>>(a); break;
+  }
+}
+
+}  // namespace
+
+bool split_rows_supported(int H, int I, int KpH, int KpI) {
+  if (KpH != H || KpI != I) return false;
+  return (H == 768 && I == 1152) || (H == 384 && I == 1152) || (H == 256 && I == 512);
+}
+
+void launch_wi_split(const SplitArgs &a, hipStream_t s) {
+  if (a.M <= 0) return;
+  const int grid = tile_grid(a.n / 64, (a.M + 31) / 32);
+  if (a.K == 768) wi_split_kernel<24><<<grid, 256, 0, s>>>(a);
+  else if (a.K == 384) wi_split_kernel<12><<<grid, 256, 0, s>>>(a);
+  else wi_split_kernel<8><<<grid, 256, 0, s>>>(a);
+}
+
+void launch_res_split(const SplitArgs &a, hipStream_t s) {
+  if (a.M <= 0) return;
+  const int grid = tile_grid(a.n / 32, (a.M + 31) / 32);
+  if (a.K == 1152) res_split_kernel<36><<<grid, 256, 0, s>>>(a);
+  else if (a.K == 768) res_split_kernel<24><<<grid, 256, 0, s>>>(a);
+  else if (a.K == 512) res_split_kernel<16><<<grid, 256, 0, s>>>(a);
+  else if (a.K == 384) res_split_kernel<12><<<grid, 256, 0, s>>>(a);
+  else res_split_kernel<8><<<grid, 256, 0, s>>>(a);
+}
+
+void launch_ln_rows(const LnRowsArgs &a, int lanes, hipStream_t s) {
+  if (a.M <= 0) return;
+  if (a.H == 768) launch_ln<768>(a, lanes, s);
+  else if (a.H == 384) launch_ln<384>(a, lanes, s);
+  else launch_ln<256>(a, lanes, s);
+}
+
+}  // namespace ixh

@@ -1,0 +1,48 @@
+"""GPU parity of the encoder on batches of few rows, whose Wo and MLP
+products run cut by output channel (split_rows.hip), against the CPU
+oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from helpers import base_cfg, bekko_cfg, f32_bits_equal, mismatch_report, small_cfg
+from indecis_amd.modernbert import Model, Weights
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {"small": small_cfg, "base": base_cfg, "bekko": bekko_cfg}
+
+
+def seqs_of(rng, vocab, *lens):
+    return [rng.integers(0, vocab, size=n, dtype=np.int32) for n in lens]
+
+
+# shape, lane width, rows past the dequantisation bound planted in a matrix
+@pytest.mark.parametrize("shape,lanes,plant", [
+    ("base", 8, None), ("base", 16, "wo"), ("base", 0, "womlp"), ("bekko", 8, "wi"), ("bekko", 4, None),
+    ("small", 8, "wo"), ("small", 16, None), ("small", 4, "womlp"), ("small", 0, "wi")])
+def test_few_rows_exact(shape, lanes, plant):
+    """Row counts around the 32-row blocks (and the 8 rows of a LayerNorm
+    workgroup), one sequence or several, a sequence over 512 keys (QKV input
+    row-major), and the two sides of the rule that picks these kernels;
+    setting a kernel option (here to its default) picks the whole-row
+    kernels, and gives the same bits."""
+    cfg = SHAPES[shape](layers=2)
+    w = Weights.random(cfg, seed=97)
+    if plant:
+        {"wi": w.wi_q, "wo": w.wo_q, "womlp": w.womlp_q}[plant][0, 3, :] = 127
+    gpu, ora = Model(w, lanes=lanes), orc.OracleModel(w, lanes=lanes)
+    rng = np.random.default_rng(97)
+    batches = [seqs_of(rng, cfg.vocab, *lens)
+               for lens in ((1,), (7, 1), (31,), (9, 0, 23), (33,), (64, 1, 192), (600, 9))]
+    want = [ora.encode_tokens(b)[0] for b in batches]
+    for b, e in zip(batches, want):
+        got = gpu.encode_tokens(b)
+        assert f32_bits_equal(got, e), ([len(s) for s in b], mismatch_report(got, e))
+    edges = [seqs_of(rng, cfg.vocab, *lens) for lens in ((500, 500, 500, 36), (500, 500, 500, 37))]
+    few = [gpu.encode_tokens(b) for b in batches + edges]
+    gpu.set_option("fuse_mlp", 2)
+    for b, e in zip(batches + edges, few):
+        got = gpu.encode_tokens(b)
+        assert f32_bits_equal(got, e), ([len(s) for s in b], mismatch_report(got, e))
+    gpu.close()
