@@ -512,12 +512,19 @@ int split_parts(const Tuning &t, int N, int B, int H) {
 }
 
 // Most rows of a pass whose Wo and MLP run cut by output channel
-// (split_rows.hip). Past it each tile's workgroups read the float32 input
-// rows too many times over: sequences of 128 tokens, a pass on the whole-row
-// kernels over one on these, measured 2.05 at 128 rows, 1.45 at 1,024, 1.14
-// at 1,536, 0.93 at 2,048 (hidden 768; hidden 384: 1.81, 1.39, 1.18, 1.01;
-// hidden 256: 1.26, 1.16, 1.12, 1.10).
-constexpr int kSplitRowsMax = 1536;
+// (split_rows.hip), by hidden size. Past it the tiles' workgroups read the
+// rows too many times over. Sequences of 128 tokens, a pass with the 64-row
+// MLP kernel (the 32-row one at hidden 768 and 256) over one on these: hidden
+// 768 1.75 (1.49) at 1,024 rows, 1.40 (1.20) at 2,048, 1.17 (1.00) at 3,072,
+// 1.10 (0.94) at 4,096; 384 1.37 at 2,048, 1.08 at 4,096, 0.91 at 6,144; 256
+// 1.20 (1.06) at 2,048, 1.10 (0.98) at 2,560.
+int split_rows_max(int H) { return H == 768 ? 3072 : H == 384 ? 4096 : 2048; }
+// Above that, most rows of a pass whose MLP runs 32 rows a workgroup
+// (mlp_res.hip): one round of the 256 CUs, where 64 rows a workgroup leave
+// half of them idle. Hidden 768: 2.51 against 2.89 ms a pass at 6,144 rows,
+// 2.90 against 3.18 at 8,192 (38 against 52 us a launch); past one round a
+// 32-row block costs as much as a 64-row one.
+constexpr int kMlp32RowsMax = 8192;
 
 // What a forward pass issued but has not waited for: its profiling records
 // and the RoPE tables its kernels read.
@@ -579,12 +586,14 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   const bool mlp_common = m->layers[0].i.qk.p && m->layers[0].omlp.qk.p && gelu_fma_cols(I, c.lanes) == I;
   bool mats_small = true;  // the 64-row kernel dequantises as f32(acc) * sb * sa
   for (int l = 0; l < c.layers; l++) mats_small = mats_small && m->layers[l].i.small && m->layers[l].omlp.small;
-  const bool mlp_block = mlp_common && tune.fuse_mlp == 2 && mats_small &&
+  const bool mlp32 = !tune.fixed && N <= kMlp32RowsMax && mlp_common && fuse_res &&
+                     mlp_res_supported(H, I, KpH, KpI, m->layers[0].i.np);
+  const bool mlp_block = !mlp32 && mlp_common && tune.fuse_mlp == 2 && mats_small &&
                          mlp_block_supported(H, I, KpH, KpI, m->layers[0].i.np);
   const bool fuse_mlp = mlp_block || (mlp_common && fuse_res && tune.fuse_mlp != 0 &&
                                       mlp_res_supported(H, I, KpH, KpI, m->layers[0].i.np));
   // few rows: Wo and the MLP cut by output channel (split_rows.hip)
-  const bool split = !tune.fixed && N <= kSplitRowsMax && split_rows_supported(H, I, KpH, KpI) &&
+  const bool split = !tune.fixed && N <= split_rows_max(H) && split_rows_supported(H, I, KpH, KpI) &&
                      m->layers[0].o.qk.p && mlp_common;
   // the fused QKV kernel's input rows K-blocked (the weight rows then stay
   // in LDS): written so by the embedding LayerNorm and by the MLP kernel of

@@ -17,20 +17,23 @@
 // chip's CUs read different weights.
 //
 //  res_split_kernel  x[:, tile] += quantizeA(A) . W^T tile: one workgroup
-//      per (32 rows, 32 output channels), 4 waves, each a quarter of the
-//      depth. A (ctx or g, float32) is quantised into an LDS panel from the
-//      row maxima its producer wrote (attention per head, wi_split per 32
-//      columns), so no pass over the row comes before the product.
+//      per (32 rows, CT tiles of 32 output channels), KS waves a tile, each
+//      its part of the depth. A (ctx or g, float32) is quantised into an LDS
+//      panel from the row maxima its producer wrote (attention per head,
+//      wi_split per 32 columns), so no pass over the row comes before the
+//      product.
 //  wi_split_kernel   g tile = GeGLU(xn . Wi^T): one workgroup per (32 rows,
 //      gated tile of 32 columns), 4 waves over the depth; also max |g| of
 //      each row's 32 columns.
 //  ln_rows_kernel    LayerNorm + quantizeA of 8 rows a workgroup.
 //
-// What bounds them: latency. At 24 rows of hidden 768 (36 and 24 workgroups)
+// What bounds them: latency at few rows. At 24 rows of hidden 768 (36 and 24 workgroups)
 // a launch takes 4.9 us (Wi), 5.1 us (Wo) and 6.4 us (WoMLP), LayerNorm 4.8
 // us: against 25 us (Wo + LayerNorm) and 50 us (the MLP block) on the
-// whole-row kernels, and 2.05 -> 0.93 ms a pass of 22 layers. Every global
-// load of a wave is in flight before its first use.
+// whole-row kernels, and 2.05 -> 0.93 ms a pass of 22 layers. A wave's
+// global loads are all issued before its first MFMA. With more rows, the
+// float32 rows read from L2 and the last-level cache by every tile's
+// workgroup: at 4,096 rows WoMLP took 69 us, Wo 47, Wi 26.
 //
 // The products are transposed as in mlp_block.hip (weights the A operand,
 // rows the B operand): a lane holds one row and 16 consecutive channels,
@@ -45,7 +48,6 @@ namespace ixh {
 namespace {
 
 constexpr int NXCD = 8;
-constexpr int WAVES = 4;  // of a workgroup, sharing a tile's depth
 
 // the weight row that lane row i loads, so that accumulator r of a lane is
 // channel 16*(lane/32) + r of the tile (mlp_block.hip)
@@ -55,32 +57,58 @@ __device__ __forceinline__ int pack4(const float4 v, float inv) {
   return (q8(v.x, inv) & 0xff) | ((q8(v.y, inv) & 0xff) << 8) | ((q8(v.z, inv) & 0xff) << 16) | (q8(v.w, inv) << 24);
 }
 
-// Workgroup -> (tile, row block): workgroup L runs on XCD L % 8, and the
-// row blocks of one tile go to one XCD, so that its L2 reads the tile's
-// weights once. False past the last tile.
+// Row blocks from which the kernels are arranged for many rows (512 rows):
+// measured with 4 waves a tile and the tiles dealt to the XCDs, then 2 waves
+// a tile, 4 tiles a workgroup (res) and the row blocks dealt to the XCDs, us
+// a launch at hidden 768: Wo 5.7 and 6.7 at 256 rows, 9.2 and 7.5 at 768, 47
+// and 16 at 4,096 (26 with the dealing alone); WoMLP 6.9 and 7.9, 12.0 and
+// 8.7, 69 and 22 (37); Wi 5.5 at 256 rows, 26 and 21 at 4,096 by the dealing.
+constexpr int kManyBlocks = 16;
+
+// Workgroup -> (tile, row block); workgroup L runs on XCD L % 8. With few
+// row blocks the row blocks of one tile go to one XCD, so that one L2 reads
+// the tile's weights; with many the tiles of one row block do, so that its
+// float32 rows reach one L2 once (they are most of the traffic). False past
+// the last tile or block.
 __device__ __forceinline__ bool tile_of(int ntiles, int nblk, int *tile, int *blk) {
-  const int i = blockIdx.x / NXCD;
-  *tile = (int)(blockIdx.x % NXCD) + NXCD * (i / nblk);
+  const int i = blockIdx.x / NXCD, x = blockIdx.x % NXCD;
+  if (nblk >= kManyBlocks) {
+    *blk = x + NXCD * (i / ntiles);
+    *tile = i % ntiles;
+    return *blk < nblk;
+  }
+  *tile = x + NXCD * (i / nblk);
   *blk = i % nblk;
   return *tile < ntiles;
 }
-int tile_grid(int ntiles, int nblk) { return NXCD * ((ntiles + NXCD - 1) / NXCD) * nblk; }
-
-// The waves' partial sums meet in LDS: wave w gets accumulators 4w .. 4w+3
-// of the whole depth. part: [WAVES][4][64] int4, acc's 4 accumulator groups.
-__device__ __forceinline__ int4 gather_sums(const int4 *part, int wave, int lane) {
-  int4 s = part[(0 * 4 + wave) * 64 + lane];
-#pragma unroll
-  for (int w = 1; w < WAVES; w++) {
-    const int4 t = part[(w * 4 + wave) * 64 + lane];
-    s = int4{s.x + t.x, s.y + t.y, s.z + t.z, s.w + t.w};
-  }
-  return s;
+int tile_grid(int ntiles, int nblk) {
+  return nblk >= kManyBlocks ? NXCD * ((nblk + NXCD - 1) / NXCD) * ntiles : NXCD * ((ntiles + NXCD - 1) / NXCD) * nblk;
 }
-__device__ __forceinline__ void put_sums(int4 *part, int wave, int lane, const v16i &acc) {
+
+// The partial sums of the KS waves that share a tile's depth meet in LDS
+// (part: [KS][4][64] int4): of its 4 groups of 4 accumulators, wave ks stores
+// the groups it does not own and gets the sums of its 4/KS own.
+template <int KS>
+__device__ __forceinline__ void put_sums(int4 *part, int ks, int lane, const v16i &acc) {
 #pragma unroll
   for (int q = 0; q < 4; q++)
-    part[(wave * 4 + q) * 64 + lane] = int4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+    if (q / (4 / KS) != ks)  // wave-uniform
+      part[(ks * 4 + q) * 64 + lane] = int4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+}
+template <int KS>
+__device__ __forceinline__ void gather_sums(const int4 *part, int ks, int lane, const v16i &acc, int4 *out) {
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    if (q / (4 / KS) == ks) {
+      int4 s = int4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+#pragma unroll
+      for (int w = 0; w < KS; w++)
+        if (w != ks) {
+          const int4 t = part[(w * 4 + q) * 64 + lane];
+          s = int4{s.x + t.x, s.y + t.y, s.z + t.z, s.w + t.w};
+        }
+      out[q % (4 / KS)] = s;
+    }
 }
 
 // ((f32(acc + 128 colsum) - zc) * sb) * sa of four channels; small: the
@@ -97,19 +125,18 @@ __device__ __forceinline__ float4 deq4(int4 t, bool small, const int32_t *c128, 
 
 template <int KT>
 __global__ __launch_bounds__(256) void wi_split_kernel(SplitArgs a) {
-  constexpr int KW = KT / WAVES;  // K steps of a wave
-  static_assert(KT % WAVES == 0, "depth over the waves");
-  __shared__ int4 part[2][WAVES * 4 * 64];
-  __shared__ float mx_s[WAVES][64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int KS = 4, KW = KT / KS;  // waves, K steps of a wave
+  static_assert(KT % KS == 0, "depth over the waves");
+  __shared__ int4 part[2][KS * 4 * 64];
+  __shared__ float mx_s[KS][64];
+  const int tid = threadIdx.x, lane = tid & 63, ks = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 31, fh = lane >> 5;
   int t, blk;
   if (!tile_of(a.n / 64, (a.M + 31) / 32, &t, &blk)) return;
   const int m0 = 32 * blk, row = min(m0 + fr, a.M - 1);  // rows past M: row M-1, never stored
-  // every load of the wave in flight at once
   v4i w[KW][2], x[KW];
-  const int8_t *wp = a.Bk + ((size_t)(wave * KW) * a.Np + 64 * t + perm32(fr)) * 32 + 16 * fh;
-  const int8_t *xp = a.Ak + ((size_t)(wave * KW) * a.ak_rows + row) * 32 + 16 * fh;
+  const int8_t *wp = a.Bk + ((size_t)(ks * KW) * a.Np + 64 * t + perm32(fr)) * 32 + 16 * fh;
+  const int8_t *xp = a.Ak + ((size_t)(ks * KW) * a.ak_rows + row) * 32 + 16 * fh;
 #pragma unroll
   for (int k = 0; k < KW; k++) {
     x[k] = *(const v4i *)(xp + (size_t)k * a.ak_rows * 32);
@@ -117,7 +144,7 @@ __global__ __launch_bounds__(256) void wi_split_kernel(SplitArgs a) {
     w[k][1] = *(const v4i *)(wp + (size_t)k * a.Np * 32 + 1024);
   }
   const float sa = a.sa[row];
-  const int ch = 64 * t + 16 * fh + 4 * wave;  // this lane's GELU-input channels (the multiplier's: + 32)
+  const int ch = 64 * t + 16 * fh + 4 * ks;  // this lane's GELU-input channels (the multiplier's: + 32)
   const float4 sba = *(const float4 *)(a.sb + ch), sbb = *(const float4 *)(a.sb + ch + 32);
   v16i acc[2] = {};
 #pragma unroll
@@ -125,72 +152,89 @@ __global__ __launch_bounds__(256) void wi_split_kernel(SplitArgs a) {
     acc[0] = mfma32(w[k][0], x[k], acc[0]);
     acc[1] = mfma32(w[k][1], x[k], acc[1]);
   }
-  put_sums(part[0], wave, lane, acc[0]);
-  put_sums(part[1], wave, lane, acc[1]);
+  put_sums<KS>(part[0], ks, lane, acc[0]);
+  put_sums<KS>(part[1], ks, lane, acc[1]);
   __syncthreads();
-  const float4 za = deq4(gather_sums(part[0], wave, lane), a.small, a.c128 + ch, a.zc + ch, sba, sa);
-  const float4 zb = deq4(gather_sums(part[1], wave, lane), a.small, a.c128 + ch + 32, a.zc + ch + 32, sbb, sa);
+  int4 ta, tb;
+  gather_sums<KS>(part[0], ks, lane, acc[0], &ta);
+  gather_sums<KS>(part[1], ks, lane, acc[1], &tb);
+  const float4 za = deq4(ta, a.small, a.c128 + ch, a.zc + ch, sba, sa);
+  const float4 zb = deq4(tb, a.small, a.c128 + ch + 32, a.zc + ch + 32, sbb, sa);
   const float4 g = make_float4(gelu_fma(za.x) * zb.x, gelu_fma(za.y) * zb.y, gelu_fma(za.z) * zb.z, gelu_fma(za.w) * zb.w);
-  if (m0 + fr < a.M) *(float4 *)(a.C + (size_t)(m0 + fr) * a.ldc + 32 * t + 16 * fh + 4 * wave) = g;
-  mx_s[wave][lane] = amax(amax(amax(amax(0.f, g.x), g.y), g.z), g.w);
+  if (m0 + fr < a.M) *(float4 *)(a.C + (size_t)row * a.ldc + 32 * t + 16 * fh + 4 * ks) = g;
+  mx_s[ks][lane] = amax(amax(amax(amax(0.f, g.x), g.y), g.z), g.w);
   __syncthreads();
   if (tid < 32 && m0 + tid < a.M) {
     float m = 0.f;
 #pragma unroll
-    for (int q = 0; q < WAVES; q++) m = __builtin_fmaxf(__builtin_fmaxf(m, mx_s[q][tid]), mx_s[q][32 + tid]);
+    for (int q = 0; q < KS; q++) m = __builtin_fmaxf(__builtin_fmaxf(m, mx_s[q][tid]), mx_s[q][32 + tid]);
     a.rmax[(size_t)(m0 + tid) * a.P + t] = m;
   }
 }
 
-template <int KT>
-__global__ __launch_bounds__(256) void res_split_kernel(SplitArgs a) {
-  constexpr int KW = KT / WAVES;
-  static_assert(KT % WAVES == 0, "depth over the waves");
+template <int KT, int KS, int CT>
+__global__ __launch_bounds__(64 * KS * CT) void res_split_kernel(SplitArgs a) {
+  constexpr int KW = KT / KS, GO = 4 / KS;                 // K steps and accumulator groups of a wave
+  constexpr int TPR = 2 * KS * CT, NV = 8 * KT / TPR;      // threads a row, float4s a thread
+  static_assert(KT % KS == 0 && 4 % KS == 0 && 8 * KT % TPR == 0, "depth and groups over the waves");
   __shared__ __attribute__((aligned(16))) int8_t panel[KT * 1024];  // [KT][64 lanes][16]
-  __shared__ int4 part[WAVES * 4 * 64];
+  __shared__ int4 part[CT][KS * 4 * 64];
   __shared__ float sa_s[32];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int fr = lane & 31, fh = lane >> 5;
+  const int fr = lane & 31, fh = lane >> 5, ks = wave % KS, ct = wave / KS;
   int t, blk;
-  if (!tile_of(a.n / 32, (a.M + 31) / 32, &t, &blk)) return;
+  if (!tile_of(a.n / 32 / CT, (a.M + 31) / 32, &t, &blk)) return;
+  t = t * CT + ct;
   const int m0 = 32 * blk;
-  // the row's maxima and its values: 8 threads a row, 32 columns a step
-  const int tr = tid >> 3, j = tid & 7;
+  // the row's maxima and its values: TPR threads a row, a float4 each a step
+  const int tr = tid / TPR, j = tid % TPR;
   const int arow = min(m0 + tr, a.M - 1);  // rows past M: row M-1, never stored
   float mx = 0.f;
-  for (int p = j; p < a.P; p += 8) mx = __builtin_fmaxf(mx, a.rmax[(size_t)arow * a.P + p]);
-  float4 v[KT];
+  for (int p = j; p < a.P; p += TPR) mx = __builtin_fmaxf(mx, a.rmax[(size_t)arow * a.P + p]);
+  float4 v[NV];
   const float *ap = a.A + (size_t)arow * a.lda + 4 * j;
 #pragma unroll
-  for (int k = 0; k < KT; k++) v[k] = *(const float4 *)(ap + 32 * k);
+  for (int u = 0; u < NV; u++) v[u] = *(const float4 *)(ap + 4 * TPR * u);
   v4i w[KW];
-  const int8_t *wp = a.Bk + ((size_t)(wave * KW) * a.Np + 32 * t + perm32(fr)) * 32 + 16 * fh;
+  const int8_t *wp = a.Bk + ((size_t)(ks * KW) * a.Np + 32 * t + perm32(fr)) * 32 + 16 * fh;
 #pragma unroll
   for (int k = 0; k < KW; k++) w[k] = *(const v4i *)(wp + (size_t)k * a.Np * 32);
-  const int ch = 32 * t + 16 * fh + 4 * wave;
-  const float4 sb = *(const float4 *)(a.sb + ch);
+  const int ch = 32 * t + 16 * fh + 4 * GO * ks;  // this lane's channels
   float *const xp = a.C + (size_t)min(m0 + fr, a.M - 1) * a.ldc + ch;
-  float4 x = *(const float4 *)xp;
+  float4 sb[GO], x[GO];
 #pragma unroll
-  for (int o = 1; o < 8; o <<= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, o));
+  for (int q = 0; q < GO; q++) {
+    sb[q] = *(const float4 *)(a.sb + ch + 4 * q);
+    x[q] = *(const float4 *)(xp + 4 * q);
+  }
+#pragma unroll
+  for (int o = 1; o < TPR; o <<= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, o));
   float s = 0.f, inv = 0.f;
   if (mx != 0.f) {  // quantizeA: s = max/127, inv = 1/s (int8.go:175-183)
     s = mx / 127.0f;
     inv = 1.0f / s;
   }
   if (j == 0) sa_s[tr] = s;
-  int8_t *pp = panel + (tr + 32 * (j >> 2)) * 16 + 4 * (j & 3);
 #pragma unroll
-  for (int k = 0; k < KT; k++) *(int *)(pp + 1024 * k) = pack4(v[k], inv);
+  for (int u = 0; u < NV; u++) {
+    const int col = 4 * (j + TPR * u);  // K step col / 32, half (col / 16) % 2, bytes col % 16 .. of row tr
+    *(int *)(panel + (col >> 5) * 1024 + (tr + 32 * ((col >> 4) & 1)) * 16 + (col & 15)) = pack4(v[u], inv);
+  }
   __syncthreads();
   v16i acc = {};
 #pragma unroll
-  for (int k = 0; k < KW; k++) acc = mfma32(w[k], *(const v4i *)(panel + 1024 * (wave * KW + k) + 16 * lane), acc);
-  put_sums(part, wave, lane, acc);
+  for (int k = 0; k < KW; k++) acc = mfma32(w[k], *(const v4i *)(panel + (ks * KW + k) * 1024 + 16 * lane), acc);
+  put_sums<KS>(part[ct], ks, lane, acc);
   __syncthreads();
-  const float4 d = deq4(gather_sums(part, wave, lane), a.small, a.c128 + ch, a.zc + ch, sb, sa_s[fr]);
-  x = make_float4(x.x + d.x, x.y + d.y, x.z + d.z, x.w + d.w);
-  if (m0 + fr < a.M) *(float4 *)xp = x;
+  int4 sum[GO];
+  gather_sums<KS>(part[ct], ks, lane, acc, sum);
+  if (m0 + fr < a.M) {
+#pragma unroll
+    for (int q = 0; q < GO; q++) {
+      const float4 d = deq4(sum[q], a.small, a.c128 + ch + 4 * q, a.zc + ch + 4 * q, sb[q], sa_s[fr]);
+      *(float4 *)(xp + 4 * q) = make_float4(x[q].x + d.x, x[q].y + d.y, x[q].z + d.z, x[q].w + d.w);
+    }
+  }
 }
 
 // LayerNorm (vec_simd.go:285-327) and quantizeA of ROWS rows a workgroup:
@@ -311,22 +355,33 @@ bool split_rows_supported(int H, int I, int KpH, int KpI) {
   return (H == 768 && I == 1152) || (H == 384 && I == 1152) || (H == 256 && I == 512);
 }
 
+namespace {
+template <int KT>
+void wi_one(const SplitArgs &a, hipStream_t s) {
+  wi_split_kernel<KT><<<tile_grid(a.n / 64, (a.M + 31) / 32), 256, 0, s>>>(a);
+}
+template <int KT>
+void res_one(const SplitArgs &a, hipStream_t s) {
+  const int nblk = (a.M + 31) / 32;
+  if (nblk < kManyBlocks) res_split_kernel<KT, 4, 1><<<tile_grid(a.n / 32, nblk), 256, 0, s>>>(a);
+  else res_split_kernel<KT, 2, 4><<<tile_grid(a.n / 128, nblk), 512, 0, s>>>(a);
+}
+}  // namespace
+
 void launch_wi_split(const SplitArgs &a, hipStream_t s) {
   if (a.M <= 0) return;
-  const int grid = tile_grid(a.n / 64, (a.M + 31) / 32);
-  if (a.K == 768) wi_split_kernel<24><<<grid, 256, 0, s>>>(a);
-  else if (a.K == 384) wi_split_kernel<12><<<grid, 256, 0, s>>>(a);
-  else wi_split_kernel<8><<<grid, 256, 0, s>>>(a);
+  if (a.K == 768) wi_one<24>(a, s);
+  else if (a.K == 384) wi_one<12>(a, s);
+  else wi_one<8>(a, s);
 }
 
 void launch_res_split(const SplitArgs &a, hipStream_t s) {
   if (a.M <= 0) return;
-  const int grid = tile_grid(a.n / 32, (a.M + 31) / 32);
-  if (a.K == 1152) res_split_kernel<36><<<grid, 256, 0, s>>>(a);
-  else if (a.K == 768) res_split_kernel<24><<<grid, 256, 0, s>>>(a);
-  else if (a.K == 512) res_split_kernel<16><<<grid, 256, 0, s>>>(a);
-  else if (a.K == 384) res_split_kernel<12><<<grid, 256, 0, s>>>(a);
-  else res_split_kernel<8><<<grid, 256, 0, s>>>(a);
+  if (a.K == 1152) res_one<36>(a, s);
+  else if (a.K == 768) res_one<24>(a, s);
+  else if (a.K == 512) res_one<16>(a, s);
+  else if (a.K == 384) res_one<12>(a, s);
+  else res_one<8>(a, s);
 }
 
 void launch_ln_rows(const LnRowsArgs &a, int lanes, hipStream_t s) {

@@ -24,9 +24,10 @@ def seqs_of(rng, vocab, *lens):
 def test_few_rows_exact(shape, lanes, plant):
     """Row counts around the 32-row blocks (and the 8 rows of a LayerNorm
     workgroup), one sequence or several, a sequence over 512 keys (QKV input
-    row-major), and the two sides of the rule that picks these kernels;
-    setting a kernel option (here to its default) picks the whole-row
-    kernels, and gives the same bits."""
+    row-major), the two arrangements of the residual kernel (from 481 rows
+    on) and the two sides of the rules that pick these kernels and the
+    32-row MLP kernel; setting a kernel option (here to its default) picks
+    the whole-row kernels, and gives the same bits."""
     cfg = SHAPES[shape](layers=2)
     w = Weights.random(cfg, seed=97)
     if plant:
@@ -34,12 +35,14 @@ def test_few_rows_exact(shape, lanes, plant):
     gpu, ora = Model(w, lanes=lanes), orc.OracleModel(w, lanes=lanes)
     rng = np.random.default_rng(97)
     batches = [seqs_of(rng, cfg.vocab, *lens)
-               for lens in ((1,), (7, 1), (31,), (9, 0, 23), (33,), (64, 1, 192), (600, 9))]
+               for lens in ((1,), (7, 1), (31,), (9, 0, 23), (33,), (64, 1, 192), (480,), (481,), (600, 9))]
+    gpu.set_option("parts", 1)
     want = [ora.encode_tokens(b)[0] for b in batches]
     for b, e in zip(batches, want):
         got = gpu.encode_tokens(b)
         assert f32_bits_equal(got, e), ([len(s) for s in b], mismatch_report(got, e))
-    edges = [seqs_of(rng, cfg.vocab, *lens) for lens in ((500, 500, 500, 36), (500, 500, 500, 37))]
+    most = {"small": 2048, "base": 3072, "bekko": 4096}[shape]
+    edges = [seqs_of(rng, cfg.vocab, *[64] * (n // 64), n % 64) for n in (most, most + 1, 8192, 8193)]
     few = [gpu.encode_tokens(b) for b in batches + edges]
     gpu.set_option("fuse_mlp", 2)
     for b, e in zip(batches + edges, few):
