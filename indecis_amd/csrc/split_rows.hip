@@ -267,7 +267,8 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(LnRowsArgs a) {
       double sum = 0.0;
       if constexpr (V > 0) {
         const float *xr = xs + cr * LD + ch % V;
-        constexpr int NE = H / V, NB = NE < 16 ? NE : 16;
+        constexpr int NE = H / V, NB = NE % 16 == 0 ? 16 : 8;  // values a lane, a batch of them
+        static_assert(NE % NB == 0, "whole batches");
         float p = 0.f, b[NB], n[NB];
 #pragma unroll
         for (int e = 0; e < NB; e++) b[e] = xr[V * e];

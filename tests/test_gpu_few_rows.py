@@ -20,6 +20,7 @@ def seqs_of(rng, vocab, *lens):
 # shape, lane width, rows past the dequantisation bound planted in a matrix
 @pytest.mark.parametrize("shape,lanes,plant", [
     ("base", 8, None), ("base", 16, "wo"), ("base", 0, "womlp"), ("bekko", 8, "wi"), ("bekko", 4, None),
+    ("bekko", 16, None), ("bekko", 0, None),
     ("small", 8, "wo"), ("small", 16, None), ("small", 4, "womlp"), ("small", 0, "wi")])
 def test_few_rows_exact(shape, lanes, plant):
     """Row counts around the 32-row blocks (and the 8 rows of a LayerNorm
