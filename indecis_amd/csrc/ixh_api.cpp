@@ -601,6 +601,9 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   const bool kblock = fused && (fuse_mlp || split) && tune.qkv_kblock != 0 && qkv_kblock_supported(KpH) &&
                       m->layers[0].qkv.qk.p;
 
+  // short sequences: QKV, Attn8.Prepare and attention in one kernel
+  const bool short_seqs = !tune.fixed && kblock && short_attn_supported(KpH, T, B * nh);
+
   int rc;
   const size_t ntab = 2 * (size_t)(B + 1) + blocks.size() + B;
   if ((rc = w->tabs.ensure(4 * ntab)) || (rc = w->pos.ensure(4 * (size_t)N)) ||
@@ -828,7 +831,12 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
     }
     // attention (infer.go:437-518)
     aa.window = global ? -1 : c.local_attention / 2;
-    if (fused) {
+    const double pairs = global ? keys_global : keys_local;
+    if (short_seqs) {
+      RUN(global ? "qkv_attn_global" : "qkv_attn_local", 2 * dN * 3 * dH * dH + 4.0 * D * nh * pairs,
+          gemm_bytes(dH, 3 * dH, 0, false) + dN * dH * 4,
+          if (!launch_short_attn(g, aa, st)) return refused("qkv_attn"));
+    } else if (fused) {
       // QKV GEMM and Attn8.Prepare in one kernel: int8 Q, K, V and their
       // scales are its only outputs
       RUN("gemm_qkv", 2 * dN * 3 * dH * dH,
@@ -840,9 +848,9 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
       RUN("attn_prologue", 0, dN * 2 * dH * 4 + dN * 2 * dH + 4 * dN * nh,
           launch_attn_prologue(aa, st));
     }
-    const double pairs = global ? keys_global : keys_local;
-    RUN(global ? "attn_global" : "attn_local", 4.0 * D * nh * pairs,
-        dN * 3 * dH + 8 * dN * nh + dN * dH * 4, launch_attn_main(aa, st));
+    if (!short_seqs)
+      RUN(global ? "attn_global" : "attn_local", 4.0 * D * nh * pairs,
+          dN * 3 * dH + 8 * dN * nh + dN * dH * 4, launch_attn_main(aa, st));
     if (split) {
       // x += ctx . Wo^T (infer.go:403), mlp_norm (infer.go:404-407), Wi +
       // GeGLU, x += g . WoMLP^T (infer.go:408-424), the next attn_norm

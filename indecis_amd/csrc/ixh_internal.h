@@ -320,6 +320,12 @@ constexpr int kKeyPad = 64;       // key slots of a sequence are padded to this
 // (2 only for an even head count where the device grants the LDS).
 constexpr int kQkvSeqMax = 512;
 void launch_qkv_attn(const GemmArgs &g, const AttnArgs &a, const int32_t *order, int heads, hipStream_t s);
+// QKV projection, Attn8.Prepare and attention in one kernel (short_attn.hip),
+// for batches of short sequences (see there) and Kp one of 768, 384, 256: g as for launch_qkv_attn with the K-blocked input, a as for
+// launch_attn_main (of the prologue's outputs nothing is written); false
+// (nothing launched) otherwise.
+bool short_attn_supported(int Kp, int max_n, int workgroups);
+bool launch_short_attn(const GemmArgs &g, const AttnArgs &a, hipStream_t s);
 // The fused QKV kernel's K-blocked input ([Kp/32][rows][32]): supported
 // for Kp a multiple of 128 whose weight rows fit in its LDS.
 bool qkv_kblock_supported(int Kp);

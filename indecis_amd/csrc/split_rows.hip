@@ -85,44 +85,6 @@ int tile_grid(int ntiles, int nblk) {
   return nblk >= kManyBlocks ? NXCD * ((nblk + NXCD - 1) / NXCD) * ntiles : NXCD * ((ntiles + NXCD - 1) / NXCD) * nblk;
 }
 
-// The partial sums of the KS waves that share a tile's depth meet in LDS
-// (part: [KS][4][64] int4): of its 4 groups of 4 accumulators, wave ks stores
-// the groups it does not own and gets the sums of its 4/KS own.
-template <int KS>
-__device__ __forceinline__ void put_sums(int4 *part, int ks, int lane, const v16i &acc) {
-#pragma unroll
-  for (int q = 0; q < 4; q++)
-    if (q / (4 / KS) != ks)  // wave-uniform
-      part[(ks * 4 + q) * 64 + lane] = int4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-}
-template <int KS>
-__device__ __forceinline__ void gather_sums(const int4 *part, int ks, int lane, const v16i &acc, int4 *out) {
-#pragma unroll
-  for (int q = 0; q < 4; q++)
-    if (q / (4 / KS) == ks) {
-      int4 s = int4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-#pragma unroll
-      for (int w = 0; w < KS; w++)
-        if (w != ks) {
-          const int4 t = part[(w * 4 + q) * 64 + lane];
-          s = int4{s.x + t.x, s.y + t.y, s.z + t.z, s.w + t.w};
-        }
-      out[q % (4 / KS)] = s;
-    }
-}
-
-// ((f32(acc + 128 colsum) - zc) * sb) * sa of four channels; small: the
-// weights' bound holds and f32(acc + 128 colsum) - zc is f32(acc)
-__device__ __forceinline__ float4 deq4(int4 t, bool small, const int32_t *c128, const float *zc, float4 sb, float sa) {
-  if (small)
-    return make_float4(((float)t.x * sb.x) * sa, ((float)t.y * sb.y) * sa, ((float)t.z * sb.z) * sa,
-                       ((float)t.w * sb.w) * sa);
-  const int4 c = *(const int4 *)c128;
-  const float4 z = *(const float4 *)zc;
-  return make_float4(deq(t.x + c.x, z.x, sb.x, sa), deq(t.y + c.y, z.y, sb.y, sa), deq(t.z + c.z, z.z, sb.z, sa),
-                     deq(t.w + c.w, z.w, sb.w, sa));
-}
-
 template <int KT>
 __global__ __launch_bounds__(256) void wi_split_kernel(SplitArgs a) {
   constexpr int KS = 4, KW = KT / KS;  // waves, K steps of a wave

@@ -50,3 +50,31 @@ def test_few_rows_exact(shape, lanes, plant):
         got = gpu.encode_tokens(b)
         assert f32_bits_equal(got, e), ([len(s) for s in b], mismatch_report(got, e))
     gpu.close()
+
+
+@pytest.mark.parametrize("shape,lanes,window,plant", [
+    ("small", 8, 128, False), ("small", 0, 16, True), ("small", 16, 16, False), ("small", 4, 128, True),
+    ("bekko", 8, 16, False), ("bekko", 16, 128, True), ("base", 8, 128, False), ("base", 4, 16, True)])
+def test_short_sequences_exact(shape, lanes, window, plant):
+    """QKV, Attn8.Prepare and attention in one kernel (short_attn.hip): the
+    longest sequence at the edges of its 1, 2 and 4 row blocks, with a local
+    window that cuts sequences and one that does not, empty sequences, QKV
+    rows past the dequantisation bound, and batches one workgroup either side
+    of the rules that pick it (two rounds of the 256 CUs up to 64 tokens, one
+    up to 128), against the oracle."""
+    cfg = SHAPES[shape](layers=2, local_attention=window)
+    w = Weights.random(cfg, seed=101)
+    if plant:
+        for row in (3, cfg.hidden + 5, 2 * cfg.hidden + 7):
+            w.wqkv_q[0, row, :] = 127
+    gpu, ora = Model(w, lanes=lanes), orc.OracleModel(w, lanes=lanes)
+    rng = np.random.default_rng(101)
+    batches = [(1,), (15, 2), (31, 0, 1), (32, 32, 17), (33, 5), (40, 0, 63, 1), (64, 33), (65, 31), (97, 8), (127,),
+               (128, 1, 90), (129, 3)]
+    two, one = 512 // cfg.heads, 256 // cfg.heads
+    batches += [(33,) + (2,) * (two - 1), (33,) + (2,) * two, (65,) + (2,) * (one - 1), (65,) + (2,) * one]
+    for lens in batches:
+        seqs = seqs_of(rng, cfg.vocab, *lens)
+        got, want = gpu.encode_tokens(seqs), ora.encode_tokens(seqs)[0]
+        assert f32_bits_equal(got, want), (lens[:4], mismatch_report(got, want))
+    gpu.close()
