@@ -529,10 +529,36 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
   // the missing 128 * sum_j v[j][d] over every key of the tiles a wave
   // processes is the same for all its queries and is added to the
   // accumulators per chunk from the prefix sums: O stays exact.
-  // P is rounded from the hardware exponential (exp255_fast) unless that
-  // lands within kExp255Tol of a half-integer; there (about 1 score in 4000)
-  // the reference formula decides: exp32 on the tail keys j >= ts (all keys
-  // when lanes = 0), ExpShift's vector formula elsewhere.
+  // With x = f32(q.k) * ks, y = 2^(x (sq log2 e) + (log2 255 - m log2 e)) is
+  // 255 exp(s - max) up to a relative error the score bounds: P is its
+  // rounding where y less that error and y plus it round alike. Where they do
+  // not (about 1 group of 4 scores in 100), s - max is formed as the reference
+  // forms it and rounded from exp255_fast, unless that lands within
+  // kExp255Tol of a half-integer; there the reference formula decides: exp32
+  // on the tail keys j >= ts (all keys when lanes = 0), ExpShift's vector
+  // formula elsewhere.
+  //
+  // The error, with u = 2^-24 and the scores that matter (P > 0: s - m >
+  // -6.3, so |s| <= |m| + 6.3): the reference's own roundings of s and of s -
+  // m move the exponent by log2 e (|s| + |s - m|) u, the products and the
+  // constants here by (|s| log2 e + 8 + |m| log2 e + 8) u, the exponent's
+  // rounding in exp255_fast 8 u: together (51.3 + 4.33 |m|) u, times ln 2 in
+  // y; exp255_fast against the reference formulas 8 u (the relative form of
+  // kExp255Tol), the hardware exponential twice and the scaling by hi 6 u:
+  // (50 + 3 |m|) u, taken as kap = (64 + 3.5 |m|) u. Past |m| = 2^15 every
+  // group takes the other way. 11 VALU slots a score instead of 13 (the
+  // exponential takes 4) and fewer scores formed twice: global layers of
+  // 8,192 tokens 2,900 -> 2,650 us a launch, of 4,096 162 -> 146, of 256 64.5
+  // -> 60.3; local layers 97 -> 93.5 and 50.2 -> 49.
+  float es = sqv * 1.44269504088896341f;
+  const float kap = (64.0f + 3.5f * fabsf(m)) * 0x1p-24f;
+  float eb = __builtin_fmaf(-m, 1.44269504088896341f, 7.99435343685885793f) - 1.4427f * kap;
+  float hi = 1.0f + 2.125f * kap;  // (1 - kap) hi >= 1 + kap
+  if (qact && !(fabsf(m) <= 32768.0f)) {  // y = 1, its upper bound 300
+    es = 0.0f;
+    eb = 0.0f;
+    hi = 300.0f;
+  }
   v16i o[2];
 #pragma unroll
   for (int dt = 0; dt < 2; dt++)
@@ -567,43 +593,48 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
       score_scale(t, c0, score_acc(t, c0), sv);
       const int k0 = t * 32;
       const bool full = k0 >= cs_hi && k0 + 32 <= ce_lo;  // every key valid for every query
-      float p[16];
-      // largest distance of 255 e from its rounding: one max per score,
-      // one compare per tile; the rare lanes past the tolerance recheck
-      // their scores one by one
-      float dev = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        sv[r] = sv[r] * sqv - m;  // s - max, as the reference forms it
-        const float y = exp255_fast(sv[r]);
-        p[r] = rne(y);
-        dev = __builtin_fmaxf(dev, fabsf(y - p[r]));  // no NaN here: one v_max
-      }
-      if (dev > 0.5f - kExp255Tol) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-          if (fabsf(exp255_fast(sv[r]) - p[r]) > 0.5f - kExp255Tol) {
-            const int j = k0 + acc_row(r, lane);
-            const float e = (j >= ts) ? exp32_scalar(sv[r]) : exp32_simd(sv[r]);
-            // QuantizeRowU8 (vec_simd.go:64-91): RNE(e*255) in [0, 255]
-            p[r] = rne(e * 255.0f);
-          }
-        }
-      }
-      if (!full) {
-        const int jb = k0 - cs + 4 * (lane >> 5);
-#pragma unroll
-        for (int r = 0; r < 16; r++) p[r] = (uint32_t)(jb + 8 * (r >> 2) + (r & 3)) < span ? p[r] : 0.0f;
-      }
       unsigned pw[4];
 #pragma unroll
       for (int g = 0; g < 4; g++) {
-        unsigned w = 0;
+        unsigned lo = 0, up = 0;
 #pragma unroll
-        for (int u = 0; u < 4; u++) w = __builtin_amdgcn_cvt_pk_u8_f32(p[4 * g + u], u, w);
-        pw[g] = w;
-        psum = __builtin_amdgcn_udot4(w, 0x01010101u, psum, false);
+        for (int u = 0; u < 4; u++) {
+          const float y = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[4 * g + u], es, eb));
+          lo = __builtin_amdgcn_cvt_pk_u8_f32(y, u, lo);
+          up = __builtin_amdgcn_cvt_pk_u8_f32(y * hi, u, up);
+        }
+        if (lo != up) {
+          // a bound either side of a half-integer: the score as the
+          // reference forms it, its exponential checked float by float
+          lo = 0;
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            const float d = sv[4 * g + u] * sqv - m;
+            const float y = exp255_fast(d);
+            float p = rne(y);
+            if (fabsf(y - p) > 0.5f - kExp255Tol) {
+              const int j = k0 + 8 * g + 4 * (lane >> 5) + u;
+              const float e = (j >= ts) ? exp32_scalar(d) : exp32_simd(d);
+              // QuantizeRowU8 (vec_simd.go:64-91): RNE(e*255) in [0, 255]
+              p = rne(e * 255.0f);
+            }
+            lo = __builtin_amdgcn_cvt_pk_u8_f32(p, u, lo);
+          }
+        }
+        pw[g] = lo;
       }
+      if (!full) {
+        // the tile's valid keys as bits, a group's 4 bits as byte masks
+        const int first = min(max(cs - k0, 0), 32), last = min(max(ce - k0, 0), 32);
+        const unsigned ok = ((unsigned)((1ull << last) - 1) & (unsigned)(~0ull << first)) >> (4 * (lane >> 5));
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const unsigned one = (((ok >> (8 * g)) & 0xfu) * 0x204081u) & 0x01010101u;
+          pw[g] &= (one << 8) - one;
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < 4; g++) psum = __builtin_amdgcn_udot4(pw[g], 0x01010101u, psum, false);
       // P - 128 as int8
       const v4i bp = {(int)(pw[0] ^ 0x80808080u), (int)(pw[1] ^ 0x80808080u),
                       (int)(pw[2] ^ 0x80808080u), (int)(pw[3] ^ 0x80808080u)};

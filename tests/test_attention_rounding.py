@@ -1,0 +1,62 @@
+"""The bound behind the attention kernel's rounding of P (attention_i8.hip):
+the exponent it forms in one fused step against the reference's roundings,
+on the CPU; and, on the GPU, scores of every magnitude against the oracle."""
+import numpy as np
+import pytest
+
+from helpers import f32_bits_equal, mismatch_report
+
+L2E, L255, U = np.float32(1.44269504088896341), np.float32(7.99435343685885793), 2.0 ** -24
+
+
+def fma(a, b, c):
+    """float32 fma (the product of two float32 is exact in float64)."""
+    return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)).astype(np.float32)
+
+
+@pytest.mark.parametrize("top", [0.01, 1.0, 8.0, 300.0, 32768.0])
+def test_exponent_error_bound(top):
+    """x = f32(q.k)*ks, sq and the row max m at random, scores s = x*sq
+    within 6.3 of m: the kernel's exponent differs from the one that
+    exp255_fast forms of f32(f32(x*sq) - m) by at most (51.3 + 4.33 |m|) u,
+    and 255*exp(s - m) lies between its two bounds."""
+    rng = np.random.default_rng(5)
+    n = 400000
+    m = (rng.uniform(-top, top, n)).astype(np.float32)
+    sq = np.exp(rng.uniform(-12, 4, n)).astype(np.float32)
+    x = ((m - rng.uniform(0, 6.3, n)) / sq).astype(np.float32)
+    s = (x * sq).astype(np.float32)
+    d = (np.minimum(s, m) - m).astype(np.float32)
+    keep = (s <= m) & (d >= -6.3)
+    m, sq, x, d = m[keep], sq[keep], x[keep], d[keep]
+    ref = fma(d, np.full_like(d, L2E), np.full_like(d, L255))
+    es = (sq * L2E).astype(np.float32)
+    base = fma(-m, np.full_like(m, L2E), np.full_like(m, L255))
+    err = np.abs(fma(x, es, base).astype(np.float64) - ref)
+    am = np.abs(m).astype(np.float64)
+    assert np.all(err <= (51.3 + 4.33 * am) * U), (err / ((51.3 + 4.33 * am) * U)).max()
+    kap = ((np.float32(64) + np.float32(3.5) * np.abs(m)) * np.float32(U)).astype(np.float32)
+    y = np.exp2(fma(x, es, (base - np.float32(1.4427) * kap).astype(np.float32)).astype(np.float64))
+    hi = (np.float32(1) + np.float32(2.125) * kap).astype(np.float64)
+    true = 255.0 * np.exp(d.astype(np.float64))
+    # 12 u: the share of the hardware exponential and of the reference formulas
+    assert np.all(y * (1 + 12 * U) <= true) and np.all(y * hi * (1 - 12 * U) >= true)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lanes", [8, 0])
+@pytest.mark.parametrize("scale", [1e-3, 0.3, 6.0, 60.0, 400.0, 1e4])
+def test_attend8_score_magnitudes(scale, lanes):
+    """Attend8 with q and k scaled by `scale` (row maxima of the scores from
+    about 1e-5 to 1e9, either side of the bound past which every score is
+    formed as the reference forms it), global and windowed, against the
+    oracle, bit for bit."""
+    from indecis_amd import linalg
+    from oracle import oracle as orc
+    rng = np.random.default_rng(int(scale * 1000) + lanes)
+    for n, window in ((33, -1), (300, 8), (700, -1), (261, 64)):
+        q, k, v = (rng.standard_normal((n, 64)).astype(np.float32) for _ in range(3))
+        q, k = q * np.float32(scale), k * np.float32(scale)
+        q[n // 2] = 0
+        got, want = linalg.attend8(q, k, v, window, 0.125, lanes), orc.attend8(q, k, v, window, 0.125, lanes)
+        assert f32_bits_equal(got, want), (n, window, mismatch_report(got, want))
