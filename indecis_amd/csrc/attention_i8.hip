@@ -46,95 +46,111 @@ __device__ __forceinline__ int pack4(int a, int b, int c, int d) {
 }
 
 constexpr int kShortSeq = 512;   // keys one prologue workgroup holds in registers
-constexpr int kStatRows = 256;   // keys per LDS slab of the long-sequence K chains
-constexpr int kStatStride = kStatRows + 4;
 
 // Statistics of a long sequence (more than kShortSeq keys) for
-// Attn8.Prepare (attention8.go:224-230, 259-269), split 8 ways per
-// (sequence, head): blockIdx.z 0..3 run the float32 chains of the K mean
-// of 16 dimensions each, in key order (AddTo, then Scale by f32(1/n));
-// blockIdx.z 4..7 take max |V| of 16 dimensions (MaxAbsTo). 4 threads own
-// a key's 16 values (a float4 each), 64 keys per load. The K chains read
-// their slab transposed from LDS (one dimension's keys contiguous), double
-// buffered, while the next slab's loads are in flight. Writes the V scale
-// to a.vs and, per (sequence, head), the K mean and 1/V scale to a.kstat.
-__global__ __launch_bounds__(256) void attn_long_stats_kernel(AttnArgs a) {
-  __shared__ __attribute__((aligned(16))) float kt[2][16][kStatStride];
-  const int b = blockIdx.x, h = blockIdx.y, z = blockIdx.z, tid = threadIdx.x;
-  const int q = tid & 3, r0 = tid >> 2;
-  const bool isk = z < 4;
-  const int dg = (z & 3) * 16;
+// Attn8.Prepare (attention8.go:224-230, 259-269), split 4 ways per
+// (sequence, head): blockIdx.z 0 and 1 run the float32 chains of the K mean
+// of 32 dimensions each, in key order (AddTo, then Scale by f32(1/n));
+// blockIdx.z 2 and 3 take max |V| of 32 dimensions (MaxAbsTo). Writes the V
+// scale to a.vs and, per (sequence, head), the K mean and 1/V scale to
+// a.kstat.
+//
+// What bounds it: the chain of n dependent adds where few sequences run (one
+// of 4,096 tokens: 48 us with the chain waiting on LDS every 4 keys and the
+// slabs one ahead), the reading of K and V where many do. So K comes into an
+// LDS ring by direct-to-LDS loads of waves 0-3, kStatRing - 1 slabs ahead,
+// and wave 4, which has no load of its own to wait for, runs the chains, 32
+// keys read from LDS ahead of their adds (about 9 cycles a key). With the
+// prologue below, one sequence of 4,096 tokens 60 -> 31 us a layer, 8 of 1,024
+// 34 -> 31, 8 of 8,192 199 -> 178 (hidden 768).
+constexpr int kStatDims = 32;    // dimensions of a workgroup: a 128-byte line of a key's row
+constexpr int kStatKeys = 128;   // keys of a slab: four loads of each loading wave
+constexpr int kStatRing = 4;     // slabs in LDS
+constexpr int kStatThreads = 320;
+__global__ __launch_bounds__(kStatThreads) void attn_long_stats_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(1024))) float ring[kStatRing][kStatKeys * kStatDims];
+  const int b = blockIdx.x, h = blockIdx.y, z = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int dg = (z & 1) * kStatDims;
   const int base = a.offs[b], n = a.offs[b + 1] - base;
   const int ld = 3 * a.H;
-  const float *seq = a.qkv + (size_t)base * ld;
-  const uint32_t voff = 4u * ((uint32_t)r0 * ld + (isk ? a.H : 2 * a.H) + h * D + dg + 4 * q);
+  const float *src = a.qkv + (size_t)base * ld + (z < 2 ? a.H : 2 * a.H) + h * D + dg;
   float *stat = a.kstat + ((size_t)b * a.nh + h) * 2 * D;
-  const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  float4 reg[4];
-  // rows c0 .. c0+255 through a buffer descriptor of the slab's valid rows:
-  // keys past the sequence read as 0
-#define IXH_STAT_LOAD(c0)                                                                   \
-  {                                                                                         \
-    const __amdgpu_buffer_rsrc_t rs =                                                       \
-        buf_rsrc(seq + (size_t)(c0) * ld, (uint32_t)min(kStatRows, n - (c0)) * ld * 4);     \
-    _Pragma("unroll") for (int u = 0; u < 4; u++) reg[u] = buf_load_f4(rs, voff, 256u * u * ld); \
-  }
-  if (isk) {
-    float ksum = 0.f;
-    if (n > 0) IXH_STAT_LOAD(0)
-    for (int c0 = 0, buf = 0; c0 < n; c0 += kStatRows, buf ^= 1) {
+  if (z < 2) {
+    const int nslab = (n + kStatKeys - 1) / kStatKeys;
+    if (wave < 4) {
+      // slab s: key 32 wave + 8 u + lane / 8 of it, 16 bytes lane % 8 (keys
+      // past n: key n-1, never added; past the last slab: the load count a
+      // wave has in flight stays the same)
+      auto issue = [&](int s) {
 #pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int r = r0 + 64 * u;
-        kt[buf][4 * q][r] = reg[u].x;
-        kt[buf][4 * q + 1][r] = reg[u].y;
-        kt[buf][4 * q + 2][r] = reg[u].z;
-        kt[buf][4 * q + 3][r] = reg[u].w;
-      }
-      __syncthreads();  // also orders the previous chain on this buffer
-      if (c0 + kStatRows < n) IXH_STAT_LOAD(c0 + kStatRows)
-      if (tid < 16) {
-        const float *row = &kt[buf][tid][0];
-        const int cnt = min(kStatRows, n - c0);
-        int r = 0;
-        for (; r + 4 <= cnt; r += 4) {
-          const float4 v = *(const float4 *)(row + r);
-          ksum = ksum + v.x;
-          ksum = ksum + v.y;
-          ksum = ksum + v.z;
-          ksum = ksum + v.w;
+        for (int u = 0; u < kStatKeys / 32; u++) {
+          const int key = min(s * kStatKeys + 32 * wave + 8 * u + (lane >> 3), n - 1);
+          __builtin_amdgcn_global_load_lds((glb_ptr)(src + (size_t)key * ld + 4 * (lane & 7)),
+                                           (lds_ptr)(&ring[s % kStatRing][(32 * wave + 8 * u) * kStatDims]), 16, 0, 0);
         }
-        for (; r < cnt; r++) ksum = ksum + row[r];
+      };
+      if (nslab > 0)
+        for (int s = 0; s < kStatRing - 1; s++) issue(s);
+      for (int s = 0; s < nslab; s++) {
+        wait_vmcnt<kStatKeys / 32 * (kStatRing - 2)>();  // slab s landed
+        __builtin_amdgcn_s_barrier();       // every wave's; the chains are past slab s - 1
+        issue(s + kStatRing - 1);
       }
+      wait_vmcnt<0>();  // no load into LDS outlives the workgroup
+    } else {
+      float ksum = 0.f;
+      for (int s = 0; s < nslab; s++) {
+        lds_barrier();  // slab s is there; this wave's reads of slab s - 1 are done
+        const float *col = &ring[s % kStatRing][lane & (kStatDims - 1)];
+        const int cnt = n - s * kStatKeys;
+        if (cnt >= kStatKeys) {
+          constexpr int NB = 32;
+          float v[2][NB];
+#pragma unroll
+          for (int r = 0; r < NB; r++) v[0][r] = col[r * kStatDims];
+#pragma unroll
+          for (int k = 0; k < kStatKeys / NB; k++) {
+            if (k + 1 < kStatKeys / NB) {
+#pragma unroll
+              for (int r = 0; r < NB; r++) v[(k + 1) & 1][r] = col[(NB * (k + 1) + r) * kStatDims];
+            }
+            __builtin_amdgcn_sched_barrier(0);  // the next batch is read before this one is added
+#pragma unroll
+            for (int r = 0; r < NB; r++) ksum = ksum + v[k & 1][r];
+          }
+        } else {
+          for (int r = 0; r < cnt; r++) ksum = ksum + col[r * kStatDims];
+        }
+      }
+      if (lane < kStatDims) stat[dg + lane] = n > 0 ? ksum * (1.0f / (float)n) : 0.f;
     }
-    if (tid < 16) stat[dg + tid] = n > 0 ? ksum * (1.0f / (float)n) : 0.f;
   } else {
-    float4 vm = zero4;
-    if (n > 0) IXH_STAT_LOAD(0)
-    for (int c0 = 0; c0 < n; c0 += kStatRows) {
-      float4 cur[4];
+    // 8 threads a key (a float4 each), 40 keys a load, 16 loads in flight
+    constexpr int KR = kStatThreads / 8, NL = 16;
+    const int q = tid & 7, r0 = tid >> 3;
+    float4 vm = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int c0 = 0; c0 < n; c0 += KR * NL) {
+      float4 v[NL];
 #pragma unroll
-      for (int u = 0; u < 4; u++) cur[u] = reg[u];
-      if (c0 + kStatRows < n) IXH_STAT_LOAD(c0 + kStatRows)
+      for (int u = 0; u < NL; u++) v[u] = *(const float4 *)(src + (size_t)min(c0 + r0 + KR * u, n - 1) * ld + 4 * q);
 #pragma unroll
-      for (int u = 0; u < 4; u++)
-        vm = make_float4(amax(vm.x, cur[u].x), amax(vm.y, cur[u].y),
-                         amax(vm.z, cur[u].z), amax(vm.w, cur[u].w));
+      for (int u = 0; u < NL; u++)
+        vm = make_float4(amax(vm.x, v[u].x), amax(vm.y, v[u].y), amax(vm.z, v[u].z), amax(vm.w, v[u].w));
     }
-    // threads with the same q hold the same 4 dimensions: xor over r0
-    for (int t = 4; t < 64; t <<= 1) {
+    // threads with the same q hold the same 4 dimensions
+    for (int t = 8; t < 64; t <<= 1) {
       vm.x = __builtin_fmaxf(vm.x, __shfl_xor(vm.x, t));
       vm.y = __builtin_fmaxf(vm.y, __shfl_xor(vm.y, t));
       vm.z = __builtin_fmaxf(vm.z, __shfl_xor(vm.z, t));
       vm.w = __builtin_fmaxf(vm.w, __shfl_xor(vm.w, t));
     }
-    float4 *red = (float4 *)&kt[0][0][0];  // [wave][q]
-    if ((tid & 63) < 4) red[(tid >> 6) * 4 + q] = vm;
+    float *red = &ring[0][0];  // [wave][32]
+    if (lane < 8) *(float4 *)(red + wave * kStatDims + 4 * q) = vm;
     __syncthreads();
-    if (tid < 16) {
-      const float *rf = (const float *)red;
+    if (tid < kStatDims) {
       float vs = 0.f;
-      for (int w = 0; w < 4; w++) vs = __builtin_fmaxf(vs, rf[w * 16 + tid]);
+      for (int w = 0; w < kStatThreads / 64; w++) vs = __builtin_fmaxf(vs, red[w * kStatDims + tid]);
       float vi = 0.f;
       if (vs > 0.f) {  // attention8.go:262-269
         vs = vs / 127.0f;
@@ -144,7 +160,6 @@ __global__ __launch_bounds__(256) void attn_long_stats_kernel(AttnArgs a) {
       stat[D + dg + tid] = vi;
     }
   }
-#undef IXH_STAT_LOAD
 }
 
 // Single-read prologue: one workgroup of 512 threads per (sequence, head,
@@ -779,7 +794,7 @@ void launch_attn_prologue(const AttnArgs &a, hipStream_t s) {
   if (a.max_n <= kShortSeq) {
     attn_prologue_rows_kernel<false><<<dim3(a.B, a.nh, 2), 512, 0, s>>>(a);
   } else {
-    attn_long_stats_kernel<<<dim3(a.B, a.nh, 8), 256, 0, s>>>(a);
+    attn_long_stats_kernel<<<dim3(a.B, a.nh, 4), kStatThreads, 0, s>>>(a);
     const int parts = (a.max_n + kShortSeq - 1) / kShortSeq;
     attn_prologue_rows_kernel<true><<<dim3(a.B, a.nh, 2 * parts), 512, 0, s>>>(a);
   }
