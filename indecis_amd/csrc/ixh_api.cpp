@@ -1907,15 +1907,12 @@ int matmul8_split(ixh_packed_b8 *b, float *c, const float *a, int m, int accumul
   g.Bk = M.qk.as<int8_t>();
   run_gemm(accumulate ? EPI_ACCUM : EPI_STORE, g, pb_tuning(b), ts.s);
   LAUNCHCK("matmul8");
-  std::vector<float> w;
   if (nc > 0 || bias) {
-    // the split channels' dequantised weight rows: f32(q) * scale (int8.go:336-340)
-    w.resize((size_t)std::max(nc, 1) * n);
-    for (int t = 0; t < nc; t++)
-      for (int col = 0; col < n; col++)
-        w[(size_t)t * n + col] = (float)b->rows[(size_t)col * k + cols[t]] * b->scale[col];
-    if ((rc = dw.ensure(4 * w.size()))) return rc;
-    HIPCK(hipMemcpyAsync(dw.p, w.data(), 4 * w.size(), hipMemcpyHostToDevice, ts.s));
+    if ((rc = dw.ensure(4 * (size_t)std::max(nc, 1) * n))) return rc;
+    if (nc > 0) {
+      launch_outlier_weights(M.q.as<int8_t>(), M.kp, M.sb.as<float>(), dcols.as<int>(), nc, n, dw.as<float>(), ts.s);
+      LAUNCHCK("outlier_weights");
+    }
     if (bias) {
       if ((rc = dbias.ensure(4 * (size_t)n))) return rc;
       HIPCK(hipMemcpyAsync(dbias.p, bias, 4 * (size_t)n, hipMemcpyHostToDevice, ts.s));
@@ -1925,7 +1922,7 @@ int matmul8_split(ixh_packed_b8 *b, float *c, const float *a, int m, int accumul
     LAUNCHCK("outlier_epilogue");
   }
   HIPCK(hipMemcpyAsync(c, dc.p, 4 * (size_t)m * n, hipMemcpyDeviceToHost, ts.s));
-  HIPCK(hipStreamSynchronize(ts.s));  // w and cols outlive their copies
+  HIPCK(hipStreamSynchronize(ts.s));  // cols outlives its copy
   return IXH_OK;
 }
 

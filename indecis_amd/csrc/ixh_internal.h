@@ -220,6 +220,9 @@ void model_config(const ::ixh_model *m, ::ixh_config *out);
 // ---- MatMul8Outliers / linear.apply (outliers.hip) --------------------------
 // out[j] |= bits of max_i |a[i][j]| (out zeroed first)
 void launch_colmax(const float *a, int ld, int m, int k, unsigned *out, hipStream_t s);
+// w[t][col] = f32(q[col][cols[t]]) * sb[col], q [n][ldq]
+void launch_outlier_weights(const int8_t *q, int ldq, const float *sb, const int *cols, int ncols, int n, float *w,
+                            hipStream_t s);
 // a[i][cols[t]] = 0
 void launch_zero_cols(float *a, int ld, int m, const int *cols, int ncols, hipStream_t s);
 // c[i][col] = (c + a[i][cols[0]] * w[0][col] + ...) + bias[col] (bias may be null)

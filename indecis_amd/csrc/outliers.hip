@@ -44,6 +44,14 @@ __global__ __launch_bounds__(256) void zero_cols_kernel(float *a, int ld, int m,
   a[(size_t)i * ld + cols[t]] = 0.f;
 }
 
+// w[t][col] = f32(q[col][cols[t]]) * sb[col]: the chosen channels' dequantised
+// weight rows (int8.go:336-340), from the resident int8 rows.
+__global__ __launch_bounds__(256) void outlier_weights_kernel(const int8_t *q, int ldq, const float *sb, const int *cols,
+                                                              int n, float *w) {
+  const int col = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
+  if (col < n) w[(size_t)t * n + col] = (float)q[(size_t)col * ldq + cols[t]] * sb[col];
+}
+
 __global__ __launch_bounds__(256) void outlier_epilogue_kernel(float *c, int ldc, int m, int n,
                                                                const float *a, int lda,
                                                                const int *cols, int ncols,
@@ -67,6 +75,12 @@ void launch_colmax(const float *a, int ld, int m, int k, unsigned *out, hipStrea
   if (m <= 0 || k <= 0) return;
   const dim3 grid((k + 255) / 256, (m + kColRows - 1) / kColRows);
   colmax_kernel<<<grid, 256, 0, s>>>(a, ld, m, k, out);
+}
+
+void launch_outlier_weights(const int8_t *q, int ldq, const float *sb, const int *cols, int ncols, int n, float *w,
+                            hipStream_t s) {
+  if (ncols <= 0 || n <= 0) return;
+  outlier_weights_kernel<<<dim3((n + 255) / 256, ncols), 256, 0, s>>>(q, ldq, sb, cols, n, w);
 }
 
 void launch_zero_cols(float *a, int ld, int m, const int *cols, int ncols, hipStream_t s) {
