@@ -333,8 +333,12 @@ __global__ __launch_bounds__(256) void attn_quant_q_kernel(AttnArgs a) {
 
 // Four waves a SIMD (at most 128 VGPRs) for both layer kinds: local layers
 // 116-118 us a launch on cfg4 against 129-131 at three waves a SIMD.
-template <bool GLOBAL>
-__global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
+// KSPL: waves that share 32 queries, each taking a part of every chunk's key
+// tiles; their maxima, sums of P and (exact int32) products meet in LDS. 1:
+// 256 threads; 2 and 4 for launches too small to fill the chip.
+template <bool GLOBAL, int KSPL>
+__global__ __launch_bounds__(256 * KSPL, KSPL == 1 ? 4 : 2) void attn_main_kernel(AttnArgs a) {
+  constexpr int T = 256 * KSPL;
   __shared__ __attribute__((aligned(16))) int8_t Ks[CHUNK * KS];
   __shared__ __attribute__((aligned(16))) int8_t Vs[D * VS];
   __shared__ __attribute__((aligned(16))) float kss[CHUNK];
@@ -345,7 +349,8 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
 
   // the wave index as a scalar: the tile loops and the full-tile tests
   // that derive from it are then scalar branches, not lane masks
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wid & 3, kh = wid >> 2;  // the wave's queries, its share of the keys
   // work item j = head * nblocks + entry (a sequence's query blocks are
   // consecutive entries). Workgroup L runs on XCD L % 8; each XCD takes a
   // contiguous run of items, so the query blocks of one (sequence, head)
@@ -418,9 +423,10 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
   // first LDS write, so the staging waits on memory once. Buffer loads:
   // keys past the sequence's slots read 0 (V^T rows continue into the next
   // sequence's slots, so those loads get an offset past the range).
-  static_assert(CHUNK == 256, "one key scale a thread (256 threads)");
-  constexpr int NKP = CHUNK * 4 / 256;         // 16-byte K pieces a thread
-  constexpr int NVG = D * (CHUNK / 32) / 256;  // V (dimension, group) items a thread
+  static_assert(CHUNK == 256, "one key scale a thread (the first 256)");
+  constexpr int NKP = CHUNK * 4 / T;                              // 16-byte K pieces a thread
+  constexpr int NVG = D * (CHUNK / 32) / T > 0 ? D * (CHUNK / 32) / T : 1;  // V (dimension, group) items a thread
+  constexpr bool VALL = D * (CHUNK / 32) >= T;                    // (KSPL 4: of the first 512)
   const auto krs = buf_rsrc(kglob, (uint32_t)npad * D);
   const auto ksrs = buf_rsrc(ksglob, (uint32_t)npad * 4);
   const auto vrs = buf_rsrc(vglob, (uint32_t)((D - 1) * a.Npad + npad));
@@ -434,24 +440,24 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
     v4i kw[NKP], vlo[NVG], vhi[NVG];
 #pragma unroll
     for (int i = 0; i < NKP; i++)
-      kw[i] = __builtin_amdgcn_raw_buffer_load_b128(krs, (uint32_t)((c0 + (tid >> 2) + 64 * i) * D + 16 * (tid & 3)), 0, 0);
+      kw[i] = __builtin_amdgcn_raw_buffer_load_b128(krs, (uint32_t)((c0 + (tid >> 2) + T / 4 * i) * D + 16 * (tid & 3)), 0, 0);
     const float kv = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ksrs, (uint32_t)(c0 + tid) * 4, 0, 0));
     if (with_v) {
 #pragma unroll
       for (int i = 0; i < NVG; i++) {
-        const int e = tid + 256 * i, d = e / (CHUNK / 32), g = e % (CHUNK / 32);
+        const int e = (tid + T * i) % (D * (CHUNK / 32)), d = e / (CHUNK / 32), g = e % (CHUNK / 32);
         const uint32_t off = c0 + 32 * g < npad ? (uint32_t)(d * a.Npad + c0 + 32 * g) : 0x7fffffe0u;
         vlo[i] = __builtin_amdgcn_raw_buffer_load_b128(vrs, off, 0, 0);
         vhi[i] = __builtin_amdgcn_raw_buffer_load_b128(vrs, off + 16, 0, 0);
       }
     }
 #pragma unroll
-    for (int i = 0; i < NKP; i++) *(v4i *)&Ks[((tid >> 2) + 64 * i) * KS + 16 * (tid & 3)] = kw[i];
-    kss[tid] = kv;
-    if (with_v) {
+    for (int i = 0; i < NKP; i++) *(v4i *)&Ks[((tid >> 2) + T / 4 * i) * KS + 16 * (tid & 3)] = kw[i];
+    if (T == 256 || tid < CHUNK) kss[tid] = kv;
+    if (with_v && (VALL || tid < D * (CHUNK / 32))) {
 #pragma unroll
       for (int i = 0; i < NVG; i++) {
-        const int e = tid + 256 * i, d = e / (CHUNK / 32), g = e % (CHUNK / 32);
+        const int e = tid + T * i, d = e / (CHUNK / 32), g = e % (CHUNK / 32);
         const int w[8] = {vlo[i][0], vlo[i][1], vlo[i][2], vlo[i][3], vhi[i][0], vhi[i][1], vhi[i][2], vhi[i][3]};
         const v4i o0 = {w[0], w[2], w[4], w[6]}, o1 = {w[1], w[3], w[5], w[7]};
         *(v4i *)&Vs[d * VS + 32 * g] = o0;
@@ -509,6 +515,15 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
     }
   };
 
+  // of the chunk's tiles t0 .. t1 - 1 of these queries, this wave's
+  auto my_tiles = [&](int &t0, int &t1) {
+    if constexpr (KSPL > 1) {
+      const int cnt = max(t1 - t0, 0), b0 = t0;
+      t0 = b0 + cnt * kh / KSPL;
+      t1 = b0 + cnt * (kh + 1) / KSPL;
+    }
+  };
+
   // ---- pass 1: row max of the valid scores ----
   // max_j f32(x_j * sq) = f32(max_j x_j * sq): rounding is monotone and
   // sq >= 0, so the query scale is applied once, to the max.
@@ -518,7 +533,8 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
     stage(c0, one_chunk);
     __syncthreads();
     if (one_chunk) prefix_v();
-    const int t0 = max(wt0, c0 / 32), t1 = min(wt1, (c0 + CHUNK) / 32);
+    int t0 = max(wt0, c0 / 32), t1 = min(wt1, (c0 + CHUNK) / 32);
+    my_tiles(t0, t1);
     for (int t = t0; t < t1; t++) {
       float sv[16];
       score_scale(t, c0, score_acc(t, c0), sv);
@@ -537,7 +553,15 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
       }
     }
   }
-  m = __builtin_fmaxf(m, __shfl_xor(m, 32)) * sqv;
+  m = __builtin_fmaxf(m, __shfl_xor(m, 32));
+  if constexpr (KSPL > 1) {
+    __shared__ float mx_s[4 * KSPL][32];
+    if (lane < 32) mx_s[wid][lane] = m;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < KSPL; q++) m = __builtin_fmaxf(m, mx_s[4 * q + wave][lane & 31]);
+  }
+  m = m * sqv;
 
   // ---- pass 2: P = RNE(255 exp(s - m)), O^T += V^T . P^T ----
   // P (0..255) enters the MFMA as P - 128 (an int8: the byte P ^ 0x80);
@@ -587,7 +611,8 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
       __syncthreads();
       prefix_v();
     }
-    const int t0 = max(wt0, c0 / 32), t1 = min(wt1, (c0 + CHUNK) / 32);
+    int t0 = max(wt0, c0 / 32), t1 = min(wt1, (c0 + CHUNK) / 32);
+    my_tiles(t0, t1);
     if (!GLOBAL && t1 > t0) {
       // rows of this lane: dims dt*32 + 8g + 4*(lane/32) + 0..3
 #pragma unroll
@@ -667,7 +692,7 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
     // (vpre is free: its last reader, the last prefix, passed its barrier)
     if (tid < D) vpre[0][tid] = vtot;
     __syncthreads();
-    if (wt1 > wt0) {
+    if (wt1 > wt0 && kh == 0) {
 #pragma unroll
       for (int dt = 0; dt < 2; dt++)
 #pragma unroll
@@ -681,6 +706,35 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
     }
   }
   psum += __shfl_xor(psum, 32);
+  if constexpr (KSPL > 1) {
+    // the other waves' products and sums of P, a wave's 32 registers a time
+    // through the free K and V staging areas (16 KB each: [4 waves][16][64])
+    __shared__ unsigned ps_s[4][32];
+    static_assert(4 * 16 * 64 * 4 <= CHUNK * KS && 4 * 16 * 64 * 4 <= D * VS, "partial products");
+    int4 *const pk = (int4 *)Ks + wave * (4 * 64) + lane, *const pv = (int4 *)Vs + wave * (4 * 64) + lane;
+#pragma unroll
+    for (int q = 1; q < KSPL; q++) {
+      __syncthreads();  // Ks and Vs are free (pass 2, or the part before)
+      if (kh == q) {
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          pk[64 * g] = int4{o[0][4 * g], o[0][4 * g + 1], o[0][4 * g + 2], o[0][4 * g + 3]};
+          pv[64 * g] = int4{o[1][4 * g], o[1][4 * g + 1], o[1][4 * g + 2], o[1][4 * g + 3]};
+        }
+        if (lane < 32) ps_s[wave][lane] = psum;
+      }
+      __syncthreads();
+      if (kh == 0) {
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const int4 x = pk[64 * g], y = pv[64 * g];
+          o[0][4 * g] += x.x; o[0][4 * g + 1] += x.y; o[0][4 * g + 2] += x.z; o[0][4 * g + 3] += x.w;
+          o[1][4 * g] += y.x; o[1][4 * g + 1] += y.y; o[1][4 * g + 2] += y.z; o[1][4 * g + 3] += y.w;
+        }
+        psum += ps_s[wave][lane & 31];
+      }
+    }
+  }
   // The context rows leave through LDS: each wave stages its 32 queries x
   // 64 dimensions in the free K or V staging area, then stores whole
   // 256-byte row pieces (16 lanes a query), non-temporal (the Wo kernel
@@ -688,6 +742,7 @@ __global__ __launch_bounds__(256, 4) void attn_main_kernel(AttnArgs a) {
   constexpr int OLD = D + 4;  // floats a staged row (conflict-free writes)
   static_assert(2 * 32 * OLD * 4 <= CHUNK * KS && 2 * 32 * OLD * 4 <= D * VS, "context staging");
   __syncthreads();  // every wave is past pass 2: Ks and Vs are free
+  if (KSPL > 1 && kh > 0) return;
   float *stg = (float *)(wave < 2 ? Ks : Vs) + (wave & 1) * (32 * OLD);
   const float sp = qact ? 1.0f / (float)(int)psum : 0.f;
   const float *vsd = a.vs + ((size_t)b * a.nh + h) * D;
@@ -803,11 +858,22 @@ void launch_attn_prologue(const AttnArgs &a, hipStream_t s) {
 void launch_attn_main(const AttnArgs &a, hipStream_t s) {
   if (a.nblocks <= 0) return;
   // 8 runs of (nblocks * nh + 7) / 8 items, one an XCD (see the kernel)
-  const dim3 grid(8 * ((a.nblocks * a.nh + 7) / 8));
-  if (a.window < 0)
-    attn_main_kernel<true><<<grid, 256, 0, s>>>(a);
-  else
-    attn_main_kernel<false><<<grid, 256, 0, s>>>(a);
+  const int items = a.nblocks * a.nh, cus = device_cus();
+  const dim3 grid(8 * ((items + 7) / 8));
+  // Waves that share a query block's keys. us a launch with 1, 2 and 4,
+  // global: 24 workgroups of 256 keys 12.8, 10.8, 11.6; 192 of 2,048 66, 48.5,
+  // 44.9; of 4,096 134, 95, 86; 384 of 4,096 152, 126, 159; 768 of 8,192 401,
+  // 374, 441. Local: 24 10.7, 10.0, 11.2; 192 11.6, 10.6, 11.5; 384 13.9, 18.0,
+  // 20.4. With one, a grid of less than three workgroups a CU leaves SIMDs with
+  // one wave, or with none.
+  if (a.window < 0) {
+    if (items <= cus && a.max_n > 512) attn_main_kernel<true, 4><<<grid, 1024, 0, s>>>(a);
+    else if (items <= 3 * cus) attn_main_kernel<true, 2><<<grid, 512, 0, s>>>(a);
+    else attn_main_kernel<true, 1><<<grid, 256, 0, s>>>(a);
+  } else {
+    if (items <= cus) attn_main_kernel<false, 2><<<grid, 512, 0, s>>>(a);
+    else attn_main_kernel<false, 1><<<grid, 256, 0, s>>>(a);
+  }
 }
 
 }  // namespace ixh

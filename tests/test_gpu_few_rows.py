@@ -78,3 +78,28 @@ def test_short_sequences_exact(shape, lanes, window, plant):
         got, want = gpu.encode_tokens(seqs), ora.encode_tokens(seqs)[0]
         assert f32_bits_equal(got, want), (lens[:4], mismatch_report(got, want))
     gpu.close()
+
+
+@pytest.mark.parametrize("shape,window", [("small", 128), ("bekko", 30)])
+def test_shared_keys_exact(shape, window):
+    """Attention with 1, 2 and 4 waves on a query block's keys
+    (attention_i8.hip), by the number of query blocks and the longest
+    sequence: one sequence around the chunks of 256 keys and past 512 keys,
+    and batches either side of 256 and of 768 workgroups, against the oracle
+    (the largest against one-sequence calls)."""
+    cfg = SHAPES[shape](layers=2, local_attention=window)
+    w = Weights.random(cfg, seed=103)
+    gpu, ora = Model(w), orc.OracleModel(w)
+    rng = np.random.default_rng(103)
+    for lens in ((129,), (255, 3), (256, 130), (257,), (512, 2), (513,), (545, 40), (1025, 1)):
+        seqs = seqs_of(rng, cfg.vocab, *lens)
+        got, want = gpu.encode_tokens(seqs), ora.encode_tokens(seqs)[0]
+        assert f32_bits_equal(got, want), (lens, mismatch_report(got, want))
+    gpu.set_option("parts", 1)
+    for items in (256, 768):
+        for blocks in (items // cfg.heads, items // cfg.heads + 1):
+            seqs = seqs_of(rng, cfg.vocab, *[150, 129] * (blocks // 4), *[140] * ((blocks % 4) // 2), *[9] * (blocks % 2))
+            got = gpu.encode_seqs(seqs)
+            want = np.concatenate([gpu.encode_seqs([s]) for s in seqs])
+            assert f32_bits_equal(got, want), (blocks, mismatch_report(got, want))
+    gpu.close()
