@@ -548,6 +548,14 @@ int split_rows_max(int H) { return H == 768 ? 3072 : H == 384 ? 4096 : 2048; }
 // 32-row block costs as much as a 64-row one.
 constexpr int kMlp32RowsMax = 8192;
 
+// Most rows of a pass whose embedding LayerNorm runs with 32 threads a row
+// (ln_rows_kernel, rownorm.hip): us a launch on it and on the segment kernel,
+// hidden 768, 6.7 and 14.3 at 24 rows, 9.8 and 16.6 at 4,096, 25.1 and 24.2 at
+// 16,384, 44 and 41 at 32,768. The final LayerNorm, which gathers no rows, takes
+// it at every size: 4.6 and 8.2 at 24 rows, 34 and 39 at 32,768, 72 and 78 at
+// 73,728 (hidden 384, 65,536 rows: 33 and 43).
+constexpr int kFewRowsMax = 8192;
+
 // What a forward pass issued but has not waited for: its profiling records
 // and the RoPE tables its kernels read.
 struct Pending {
@@ -725,6 +733,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
     ra.qk_rows = N;
   }
   ra.seg = tune.ln_seg;
+  ra.few = !tune.fixed && N <= kFewRowsMax;
   RUN("emb_ln_quant", 0, dN * (4 + row_bytes + 4 * dH + dH + 4), launch_rownorm(ra, st));
 
   auto gemm = [&](int epi, const Mat &M, int Kp, float *C, int ldc, int n_valid) {
@@ -790,6 +799,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   ln.ldq = KpH;
   ln.sa = w->sa.as<float>();
   ln.seg = tune.ln_seg;
+  ln.few = !tune.fixed;
   const double ln_bytes = dN * (4 * dH + dH + 4);
 
   float *const cmax = stream_ctx || split ? w->cmax.as<float>() : nullptr;
@@ -898,17 +908,13 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
         r.M = N;
         return r;
       };
-      LnRowsArgs lr{};
-      lr.x = w->x.as<float>();
-      lr.M = N;
-      lr.H = H;
+      RowArgs lr = ln;
       lr.gamma = L.mlp_norm.as<float>();
-      lr.eps = c.norm_eps;
       lr.qk = w->xqk.as<int8_t>();
-      lr.sa = w->sa.as<float>();
+      lr.qk_rows = N;
       RUN("gemm_wo", 2 * dN * dH * dH, res_bytes(dH, false),
           launch_res_split(product(L.o, w->ctx.as<float>(), H, cmax, nh, w->x.as<float>(), H, H), st));
-      RUN("ln_quant", 0, ln_bytes, launch_ln_rows(lr, c.lanes, st));
+      RUN("ln_quant", 0, ln_bytes, launch_rownorm(lr, st));
       float *const gm = w->gmax.as<float>();
       RUN("gemm_wi", 2 * dN * 2 * dI * dH, gemm_bytes(dH, 2 * dI, dI, false),
           launch_wi_split(product(L.i, nullptr, H, gm, I / 32, w->g.as<float>(), I, 2 * I), st));
@@ -917,9 +923,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
       if (l + 1 < c.layers) {
         lr.gamma = m->layers[l + 1].attn_norm.as<float>();
         lr.qk = kblock ? w->xqk.as<int8_t>() : nullptr;
-        lr.q = kblock ? nullptr : w->xq.as<int8_t>();
-        lr.ldq = KpH;
-        RUN("ln_quant", 0, ln_bytes, launch_ln_rows(lr, c.lanes, st));
+        RUN("ln_quant", 0, ln_bytes, launch_rownorm(lr, st));
         ln_done = true;
       }
       continue;
@@ -1027,6 +1031,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
     r.eps = c.norm_eps;
     r.lanes = c.lanes;
     r.seg = tune.ln_seg;
+    r.few = !tune.fixed;
     r.out = xn;
     RUN("final_norm", 0, dN * 8 * dH, launch_rownorm(r, st));
   }

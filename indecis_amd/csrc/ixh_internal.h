@@ -194,20 +194,6 @@ struct SplitArgs {
 bool split_rows_supported(int H, int I, int KpH, int KpI);
 void launch_wi_split(const SplitArgs &a, hipStream_t s);
 void launch_res_split(const SplitArgs &a, hipStream_t s);
-// LayerNorm + quantizeA of the rows of x [M][H]: sa [M], and q [M][ldq] or
-// K-blocked qk [H/32][M][32], whichever is not null.
-struct LnRowsArgs {
-  const float *x;
-  int M, H;
-  const float *gamma;
-  double eps;
-  int8_t *q;
-  int ldq;
-  int8_t *qk;
-  float *sa;
-};
-void launch_ln_rows(const LnRowsArgs &a, int lanes, hipStream_t s);
-
 // ---- host helpers (ixh_api.cpp) ---------------------------------------------
 // Sets the calling thread's ixh_last_error message; returns code.
 int set_error(int code, const char *msg);
@@ -255,6 +241,7 @@ struct RowArgs {
   // [H/32][qk_rows][32] (H a multiple of 32; nothing is written to q)
   int8_t *qk = nullptr;
   int qk_rows = 0;
+  int few = 0;  // the kernel of 32 threads a row, where the shape allows it
 };
 void launch_rownorm(const RowArgs &a, hipStream_t s);
 

@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace ixh {
 
@@ -834,10 +835,142 @@ void launch_resident(Kern kern, int work, int threads, const RowArgs &a, hipStre
   kern<<<std::min(work, n), threads, 0, s>>>(a);
 }
 
+// LayerNorm (vec_simd.go:285-327) of ROWS rows a workgroup, 32 threads a row
+// holding its values in registers, the lane chains over a copy in LDS. At few
+// rows what bounds it is latency (the row's load, then H / V dependent adds
+// twice): a workgroup takes few rows and a row many threads, 4.6 us for 24 rows
+// of 768 where the segment kernel takes 8.2; at many, HBM (6.3 TB/s at 73,728).
+template <int H, int V, bool GATHER>
+__global__ __launch_bounds__(256) void ln_rows_kernel(RowArgs a) {
+  constexpr int ROWS = 8, LD = H + 8;  // floats a row in LDS
+  constexpr int C4 = H / 128;          // float4 a thread
+  __shared__ __attribute__((aligned(16))) float xs[ROWS * LD];
+  __shared__ float mean_s[ROWS], rstd_s[ROWS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int r = tid >> 5, c = tid & 31, m0 = ROWS * blockIdx.x;
+  const int row = min(m0 + r, a.M - 1);
+  const std::conditional_t<GATHER, RowSrc, RowLoad<0>> src(a, row);
+  float4 v[C4], g[C4];
+#pragma unroll
+  for (int u = 0; u < C4; u++) v[u] = src.load4(4 * (c + 32 * u));
+#pragma unroll
+  for (int u = 0; u < C4; u++) g[u] = *(const float4 *)(a.gamma + 4 * (c + 32 * u));
+#pragma unroll
+  for (int u = 0; u < C4; u++) *(float4 *)&xs[r * LD + 4 * (c + 32 * u)] = v[u];
+  __syncthreads();
+  // chain ch: lane partial ch % V of row ch / V (V 0: one float64 chain a row)
+  constexpr int NCH = V > 0 ? ROWS * V : ROWS;
+  if (tid < (NCH + 63) / 64 * 64) {
+    const int ch = min(tid, NCH - 1), cr = V > 0 ? ch / (V > 0 ? V : 1) : ch;
+    float mean = 0.f;
+#pragma unroll
+    for (int pass = 0; pass < 2; pass++) {
+      double sum = 0.0;
+      if constexpr (V > 0) {
+        const float *xr = xs + cr * LD + ch % V;
+        constexpr int NE = H / V, NB = NE % 16 == 0 ? 16 : 8;  // values a lane, a batch of them
+        static_assert(NE % NB == 0, "whole batches");
+        float p = 0.f, b[NB], n[NB];
+#pragma unroll
+        for (int e = 0; e < NB; e++) b[e] = xr[V * e];
+#pragma unroll
+        for (int e0 = 0; e0 < NE; e0 += NB) {
+          if (e0 + NB < NE) {
+#pragma unroll
+            for (int e = 0; e < NB; e++) n[e] = xr[V * (e0 + NB + e)];
+          }
+#pragma unroll
+          for (int e = 0; e < NB; e++) {
+            if (pass == 0) {
+              p = p + b[e];
+            } else {
+              const float d = b[e] - mean;
+              p = __builtin_fmaf(d, d, p);
+            }
+          }
+#pragma unroll
+          for (int e = 0; e < NB; e++) b[e] = n[e];
+        }
+        const int base = lane & ~(V - 1);
+#pragma unroll
+        for (int q = 0; q < V; q++) sum += (double)__shfl(p, base + q);
+      } else {
+        const float *xr = xs + cr * LD;
+        for (int e = 0; e < H; e++) {
+          if (pass == 0) {
+            sum += (double)xr[e];
+          } else {
+            const double d = (double)(xr[e] - mean);
+            sum += d * d;
+          }
+        }
+      }
+      if (pass == 0) {
+        mean = (float)(sum / (double)H);
+      } else if (tid < NCH && (V == 0 || tid % (V > 0 ? V : 1) == 0)) {
+        mean_s[cr] = mean;
+        rstd_s[cr] = (float)(1.0 / __builtin_sqrt(sum / (double)H + a.eps));
+      }
+    }
+  }
+  __syncthreads();
+  const float mean = mean_s[r], rstd = rstd_s[r];
+  float mx = 0.f;
+#pragma unroll
+  for (int u = 0; u < C4; u++) {
+    v[u] = make_float4(((v[u].x - mean) * rstd) * g[u].x, ((v[u].y - mean) * rstd) * g[u].y,
+                       ((v[u].z - mean) * rstd) * g[u].z, ((v[u].w - mean) * rstd) * g[u].w);
+    mx = amax(amax(amax(amax(mx, v[u].x), v[u].y), v[u].z), v[u].w);
+    if (a.out && m0 + r < a.M) *(float4 *)(a.out + (size_t)row * H + 4 * (c + 32 * u)) = v[u];
+  }
+  if (!a.q && !a.qk) return;
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, o));
+  float s = 0.f, inv = 0.f;
+  if (mx != 0.f) {
+    s = mx / 127.0f;
+    inv = 1.0f / s;
+  }
+  if (m0 + r >= a.M) return;
+  if (c == 0) a.sa[row] = s;
+#pragma unroll
+  for (int u = 0; u < C4; u++) {
+    const float4 t = v[u];
+    *(int *)qbyte(a, row, 4 * (c + 32 * u)) = (q8(t.x, inv) & 0xff) | ((q8(t.y, inv) & 0xff) << 8) |
+                                              ((q8(t.z, inv) & 0xff) << 16) | (q8(t.w, inv) << 24);
+  }
+}
+
+template <int H, int V>
+void launch_ln_rows_v(const RowArgs &a, hipStream_t s) {
+  const int grid = (a.M + 7) / 8;
+  if (a.ids) ln_rows_kernel<H, V, true><<<grid, 256, 0, s>>>(a);
+  else ln_rows_kernel<H, V, false><<<grid, 256, 0, s>>>(a);
+}
+template <int H>
+void launch_ln_rows(const RowArgs &a, hipStream_t s) {
+  switch (a.lanes) {
+  case 0: launch_ln_rows_v<H, 0>(a, s); break;
+  case 4: launch_ln_rows_v<H, 4>(a, s); break;
+  case 8: launch_ln_rows_v<H, 8>(a, s); break;
+  default: launch_ln_rows_v<H, 16>(a, s); break;
+  }
+}
+// The rows kernel's: LayerNorm at the model widths, quantised rows unpadded.
+bool ln_rows_fits(const RowArgs &a) {
+  return a.few && a.gamma && (a.H == 768 || a.H == 384 || a.H == 256) && (!a.q || a.qk || a.ldq == a.H);
+}
+
 }  // namespace
 
 void launch_rownorm(const RowArgs &a, hipStream_t s) {
   if (a.M <= 0) return;
+  if (ln_rows_fits(a)) {
+    if (a.H == 768) launch_ln_rows<768>(a, s);
+    else if (a.H == 384) launch_ln_rows<384>(a, s);
+    else launch_ln_rows<256>(a, s);
+    return;
+  }
   const int src = !a.ids ? 0 : a.emb_format == 0 ? 1 : a.emb_format == 1 ? 2 : 3;
   if ((a.lanes == 8 || a.lanes == 16) && a.H == 384 && a.seg != 0) {
     // a 256-column segment and a 128-column one

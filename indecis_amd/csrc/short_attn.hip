@@ -101,6 +101,38 @@ __global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a)
   };
 #pragma unroll
   for (int k = 0; k < PF; k++) load(k, k);
+  // what the dequantisation needs: with one row block loaded here, its
+  // latency under the products'; with more, after them (registers)
+  float4 pcos[GO], psin[GO], psb[2][GO];
+  float psa[GO][4], vsb[2], vzc[2];
+  int vc1[2];
+  auto constants = [&] {
+    if (part < 2) {
+      psa[0][0] = g.sa[base + tok];
+#pragma unroll
+      for (int q = 0; q < GO; q++) {
+        const int d0 = 16 * fh + 4 * (GO * ks + q);
+        pcos[q] = *(const float4 *)(g.rope_cos + (size_t)tok * 32 + d0);
+        psin[q] = *(const float4 *)(g.rope_sin + (size_t)tok * 32 + d0);
+        psb[0][q] = *(const float4 *)(g.sb + wrow + d0);
+        psb[1][q] = *(const float4 *)(g.sb + wrow + d0 + 32);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const int ch = wrow + 32 * j + fr;
+        vsb[j] = g.sb[ch];
+        vzc[j] = g.zc[ch];
+        vc1[j] = g.c128[ch];
+      }
+#pragma unroll
+      for (int q = 0; q < GO; q++)
+#pragma unroll
+        for (int u = 0; u < 4; u++)  // rows past n: row n-1 again
+          psa[q][u] = g.sa[base + min(32 * rt + 8 * (GO * ks + q) + 4 * fh + u, n - 1)];
+    }
+  };
+  if constexpr (RT == 1) constants();
   const bool small = g.small;
   v16i acc[2] = {};
   auto products = [&](auto vpart) {
@@ -134,16 +166,17 @@ __global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a)
   }
 
   // ---- dequantisation; RoPE and the float32 Q and K; max |V| ----
+  if constexpr (RT > 1) constants();
   float v[2][GO][4];  // V: rows 8 (GO ks + q) + 4 fh + u of the block, dimension 32 j + fr
   if (part < 2) {
-    const float sa = g.sa[base + tok];
+    const float sa = psa[0][0];
     float *const dst = (part ? kf : qf) + (32 * rt + fr) * FLD;
 #pragma unroll
     for (int q = 0; q < GO; q++) {
       const int d0 = 16 * fh + 4 * (GO * ks + q), ch = wrow + d0;
-      const float4 c = *(const float4 *)(g.rope_cos + (size_t)tok * 32 + d0), s = *(const float4 *)(g.rope_sin + (size_t)tok * 32 + d0);
-      const float4 x1 = deq4(sum[0][q], small, g.c128 + ch, g.zc + ch, *(const float4 *)(g.sb + ch), sa);
-      const float4 x2 = deq4(sum[1][q], small, g.c128 + ch + 32, g.zc + ch + 32, *(const float4 *)(g.sb + ch + 32), sa);
+      const float4 c = pcos[q], s = psin[q];
+      const float4 x1 = deq4(sum[0][q], small, g.c128 + ch, g.zc + ch, psb[0][q], sa);
+      const float4 x2 = deq4(sum[1][q], small, g.c128 + ch + 32, g.zc + ch + 32, psb[1][q], sa);
       // linalg.Rope (vec_simd.go:408-425): x1' = x1*c - x2*s, x2' = x2*c + x1*s
       *(float4 *)(dst + d0) = make_float4(x1.x * c.x - x2.x * s.x, x1.y * c.y - x2.y * s.y, x1.z * c.z - x2.z * s.z, x1.w * c.w - x2.w * s.w);
       *(float4 *)(dst + 32 + d0) = make_float4(x2.x * c.x + x1.x * s.x, x2.y * c.y + x1.y * s.y, x2.z * c.z + x1.z * s.z, x2.w * c.w + x1.w * s.w);
@@ -152,17 +185,13 @@ __global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a)
     float vm[2] = {0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      const int ch = wrow + 32 * j + fr;
-      const float sb = g.sb[ch], zc = g.zc[ch];
-      const int c1 = g.c128[ch];
 #pragma unroll
       for (int q = 0; q < GO; q++)
 #pragma unroll
         for (int u = 0; u < 4; u++) {
           // rows past n are row n-1 again: they leave the maximum as it is
-          const float sa = g.sa[base + min(32 * rt + 8 * (GO * ks + q) + 4 * fh + u, n - 1)];
           const int t = u == 0 ? sum[j][q].x : u == 1 ? sum[j][q].y : u == 2 ? sum[j][q].z : sum[j][q].w;
-          v[j][q][u] = small ? ((float)t * sb) * sa : deq(t + c1, zc, sb, sa);
+          v[j][q][u] = small ? ((float)t * vsb[j]) * psa[q][u] : deq(t + vc1[j], vzc[j], vsb[j], psa[q][u]);
           vm[j] = amax(vm[j], v[j][q][u]);
         }
       vm[j] = __builtin_fmaxf(vm[j], __shfl_xor(vm[j], 32));

@@ -7,8 +7,7 @@
 // GeluMul, MatMul8N of g into x, the next attn_norm), with the same
 // arithmetic: quantizeA of the input rows (int8.go:160-191), q*w summed in
 // int32 by v_mfma_i32_32x32x32_i8, the reference tile's dequantisation
-// ((f32(tile) - zc) * sb) * sa, GELU in the FMA form, the LayerNorm's V
-// float32 lane chains in column order combined in float64 in lane order.
+// ((f32(tile) - zc) * sb) * sa, GELU in the FMA form.
 //
 // Why: a whole-row kernel gives 32 or 64 rows to one workgroup, which then
 // streams every weight of the block through one CU; one row costs it as
@@ -25,11 +24,10 @@
 //  wi_split_kernel   g tile = GeGLU(xn . Wi^T): one workgroup per (32 rows,
 //      gated tile of 32 columns), 4 waves over the depth; also max |g| of
 //      each row's 32 columns.
-//  ln_rows_kernel    LayerNorm + quantizeA of 8 rows a workgroup.
 //
 // What bounds them: latency at few rows. At 24 rows of hidden 768 (36 and 24 workgroups)
-// a launch takes 4.9 us (Wi), 5.1 us (Wo) and 6.4 us (WoMLP), LayerNorm 4.8
-// us: against 25 us (Wo + LayerNorm) and 50 us (the MLP block) on the
+// a launch takes 4.9 us (Wi), 5.1 us (Wo) and 6.4 us (WoMLP), the LayerNorm
+// between them (ln_rows_kernel, rownorm.hip) 4.8: against 25 us (Wo + LayerNorm) and 50 us (the MLP block) on the
 // whole-row kernels, and 2.05 -> 0.93 ms a pass of 22 layers. A wave's
 // global loads are all issued before its first MFMA. With more rows, the
 // float32 rows read from L2 and the last-level cache by every tile's
@@ -199,118 +197,6 @@ __global__ __launch_bounds__(64 * KS * CT) void res_split_kernel(SplitArgs a) {
   }
 }
 
-// LayerNorm (vec_simd.go:285-327) and quantizeA of ROWS rows a workgroup:
-// 32 threads a row hold its values in registers, the lane chains run over
-// a copy in LDS.
-template <int H, int V>
-__global__ __launch_bounds__(256) void ln_rows_kernel(LnRowsArgs a) {
-  constexpr int ROWS = 8, LD = H + 8;  // floats a row in LDS
-  constexpr int C4 = H / 128;          // float4 a thread
-  __shared__ __attribute__((aligned(16))) float xs[ROWS * LD];
-  __shared__ float mean_s[ROWS], rstd_s[ROWS];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int r = tid >> 5, c = tid & 31, m0 = ROWS * blockIdx.x;
-  const int row = min(m0 + r, a.M - 1);
-  float4 v[C4], g[C4];
-#pragma unroll
-  for (int u = 0; u < C4; u++) v[u] = *(const float4 *)(a.x + (size_t)row * H + 4 * (c + 32 * u));
-#pragma unroll
-  for (int u = 0; u < C4; u++) g[u] = *(const float4 *)(a.gamma + 4 * (c + 32 * u));
-#pragma unroll
-  for (int u = 0; u < C4; u++) *(float4 *)&xs[r * LD + 4 * (c + 32 * u)] = v[u];
-  __syncthreads();
-  // chain ch: lane partial ch % V of row ch / V (V 0: one float64 chain a row)
-  constexpr int NCH = V > 0 ? ROWS * V : ROWS;
-  if (tid < (NCH + 63) / 64 * 64) {
-    const int ch = min(tid, NCH - 1), cr = V > 0 ? ch / (V > 0 ? V : 1) : ch;
-    float mean = 0.f;
-#pragma unroll
-    for (int pass = 0; pass < 2; pass++) {
-      double sum = 0.0;
-      if constexpr (V > 0) {
-        const float *xr = xs + cr * LD + ch % V;
-        constexpr int NE = H / V, NB = NE % 16 == 0 ? 16 : 8;  // values a lane, a batch of them
-        static_assert(NE % NB == 0, "whole batches");
-        float p = 0.f, b[NB], n[NB];
-#pragma unroll
-        for (int e = 0; e < NB; e++) b[e] = xr[V * e];
-#pragma unroll
-        for (int e0 = 0; e0 < NE; e0 += NB) {
-          if (e0 + NB < NE) {
-#pragma unroll
-            for (int e = 0; e < NB; e++) n[e] = xr[V * (e0 + NB + e)];
-          }
-#pragma unroll
-          for (int e = 0; e < NB; e++) {
-            if (pass == 0) {
-              p = p + b[e];
-            } else {
-              const float d = b[e] - mean;
-              p = __builtin_fmaf(d, d, p);
-            }
-          }
-#pragma unroll
-          for (int e = 0; e < NB; e++) b[e] = n[e];
-        }
-        const int base = lane & ~(V - 1);
-#pragma unroll
-        for (int q = 0; q < V; q++) sum += (double)__shfl(p, base + q);
-      } else {
-        const float *xr = xs + cr * LD;
-        for (int e = 0; e < H; e++) {
-          if (pass == 0) {
-            sum += (double)xr[e];
-          } else {
-            const double d = (double)(xr[e] - mean);
-            sum += d * d;
-          }
-        }
-      }
-      if (pass == 0) {
-        mean = (float)(sum / (double)H);
-      } else if (tid < NCH && (V == 0 || tid % (V > 0 ? V : 1) == 0)) {
-        mean_s[cr] = mean;
-        rstd_s[cr] = (float)(1.0 / __builtin_sqrt(sum / (double)H + a.eps));
-      }
-    }
-  }
-  __syncthreads();
-  const float mean = mean_s[r], rstd = rstd_s[r];
-  float mx = 0.f;
-#pragma unroll
-  for (int u = 0; u < C4; u++) {
-    v[u] = make_float4(((v[u].x - mean) * rstd) * g[u].x, ((v[u].y - mean) * rstd) * g[u].y,
-                       ((v[u].z - mean) * rstd) * g[u].z, ((v[u].w - mean) * rstd) * g[u].w);
-    mx = amax(amax(amax(amax(mx, v[u].x), v[u].y), v[u].z), v[u].w);
-  }
-#pragma unroll
-  for (int o = 1; o < 32; o <<= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, o));
-  float s = 0.f, inv = 0.f;
-  if (mx != 0.f) {
-    s = mx / 127.0f;
-    inv = 1.0f / s;
-  }
-  if (m0 + r >= a.M) return;
-  if (c == 0) a.sa[row] = s;
-#pragma unroll
-  for (int u = 0; u < C4; u++) {
-    const int col = 4 * (c + 32 * u), w = pack4(v[u], inv);
-    if (a.qk) *(int *)(a.qk + ((size_t)(col >> 5) * a.M + row) * 32 + (col & 31)) = w;
-    if (a.q) *(int *)(a.q + (size_t)row * a.ldq + col) = w;
-  }
-}
-
-template <int H>
-void launch_ln(const LnRowsArgs &a, int lanes, hipStream_t s) {
-  const int grid = (a.M + 7) / 8;
-  switch (lanes) {
-  case 0: ln_rows_kernel<H, 0><<<grid, 256, 0, s>>>(a); break;
-  case 4: ln_rows_kernel<H, 4><<<grid, 256, 0, s>>>(a); break;
-  case 8: ln_rows_kernel<H, 8><<<grid, 256, 0, s>>>(a); break;
-  default: ln_rows_kernel<H, 16><<<grid, 256, 0, s>>>(a); break;
-  }
-}
-
 }  // namespace
 
 bool split_rows_supported(int H, int I, int KpH, int KpI) {
@@ -345,13 +231,6 @@ void launch_res_split(const SplitArgs &a, hipStream_t s) {
   else if (a.K == 512) res_one<16>(a, s);
   else if (a.K == 384) res_one<12>(a, s);
   else res_one<8>(a, s);
-}
-
-void launch_ln_rows(const LnRowsArgs &a, int lanes, hipStream_t s) {
-  if (a.M <= 0) return;
-  if (a.H == 768) launch_ln<768>(a, lanes, s);
-  else if (a.H == 384) launch_ln<384>(a, lanes, s);
-  else launch_ln<256>(a, lanes, s);
 }
 
 }  // namespace ixh
