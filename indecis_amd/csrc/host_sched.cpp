@@ -114,6 +114,28 @@ int check_offs(const int32_t *offs, int B) {
   return IXH_OK;
 }
 
+void qkv_groups(const int32_t *offs, const std::vector<int32_t> &order, std::vector<int32_t> &groups) {
+  groups.clear();
+  std::vector<int> open[9];  // groups with w free waves (w 1 .. 7)
+  for (int32_t b : order) {
+    const int n = offs[b + 1] - offs[b];
+    const int nw = std::max(2, std::min(8, (n + 63) / 64 * 2));
+    int w = nw;
+    while (w < 8 && (nw == 8 || open[w].empty())) w++;  // the fullest group it fits into
+    int g;
+    if (w < 8) {
+      g = open[w].back();
+      open[w].pop_back();
+    } else {
+      g = (int)groups.size() / 8;
+      groups.insert(groups.end(), 8, -1);
+    }
+    const int first = 8 - w;
+    for (int k = 0; k < nw; k++) groups[8 * g + first + k] = 16 * b + k;
+    if (w - nw > 0) open[w - nw].push_back(g);
+  }
+}
+
 // Rows do not depend on their batch (TestMatMul8RowsIndependent), so the
 // results of several passes are those of one.
 int plan_passes(const Tuning &t, int H, int I, const int32_t *offs, int B, std::vector<int> &cut) {

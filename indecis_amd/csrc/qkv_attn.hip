@@ -35,7 +35,11 @@
 // K loop (64 rows x Kp bytes, K-blocked from the weights' K-blocked copy),
 // and each wave streams its own row blocks' fragments into registers, PF
 // K-blocks ahead: no ring, no barrier in the K loop, LDS read traffic of B
-// only.
+// only. A workgroup's time is about 4.7 us + 0.03 us a row whatever its
+// sequence, so here the waves of one workgroup are shared out among several
+// sequences of at most 256 rows (qkv_groups, host_sched.h: a wave a row
+// block): 128 tokens a sequence 157 -> 118 us a launch of 32,768 rows, 64 tokens
+// (hidden 256) 74 -> 35 of 35,000.
 #include <type_traits>
 
 #include "ixh_device.h"
@@ -72,14 +76,14 @@ __device__ __forceinline__ void wait_vmcnt_upto(int n) {
 }
 
 template <int NH, bool KB>
-__global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnArgs a, const int32_t *order) {
+__global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnArgs a, const int32_t *work, int nwork) {
   static_assert(!KB || NH == 1, "K-blocked input: one head a workgroup");
   using S = Shape<NH>;
   constexpr int NW = S::NW, RING = S::RING, STAGE = S::STAGE;
   extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
   __shared__ float sa_s[SEQ_MAX];
   __shared__ float red_s[NH][8][D];
-  __shared__ __attribute__((aligned(16))) float stat_s[NH][D];
+  __shared__ __attribute__((aligned(16))) float stat_s[KB ? 8 : NH][D];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hf = wave >> 3, wv = wave & 7, tidh = tid & 511;  // half, wave and thread in the half
   const int fr = lane & 31, fh = lane >> 5;
@@ -87,17 +91,27 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   const int per_seq = 3 * hgroups;
   const int xcd = blockIdx.x % NXCD, k = blockIdx.x / NXCD;
   const int si = xcd + NXCD * (k / per_seq);
-  if (si >= a.B) return;
-  const int b = order[si];
+  if (si >= nwork) return;
+  // this wave's sequence and first row block in it (its second is 8 on): KB,
+  // from the table (-1: none); else the workgroup's sequence, block wv
+  const int ent = KB ? __builtin_amdgcn_readfirstlane(work[8 * si + wv]) : 16 * work[si] + wv;
+  const bool valid = !KB || ent >= 0;
+  const int b = valid ? ent >> 4 : 0, rb0 = valid ? ent & 15 : 0;
   const int part = (k % per_seq) / hgroups, h0 = NH * ((k % per_seq) % hgroups), h = h0 + hf;
-  const int base = a.offs[b], n = a.offs[b + 1] - base;
+  const int base = a.offs[b], n = valid ? a.offs[b + 1] - base : 0;
+  const int last = max(n - 1, 0);  // the row that stands for those past n
   const int slot0 = a.padoff[b];  // the sequence's first key slot (K and V outputs)
   const int npad = (n + kKeyPad - 1) / kKeyPad * kKeyPad;
   const int nb = npad / 32;            // 32-row blocks stored (even, at most 16)
   const int nbc = (n + 31) / 32;       // blocks computed: a block past n is all zeros
+  const int sw = KB ? wv - rb0 : hf;   // the sequence's place in stat_s (KB: its first wave)
+  // whether the workgroup's waves have second blocks: one sequence over 256
+  // rows (wave 0 always has a sequence)
+  const int b0 = KB ? work[8 * si] >> 4 : b;
+  const bool two_rounds = a.offs[b0 + 1] - a.offs[b0] > 256;
   const int col0 = part * a.H + h * D;   // this half's head: first output column
   const int colb = part * a.H + h0 * D;  // the workgroup's first weight row
-  if (n == 0) {
+  if (!KB && n == 0) {
     if (part == 2 && tidh < D) a.vs[((size_t)b * a.nh + h) * D + tidh] = 0.f;
     return;
   }
@@ -105,7 +119,10 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   // retire in order, so the loop's first wait covers them): the row scales
   // (stored to LDS after the loop) and this lane's column constants.
   static_assert(SEQ_MAX <= 512, "one row scale a thread");
-  const float sa_v = tid < 32 * nb ? g.sa[base + min(tid, n - 1)] : 0.f;
+  // KB: lanes 0-31 the rows of the wave's first block, 32-63 of its second
+  // (an empty sequence at the batch's end has no row of its own)
+  const float sa_v = KB ? g.sa[min(base + min(32 * (rb0 + 8 * fh) + fr, last), a.N - 1)]
+                        : tid < 32 * nb ? g.sa[base + min(tid, n - 1)] : 0.f;
   float zc[2], sb[2];
   int c128[2];
 #pragma unroll
@@ -184,9 +201,9 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     const auto ars = buf_rsrc(g.Ak, (uint32_t)nkb * g.ak_rows * 32);
     uint32_t avo[2];
 #pragma unroll
-    for (int i = 0; i < 2; i++) avo[i] = (uint32_t)(base + min(32 * (wv_u + 8 * i) + fr, n - 1)) * 32 + 16 * fh;
+    for (int i = 0; i < 2; i++) avo[i] = (uint32_t)(base + min(32 * (rb0 + 8 * i) + fr, last)) * 32 + 16 * fh;
     const uint32_t akstep = (uint32_t)g.ak_rows * 32;
-    const bool two = wv_u + 8 < nbc;  // this wave's second row block
+    const bool two = rb0 + 8 < nbc;  // this wave's second row block
     // Both row blocks' fragments are loaded every K-block, past the last
     // K-block the last one again, whether or not the wave has a second
     // block (then row n-1: one 32-byte piece): with a load count that does
@@ -220,7 +237,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
         loadA(kb + PF, fa[u]);
       }
     };
-    if (wv_u < nbc) {
+    if (rb0 < nbc) {
       round(0, std::true_type{});
       for (int k0 = PF; k0 < nkb; k0 += PF) round(k0, std::false_type{});
     }
@@ -257,7 +274,8 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     }
   }
   }  // !KB
-  if (tid < 32 * nb) sa_s[tid] = sa_v;
+  if constexpr (KB) sa_s[32 * (wv + 8 * fh) + fr] = sa_v;
+  else if (tid < 32 * nb) sa_s[tid] = sa_v;
   __syncthreads();  // the ring is no longer read; the row scales are in LDS
 
   // ---- dequantisation (and RoPE on Q and K) in the MFMA layout ----
@@ -273,18 +291,18 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   auto tables = [&](int i) {
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      const int p = min(32 * (wv + 8 * i) + 8 * u + (lane >> 3), n - 1);
+      const int p = min(32 * (rb0 + 8 * i) + 8 * u + (lane >> 3), last);
       const size_t off = (size_t)p * 32 + 4 * (lane & 7);
       __builtin_amdgcn_global_load_lds((glb_ptr)(g.rope_cos + off), (lds_ptr)(smem + wave * 8192 + 1024 * u), 16, 0, 0);
       __builtin_amdgcn_global_load_lds((glb_ptr)(g.rope_sin + off), (lds_ptr)(smem + wave * 8192 + 4096 + 1024 * u), 16, 0, 0);
     }
   };
-  if (rope && wv < nbc) tables(0);
+  if (rope && rb0 < nbc) tables(0);
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     // a block past n (stored as padding keys) is not computed: its values
     // reach only rows past n, which every store below writes as zeros
-    if (wv + 8 * i >= nbc) continue;
+    if (rb0 + 8 * i >= nbc) continue;
     if (g.small) {
       // the weights' bound holds (checked on upload): f32(acc + 128
       // colsum) - zc is f32(acc) exactly
@@ -306,7 +324,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   if (rope) {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      if (wv + 8 * i >= nbc) continue;
+      if (rb0 + 8 * i >= nbc) continue;
       if (i == 1) {
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt 0: this wave's reads of the first tables returned
         tables(1);
@@ -332,7 +350,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     // they are; a block past n that was not computed is left out
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      if (wv + 8 * i >= nbc) continue;
+      if (rb0 + 8 * i >= nbc) continue;
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         vm[0] = amax(vm[0], v[i][0][r]);
@@ -345,24 +363,25 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
       if (fh == 0) red_s[hf][wv][32 * j + fr] = vm[j];
     }
     __syncthreads();
-    if (tidh < D) {
+    // over the sequence's waves (KB: from its first, sw; the others hold 0)
+    float vi[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
       float vs = 0.f;
-      for (int w = 0; w < 8; w++) vs = __builtin_fmaxf(vs, red_s[hf][w][tidh]);
-      float vi = 0.f;
+      const int w0 = KB ? sw : 0, w1 = KB ? min(sw + nbc, 8) : 8;
+      for (int w = w0; w < w1; w++) vs = __builtin_fmaxf(vs, red_s[hf][w][32 * j + fr]);
+      vi[j] = 0.f;
       if (vs > 0.f) {  // attention8.go:262-269
         vs = vs / 127.0f;
-        vi = 1.0f / vs;
+        vi[j] = 1.0f / vs;
       }
-      a.vs[((size_t)b * a.nh + h) * D + tidh] = vs;
-      stat_s[hf][tidh] = vi;
+      if (valid && rb0 == 0 && fh == 0) a.vs[((size_t)b * a.nh + h) * D + 32 * j + fr] = vs;
     }
-    __syncthreads();
-    const float vi0 = stat_s[hf][fr], vi1 = stat_s[hf][32 + fr];
     int8_t *vt_s = smem + wave * (D * VT_LD);  // [64 dims][32 keys] of this wave's block
     int8_t *vt = a.vt + (size_t)h * D * a.Npad + slot0;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      const int rb = wv + 8 * i;
+      const int rb = rb0 + 8 * i;
       if (rb < nb) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
@@ -374,7 +393,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
             if (rb < nbc) {
               int qv[4];
 #pragma unroll
-              for (int u = 0; u < 4; u++) qv[u] = q8(v[i][j][4 * gq + u], j ? vi1 : vi0);
+              for (int u = 0; u < 4; u++) qv[u] = q8(v[i][j][4 * gq + u], vi[j]);
               const int lim = n - (32 * rb + 8 * gq + 4 * fh);  // keys of the four still in the sequence
               const unsigned keep = lim >= 4 ? 0xffffffffu : lim <= 0 ? 0u : (1u << (8 * lim)) - 1u;
               w = (int)(((unsigned)(qv[0] & 0xff) | ((unsigned)(qv[1] & 0xff) << 8) |
@@ -400,7 +419,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   // slab, in the MFMA layout
   float *slab = (float *)(smem + hf * SLAB_BYTES);  // [256 rows][KT_LD], one a half
 #define PUT(t)                                                    \
-  if (wv + 8 * (t) < nb) {                                        \
+  if (rb0 + 8 * (t) < nb) {                                       \
     _Pragma("unroll") for (int r = 0; r < 16; r++) {              \
       const int lr = 32 * wv + acc_row(r, lane);                  \
       slab[lr * KT_LD + fr] = v[t][0][r];                         \
@@ -413,16 +432,16 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     float ksum = 0.f;
 #pragma unroll
     for (int t = 0; t < 2; t++) {
-      if (256 * t < n) {  // block-uniform
+      if (t == 0 || two_rounds) {  // block-uniform
         PUT(t)
         __syncthreads();
-        if (wv == 0) {
+        if (rb0 == 0) {  // the sequence's first wave (none: no rows)
           // the sums stay in key order; KN slab reads are issued together
           // before their KN adds, so the chain waits on LDS once a batch
           // (KN = 8 where NH = 2 leaves fewer registers)
           constexpr int KN = NH == 1 ? 16 : 8;
           const int cnt = min(256, n - 256 * t);
-          const float *col = slab + lane;
+          const float *col = slab + 32 * wv * KT_LD + lane;
           int lr = 0;
           for (; lr + KN <= cnt; lr += KN) {
             float bt[KN];
@@ -437,7 +456,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
         __syncthreads();
       }
     }
-    if (wv == 0) stat_s[hf][lane] = ksum * (1.0f / (float)n);  // Scale(mean, 1/n)
+    if (rb0 == 0) stat_s[sw][lane] = ksum * (1.0f / (float)n);  // Scale(mean, 1/n)
     __syncthreads();
   }
 
@@ -451,9 +470,9 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   const int hh = (lane >> 4) & 1;
   const int lr = 32 * wv + 16 * (lane >> 5) + (lane & 15);
   auto quant_round = [&](int t) {
-    const int row = 256 * t + lr;
+    const int row = 32 * (rb0 + 8 * t) + 16 * (lane >> 5) + (lane & 15);
     const float4 *src = (const float4 *)(slab + lr * KT_LD + 32 * hh);
-    const float4 *mu = (const float4 *)(stat_s[hf] + 32 * hh);
+    const float4 *mu = (const float4 *)(stat_s[sw] + 32 * hh);
     // the slab is read twice (max, then quantisation): fewer live registers
     auto value = [&](int c) {
       float4 x = src[c];
@@ -502,7 +521,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   };
   if (part == 1) {
     // the slab holds the chains' last round
-    if (n > 256) {
+    if (two_rounds) {
       quant_round(1);
       __syncthreads();
       PUT(0)
@@ -513,7 +532,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     PUT(0)
     __syncthreads();
     quant_round(0);
-    if (n > 256) {
+    if (two_rounds) {
       __syncthreads();
       PUT(1)
       __syncthreads();
@@ -541,9 +560,9 @@ bool smem_ready() {
 }
 
 template <int NH, bool KB>
-void launch_nh(const GemmArgs &g, const AttnArgs &a, const int32_t *order, hipStream_t s) {
-  const int grid = NXCD * 3 * (a.nh / NH) * ((a.B + NXCD - 1) / NXCD);
-  qkv_attn_kernel<NH, KB><<<grid, 512 * NH, Shape<NH>::SMEM, s>>>(g, a, order);
+void launch_nh(const GemmArgs &g, const AttnArgs &a, const int32_t *work, int nwork, hipStream_t s) {
+  const int grid = NXCD * 3 * (a.nh / NH) * ((nwork + NXCD - 1) / NXCD);
+  qkv_attn_kernel<NH, KB><<<grid, 512 * NH, Shape<NH>::SMEM, s>>>(g, a, work, nwork);
 }
 
 }  // namespace
@@ -556,17 +575,18 @@ bool qkv_kblock_supported(int Kp) { return Kp % 128 == 0 && Kp * 64 <= Shape<1>:
 // dequantisation and Attn8.Prepare phases (40% of a workgroup's time) no
 // longer overlap another workgroup's K loop: slower on cfg4 (339 against
 // 315 us a launch).
-void launch_qkv_attn(const GemmArgs &g, const AttnArgs &a, const int32_t *order, int heads, hipStream_t s) {
+void launch_qkv_attn(const GemmArgs &g, const AttnArgs &a, const int32_t *order, const int32_t *groups, int ngroups,
+                     int heads, hipStream_t s) {
   if (a.B <= 0) return;
   const bool pair = heads == 2 && a.nh % 2 == 0 && !g.Ak;
   if (pair && smem_ready<2, false>()) {
-    launch_nh<2, false>(g, a, order, s);
+    launch_nh<2, false>(g, a, order, a.B, s);
   } else if (g.Ak) {
     (void)smem_ready<1, true>();
-    launch_nh<1, true>(g, a, order, s);
+    launch_nh<1, true>(g, a, groups, ngroups, s);
   } else {
     (void)smem_ready<1, false>();
-    launch_nh<1, false>(g, a, order, s);
+    launch_nh<1, false>(g, a, order, a.B, s);
   }
 }
 

@@ -103,3 +103,26 @@ def test_shared_keys_exact(shape, window):
             want = np.concatenate([gpu.encode_seqs([s]) for s in seqs])
             assert f32_bits_equal(got, want), (blocks, mismatch_report(got, want))
     gpu.close()
+
+
+@pytest.mark.parametrize("shape,lanes,plant", [("small", 8, False), ("bekko", 16, True), ("base", 8, False)])
+def test_shared_qkv_workgroups_exact(shape, lanes, plant):
+    """The fused QKV kernel's workgroups shared by sequences of at most 256
+    tokens (qkv_groups): random lengths, every padded block count beside every
+    other, empty sequences between and at the end, sequences over 256 tokens
+    among them, and QKV rows past the dequantisation bound, against the
+    oracle."""
+    cfg = SHAPES[shape](layers=2)
+    w = Weights.random(cfg, seed=107)
+    if plant:
+        w.wqkv_q[0, cfg.hidden + 5, :] = 127
+    gpu, ora = Model(w, lanes=lanes), orc.OracleModel(w, lanes=lanes)
+    rng = np.random.default_rng(107)
+    batches = [(129, 64, 1, 128, 0, 65, 192, 2, 256, 0), (193, 63, 130, 127, 33, 257, 31, 32, 512, 0, 0),
+               tuple(int(n) for n in rng.integers(0, 300, 40 if shape == "small" else 12)) + (0,)]
+    for lens in batches:
+        seqs = seqs_of(rng, cfg.vocab, *lens)
+        got, want = gpu.encode_tokens(seqs), ora.encode_tokens(seqs)[0]
+        assert f32_bits_equal(got, want), (lens, mismatch_report(got, want))
+        assert f32_bits_equal(gpu.encode_seqs(seqs), ora.encode_seqs(seqs)), lens
+    gpu.close()
