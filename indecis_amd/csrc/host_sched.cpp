@@ -114,25 +114,38 @@ int check_offs(const int32_t *offs, int B) {
   return IXH_OK;
 }
 
-void qkv_groups(const int32_t *offs, const std::vector<int32_t> &order, std::vector<int32_t> &groups) {
+void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<int32_t> &order,
+                std::vector<int32_t> &groups) {
+  constexpr int kSlots = 16, kSeqs = 8;
   groups.clear();
-  std::vector<int> open[9];  // groups with w free waves (w 1 .. 7)
+  std::vector<int> open[kSlots], count;  // groups with w free slots; their sequences
   for (int32_t b : order) {
     const int n = offs[b + 1] - offs[b];
-    const int nw = std::max(2, std::min(8, (n + 63) / 64 * 2));
-    int w = nw;
-    while (w < 8 && (nw == 8 || open[w].empty())) w++;  // the fullest group it fits into
+    const int nb = std::max(2, (n + 63) / 64 * 2);
+    int w = nb;
+    while (w < kSlots && open[w].empty()) w++;  // the fullest group it fits into
     int g;
-    if (w < 8) {
+    if (w < kSlots) {
       g = open[w].back();
       open[w].pop_back();
     } else {
-      g = (int)groups.size() / 8;
-      groups.insert(groups.end(), 8, -1);
+      g = (int)count.size();
+      groups.insert(groups.end(), kQkvGroup, 0);
+      for (int s = 0; s < kSlots; s++) groups[(size_t)kQkvGroup * g + 4 * s] = -1;
+      for (int s = 0; s < kSeqs; s++) groups[(size_t)kQkvGroup * g + 64 + s] = -1;
+      count.push_back(0);
     }
-    const int first = 8 - w;
-    for (int k = 0; k < nw; k++) groups[8 * g + first + k] = 16 * b + k;
-    if (w - nw > 0) open[w - nw].push_back(g);
+    int32_t *e = &groups[(size_t)kQkvGroup * g];
+    const int first = kSlots - w;
+    for (int k = 0; k < nb; k++) {
+      int32_t *s = e + 4 * (first + k);
+      s[0] = 16 * b + k;
+      s[1] = offs[b];
+      s[2] = n;
+      s[3] = padoff[b];
+    }
+    e[64 + count[g]++] = 16 * n + first;
+    if (w - nb > 0 && count[g] < kSeqs) open[w - nb].push_back(g);
   }
 }
 

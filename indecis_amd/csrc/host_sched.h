@@ -69,13 +69,16 @@ int plan_passes(const Tuning &t, int H, int I, const int32_t *offs, int B, std::
 // empty). cut has P+1 entries, cut[0] 0 and cut[P] B.
 void split_points(const int32_t *offs, int B, int P, std::vector<int> &cut);
 
-// The fused QKV kernel's workgroups, 8 waves each: groups[8 g + w] is wave w's
-// sequence and first 32-row block in it, 16 sequence + block, or -1. A
-// sequence over 256 tokens (at most 512) has a group of its own (wave w: its
-// blocks w and w + 8); shorter ones share groups, a sequence of n tokens
-// taking the consecutive waves of its blocks padded to 64 rows (an empty one
-// takes two). order: the sequences, longest first; groups come in that order.
-void qkv_groups(const int32_t *offs, const std::vector<int32_t> &order, std::vector<int32_t> &groups);
+// The fused QKV kernel's workgroups of 8 waves, kQkvGroup integers each: slot
+// s < 16 (wave w computes slots w and w + 8) is the four at 4 s: its sequence
+// and 32-row block in it, 16 sequence + block (-1: none), the sequence's first
+// row, its length and its first key slot; 64 + w: 16 times the length of the
+// group's w-th sequence plus its first slot (-1: none). A sequence (at most 512
+// tokens) takes the consecutive slots of its blocks padded to 64 rows, an
+// empty one two; slots are taken in order. order: the sequences, longest first.
+constexpr int kQkvGroup = 72;
+void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<int32_t> &order,
+                std::vector<int32_t> &groups);
 
 // What a pass writes (null: not wanted). states [N][H] final states
 // (EncodeTokens); pooled [B][H] (EncodeSeqs); zp [B][rp] pooled-row head

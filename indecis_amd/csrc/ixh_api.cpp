@@ -636,7 +636,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
 
   int rc;
   std::vector<int32_t> groups;
-  if (kblock) qkv_groups(offs, order, groups);
+  if (kblock) qkv_groups(offs, padoff.data(), order, groups);
   const size_t ntab = 2 * (size_t)(B + 1) + blocks.size() + B + groups.size();
   if ((rc = w->tabs.ensure(4 * ntab)) || (rc = w->pos.ensure(4 * (size_t)N)) ||
       (rc = w->x.ensure(4 * (size_t)N * H)) || (rc = w->xn.ensure(4 * (size_t)N * H)) ||
@@ -654,14 +654,15 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   // small host-built tables through pinned memory, one copy
   if ((rc = w->host.ensure(4 * ntab))) return rc;
   int32_t *hs = (int32_t *)w->host.p;
+  if (!groups.empty()) memcpy(hs, groups.data(), 4 * groups.size());  // first: read 16 bytes at a time
+  hs += groups.size();
   memcpy(hs, offs, 4 * (B + 1));
   memcpy(hs + B + 1, padoff.data(), 4 * (B + 1));
   if (!blocks.empty()) memcpy(hs + 2 * (B + 1), blocks.data(), 4 * blocks.size());
   if (B > 0) memcpy(hs + 2 * (B + 1) + blocks.size(), order.data(), 4 * (size_t)B);
-  if (!groups.empty()) memcpy(hs + 2 * (B + 1) + blocks.size() + B, groups.data(), 4 * groups.size());
-  HIPCK(hipMemcpyAsync(w->tabs.p, hs, 4 * ntab, hipMemcpyHostToDevice, st));
-  const int32_t *d_offs = w->tabs.as<int32_t>(), *d_padoff = d_offs + B + 1,
-                *d_blocks = d_offs + 2 * (B + 1), *d_order = d_blocks + blocks.size(), *d_groups = d_order + B;
+  HIPCK(hipMemcpyAsync(w->tabs.p, w->host.p, 4 * ntab, hipMemcpyHostToDevice, st));
+  const int32_t *d_groups = w->tabs.as<int32_t>(), *d_offs = d_groups + groups.size(), *d_padoff = d_offs + B + 1,
+                *d_blocks = d_offs + 2 * (B + 1), *d_order = d_blocks + blocks.size();
 
   Pending local;
   Pending &pend = defer ? *defer : local;
@@ -876,7 +877,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
       // scales are its only outputs
       RUN("gemm_qkv", 2 * dN * 3 * dH * dH,
           gemm_bytes(dH, 3 * dH, 0, false) + dN * (3 * dH + 8 * nh) + 4.0 * B * dH,
-          launch_qkv_attn(g, aa, d_order, d_groups, (int)groups.size() / 8, tune.qkv_heads, st));
+          launch_qkv_attn(g, aa, d_order, d_groups, (int)groups.size() / kQkvGroup, tune.qkv_heads, st));
     } else {
       RUN("gemm_qkv", 2 * dN * 3 * dH * dH,
           gemm_bytes(dH, 3 * dH, 2 * dH, false) + dN * (4 + dH + 4 * nh), launch_gemm(EPI_ROPE, g, st));

@@ -306,7 +306,7 @@ constexpr int kKeyPad = 64;       // key slots of a sequence are padded to this
 // batches whose sequences have at most kQkvSeqMax keys: g as for the
 // EPI_ROPE GEMM (A, sa, B, sb, zc, c128, Kp, rope tables, pos, qq, sq,
 // attn_scale; C unused), a as for launch_attn_prologue (qkv unused);
-// order[B]: the sequences, longest first; groups[8 ngroups]: the workgroups'
+// order[B]: the sequences, longest first; groups[kQkvGroup ngroups]: the workgroups'
 // waves as qkv_groups makes them (K-blocked input); heads: per workgroup, 1 or
 // 2 (2 only for an even head count where the device grants the LDS).
 constexpr int kQkvSeqMax = 512;

@@ -36,10 +36,12 @@
 // and each wave streams its own row blocks' fragments into registers, PF
 // K-blocks ahead: no ring, no barrier in the K loop, LDS read traffic of B
 // only. A workgroup's time is about 4.7 us + 0.03 us a row whatever its
-// sequence, so here the waves of one workgroup are shared out among several
-// sequences of at most 256 rows (qkv_groups, host_sched.h: a wave a row
-// block): 128 tokens a sequence 157 -> 118 us a launch of 32,768 rows, 64 tokens
-// (hidden 256) 74 -> 35 of 35,000.
+// sequence (hidden 768), so here the 16 row blocks of a workgroup are shared
+// out among sequences (qkv_groups, host_sched.h, which also lays down each
+// block's first row and length, so that no load waits for another): 128 tokens
+// a sequence 157 -> 101 us a launch of 32,768 rows, 200 tokens 141 -> 125, 64
+// tokens (hidden 256) 74 -> 35 of 35,000; 288 tokens, which fill no workgroup
+// with others of their length, 267 and 268, 512 tokens 187 and 187.
 #include <type_traits>
 
 #include "ixh_device.h"
@@ -82,33 +84,60 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   constexpr int NW = S::NW, RING = S::RING, STAGE = S::STAGE;
   extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
   __shared__ float sa_s[SEQ_MAX];
-  __shared__ float red_s[NH][8][D];
-  __shared__ __attribute__((aligned(16))) float stat_s[KB ? 8 : NH][D];
+  // V: maxima of a wave's (KB: a slot's) rows; K: means by sequence
+  __shared__ __attribute__((aligned(16))) float stat_s[KB ? 16 : 8 * NH][D];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int hf = wave >> 3, wv = wave & 7, tidh = tid & 511;  // half, wave and thread in the half
   const int fr = lane & 31, fh = lane >> 5;
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave), wv_u = wave_u & 7;
   const int hgroups = a.nh / NH;
   const int per_seq = 3 * hgroups;
   const int xcd = blockIdx.x % NXCD, k = blockIdx.x / NXCD;
   const int si = xcd + NXCD * (k / per_seq);
   if (si >= nwork) return;
-  // this wave's sequence and first row block in it (its second is 8 on): KB,
-  // from the table (-1: none); else the workgroup's sequence, block wv
-  const int ent = KB ? __builtin_amdgcn_readfirstlane(work[8 * si + wv]) : 16 * work[si] + wv;
-  const bool valid = !KB || ent >= 0;
-  const int b = valid ? ent >> 4 : 0, rb0 = valid ? ent & 15 : 0;
+  // this wave's two row blocks: KB, the table's slots wv and wv + 8 (-1: none);
+  // else blocks wv and wv + 8 of the workgroup's sequence
+  struct Block {
+    int slot;                  // its slot, or in a workgroup of one sequence its block
+    bool valid;
+    int b, rb, base, n, last;  // sequence, block in it, first row, rows; the row that stands for those past n
+    int npad, nb, nbc;         // rows and blocks stored (even), blocks computed (one past n is all zeros)
+    int slot0, sw;             // first key slot (K and V outputs); place in stat_s
+    __device__ bool on() const { return rb < nbc; }
+  } e[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    Block &x = e[i];
+    x.slot = wv + 8 * i;
+    if constexpr (KB) {
+      const int4 t = ((const int4 *)(work + kQkvGroup * si))[wv_u + 8 * i];
+      x.valid = t.x >= 0;
+      x.b = x.valid ? t.x >> 4 : 0;
+      x.rb = x.valid ? t.x & 15 : 0;
+      x.base = t.y;
+      x.n = t.z;
+      x.slot0 = t.w;
+    } else {
+      x.valid = true;
+      x.b = work[si];
+      x.rb = x.slot;
+      x.base = a.offs[x.b];
+      x.n = a.offs[x.b + 1] - x.base;
+      x.slot0 = a.padoff[x.b];
+    }
+    x.last = max(x.n - 1, 0);
+    x.npad = (x.n + kKeyPad - 1) / kKeyPad * kKeyPad;
+    x.nb = x.npad / 32;
+    x.nbc = (x.n + 31) / 32;
+    x.sw = KB ? x.slot - x.rb : hf;
+  }
   const int part = (k % per_seq) / hgroups, h0 = NH * ((k % per_seq) % hgroups), h = h0 + hf;
-  const int base = a.offs[b], n = valid ? a.offs[b + 1] - base : 0;
-  const int last = max(n - 1, 0);  // the row that stands for those past n
-  const int slot0 = a.padoff[b];  // the sequence's first key slot (K and V outputs)
-  const int npad = (n + kKeyPad - 1) / kKeyPad * kKeyPad;
-  const int nb = npad / 32;            // 32-row blocks stored (even, at most 16)
-  const int nbc = (n + 31) / 32;       // blocks computed: a block past n is all zeros
-  const int sw = KB ? wv - rb0 : hf;   // the sequence's place in stat_s (KB: its first wave)
-  // whether the workgroup's waves have second blocks: one sequence over 256
-  // rows (wave 0 always has a sequence)
-  const int b0 = KB ? work[8 * si] >> 4 : b;
-  const bool two_rounds = a.offs[b0 + 1] - a.offs[b0] > 256;
+  // the ring path's sequence
+  const int b = e[0].b, base = e[0].base, n = e[0].n, nb = e[0].nb, nbc = e[0].nbc;
+  // whether second blocks are in use (slots are taken in order)
+  const bool two_rounds = KB ? work[kQkvGroup * si + 4 * 8] >= 0 : n > 256;
+  // the sequence whose K mean this wave sums: its first slot, its rows
+  const int own = KB ? work[kQkvGroup * si + 64 + wv_u] : wv == 0 ? 16 * n : -1;
   const int col0 = part * a.H + h * D;   // this half's head: first output column
   const int colb = part * a.H + h0 * D;  // the workgroup's first weight row
   if (!KB && n == 0) {
@@ -121,7 +150,8 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   static_assert(SEQ_MAX <= 512, "one row scale a thread");
   // KB: lanes 0-31 the rows of the wave's first block, 32-63 of its second
   // (an empty sequence at the batch's end has no row of its own)
-  const float sa_v = KB ? g.sa[min(base + min(32 * (rb0 + 8 * fh) + fr, last), a.N - 1)]
+  const float sa_v = KB ? g.sa[min(fh ? e[1].base + min(32 * e[1].rb + fr, e[1].last)
+                                      : e[0].base + min(32 * e[0].rb + fr, e[0].last), a.N - 1)]
                         : tid < 32 * nb ? g.sa[base + min(tid, n - 1)] : 0.f;
   float zc[2], sb[2];
   int c128[2];
@@ -146,8 +176,6 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   // a K step then only adds kt * BK.
   constexpr int MAXCH = (2 * (SEQ_MAX / 32) + 4 * NH + NW - 1) / NW;
   static_assert(MAXCH <= 3 || RING == 2, "wait_vmcnt_upto covers 3 chunks a stage");
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const int wv_u = wave_u & 7;
   const int nch = wave_u < nchunk ? (nchunk - wave_u + NW - 1) / NW : 0;
   const int8_t *csrc[MAXCH];
   int cdst[MAXCH];
@@ -201,9 +229,9 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     const auto ars = buf_rsrc(g.Ak, (uint32_t)nkb * g.ak_rows * 32);
     uint32_t avo[2];
 #pragma unroll
-    for (int i = 0; i < 2; i++) avo[i] = (uint32_t)(base + min(32 * (rb0 + 8 * i) + fr, last)) * 32 + 16 * fh;
+    for (int i = 0; i < 2; i++) avo[i] = (uint32_t)(e[i].base + min(32 * e[i].rb + fr, e[i].last)) * 32 + 16 * fh;
     const uint32_t akstep = (uint32_t)g.ak_rows * 32;
-    const bool two = rb0 + 8 < nbc;  // this wave's second row block
+    const bool two = e[1].on();  // this wave's second row block
     // Both row blocks' fragments are loaded every K-block, past the last
     // K-block the last one again, whether or not the wave has a second
     // block (then row n-1: one 32-byte piece): with a load count that does
@@ -237,7 +265,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
         loadA(kb + PF, fa[u]);
       }
     };
-    if (rb0 < nbc) {
+    if (e[0].on() || two) {
       round(0, std::true_type{});
       for (int k0 = PF; k0 < nkb; k0 += PF) round(k0, std::false_type{});
     }
@@ -291,18 +319,18 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   auto tables = [&](int i) {
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-      const int p = min(32 * (rb0 + 8 * i) + 8 * u + (lane >> 3), last);
+      const int p = min(32 * e[i].rb + 8 * u + (lane >> 3), e[i].last);
       const size_t off = (size_t)p * 32 + 4 * (lane & 7);
       __builtin_amdgcn_global_load_lds((glb_ptr)(g.rope_cos + off), (lds_ptr)(smem + wave * 8192 + 1024 * u), 16, 0, 0);
       __builtin_amdgcn_global_load_lds((glb_ptr)(g.rope_sin + off), (lds_ptr)(smem + wave * 8192 + 4096 + 1024 * u), 16, 0, 0);
     }
   };
-  if (rope && rb0 < nbc) tables(0);
+  if (rope && e[0].on()) tables(0);
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     // a block past n (stored as padding keys) is not computed: its values
     // reach only rows past n, which every store below writes as zeros
-    if (rb0 + 8 * i >= nbc) continue;
+    if (!e[i].on()) continue;
     if (g.small) {
       // the weights' bound holds (checked on upload): f32(acc + 128
       // colsum) - zc is f32(acc) exactly
@@ -324,7 +352,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   if (rope) {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      if (rb0 + 8 * i >= nbc) continue;
+      if (!e[i].on()) continue;
       if (i == 1) {
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt 0: this wave's reads of the first tables returned
         tables(1);
@@ -344,44 +372,56 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
 
   if (part == 2) {
     // ---- V: max |V| per dimension, scale, quantCols, V^T ----
-    float vm[2] = {0.f, 0.f};
     // every row of a computed block: the rows past n in the last one are
     // row n-1 again (its A row and row scale), so they leave the maxima as
     // they are; a block past n that was not computed is left out
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      if (rb0 + 8 * i >= nbc) continue;
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        vm[0] = amax(vm[0], v[i][0][r]);
-        vm[1] = amax(vm[1], v[i][1][r]);
+      for (int j = 0; j < 2; j++) {
+        float vm = 0.f;
+        if (e[i].on()) {
+#pragma unroll
+          for (int r = 0; r < 16; r++) vm = amax(vm, v[i][j][r]);
+        }
+        vm = __builtin_fmaxf(vm, __shfl_xor(vm, 32));
+        if constexpr (KB) {
+          if (fh == 0) stat_s[wv + 8 * i][32 * j + fr] = vm;
+        } else if (fh == 0) {
+          float *const m = &stat_s[8 * hf + wv][32 * j + fr];
+          *m = i ? __builtin_fmaxf(*m, vm) : vm;
+        }
       }
-    }
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-      vm[j] = __builtin_fmaxf(vm[j], __shfl_xor(vm[j], 32));
-      if (fh == 0) red_s[hf][wv][32 * j + fr] = vm[j];
     }
     __syncthreads();
-    // over the sequence's waves (KB: from its first, sw; the others hold 0)
-    float vi[2];
+    // the maxima over each block's sequence (KB: its slots from sw on), every
+    // slot's read before the first is used
+    constexpr int NS = KB ? 16 : 8;
+    float vi[2][2];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
-      float vs = 0.f;
-      const int w0 = KB ? sw : 0, w1 = KB ? min(sw + nbc, 8) : 8;
-      for (int w = w0; w < w1; w++) vs = __builtin_fmaxf(vs, red_s[hf][w][32 * j + fr]);
-      vi[j] = 0.f;
-      if (vs > 0.f) {  // attention8.go:262-269
-        vs = vs / 127.0f;
-        vi[j] = 1.0f / vs;
+      float m[NS];
+#pragma unroll
+      for (int w = 0; w < NS; w++) m[w] = stat_s[(KB ? 0 : 8 * hf) + w][32 * j + fr];
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        const int w0 = KB ? e[i].sw : 0, w1 = KB ? e[i].sw + e[i].nbc : NS;
+        float vs = 0.f;
+#pragma unroll
+        for (int w = 0; w < NS; w++) vs = __builtin_fmaxf(vs, w >= w0 && w < w1 ? m[w] : 0.f);
+        vi[i][j] = 0.f;
+        if (vs > 0.f) {  // attention8.go:262-269
+          vs = vs / 127.0f;
+          vi[i][j] = 1.0f / vs;
+        }
+        if (e[i].valid && e[i].rb == 0 && fh == 0) a.vs[((size_t)e[i].b * a.nh + h) * D + 32 * j + fr] = vs;
       }
-      if (valid && rb0 == 0 && fh == 0) a.vs[((size_t)b * a.nh + h) * D + 32 * j + fr] = vs;
     }
     int8_t *vt_s = smem + wave * (D * VT_LD);  // [64 dims][32 keys] of this wave's block
-    int8_t *vt = a.vt + (size_t)h * D * a.Npad + slot0;
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      const int rb = rb0 + 8 * i;
+      const int rb = e[i].rb, nb = e[i].nb, nbc = e[i].nbc, n = e[i].n;
+      int8_t *vt = a.vt + (size_t)h * D * a.Npad + e[i].slot0;
       if (rb < nb) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
@@ -393,7 +433,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
             if (rb < nbc) {
               int qv[4];
 #pragma unroll
-              for (int u = 0; u < 4; u++) qv[u] = q8(v[i][j][4 * gq + u], vi[j]);
+              for (int u = 0; u < 4; u++) qv[u] = q8(v[i][j][4 * gq + u], vi[i][j]);
               const int lim = n - (32 * rb + 8 * gq + 4 * fh);  // keys of the four still in the sequence
               const unsigned keep = lim >= 4 ? 0xffffffffu : lim <= 0 ? 0u : (1u << (8 * lim)) - 1u;
               w = (int)(((unsigned)(qv[0] & 0xff) | ((unsigned)(qv[1] & 0xff) << 8) |
@@ -419,7 +459,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   // slab, in the MFMA layout
   float *slab = (float *)(smem + hf * SLAB_BYTES);  // [256 rows][KT_LD], one a half
 #define PUT(t)                                                    \
-  if (rb0 + 8 * (t) < nb) {                                       \
+  if (e[t].rb < e[t].nb) {                                        \
     _Pragma("unroll") for (int r = 0; r < 16; r++) {              \
       const int lr = 32 * wv + acc_row(r, lane);                  \
       slab[lr * KT_LD + fr] = v[t][0][r];                         \
@@ -427,21 +467,23 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     }                                                             \
   }
   if (part == 1) {
-    // K mean over the sequence: 64 float32 chains in key order, one lane
-    // a dimension
+    // K mean over each sequence: 64 float32 chains in key order, one lane
+    // a dimension; KB: wave w runs those of the w-th sequence, from slot ks0
+    const int ks0 = own < 0 ? -1 : own & 15, kn = own < 0 ? 0 : own >> 4;
     float ksum = 0.f;
 #pragma unroll
     for (int t = 0; t < 2; t++) {
       if (t == 0 || two_rounds) {  // block-uniform
         PUT(t)
         __syncthreads();
-        if (rb0 == 0) {  // the sequence's first wave (none: no rows)
+        // its rows in the slab: slots 8 t .. 8 t + 7
+        const int s0 = max(ks0, 8 * t), cnt = min(kn - 32 * (s0 - ks0), 32 * (8 * t + 8 - s0));
+        if (ks0 >= 0 && cnt > 0) {
           // the sums stay in key order; KN slab reads are issued together
           // before their KN adds, so the chain waits on LDS once a batch
           // (KN = 8 where NH = 2 leaves fewer registers)
           constexpr int KN = NH == 1 ? 16 : 8;
-          const int cnt = min(256, n - 256 * t);
-          const float *col = slab + 32 * wv * KT_LD + lane;
+          const float *col = slab + 32 * (s0 - 8 * t) * KT_LD + lane;
           int lr = 0;
           for (; lr + KN <= cnt; lr += KN) {
             float bt[KN];
@@ -456,7 +498,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
         __syncthreads();
       }
     }
-    if (rb0 == 0) stat_s[sw][lane] = ksum * (1.0f / (float)n);  // Scale(mean, 1/n)
+    if (ks0 >= 0) stat_s[KB ? ks0 : hf][lane] = ksum * (1.0f / (float)kn);  // Scale(mean, 1/n)
     __syncthreads();
   }
 
@@ -465,14 +507,13 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   // 32, half (lane / 16) % 2), K centred first (quantRowAVX2 without the
   // flip, attention8.go:240-251), Q as Attn8.Prepare quantises queries
   // (attention8.go:211-220).
-  int8_t *kp = a.kp + ((size_t)h * a.Npad + slot0) * D;
-  float *ks = a.ks + (size_t)h * a.Npad + slot0;
   const int hh = (lane >> 4) & 1;
   const int lr = 32 * wv + 16 * (lane >> 5) + (lane & 15);
-  auto quant_round = [&](int t) {
-    const int row = 32 * (rb0 + 8 * t) + 16 * (lane >> 5) + (lane & 15);
+  auto quant_round = [&](auto tv) {
+    constexpr int t = decltype(tv)::value;
+    const int n = e[t].n, base = e[t].base, row = 32 * e[t].rb + 16 * (lane >> 5) + (lane & 15);
     const float4 *src = (const float4 *)(slab + lr * KT_LD + 32 * hh);
-    const float4 *mu = (const float4 *)(stat_s[sw] + 32 * hh);
+    const float4 *mu = (const float4 *)(stat_s[e[t].sw] + 32 * hh);
     // the slab is read twice (max, then quantisation): fewer live registers
     auto value = [&](int c) {
       float4 x = src[c];
@@ -512,31 +553,32 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
         *(v4i *)(dst + 16) = hi;
         if (hh == 0) g.sq[(size_t)(base + row) * a.nh + h] = sc * g.attn_scale;
       }
-    } else if (row < npad) {
-      int8_t *dst = kp + (size_t)row * D + 32 * hh;
+    } else if (row < e[t].npad) {
+      const size_t at = (size_t)h * a.Npad + e[t].slot0 + row;
+      int8_t *dst = a.kp + at * D + 32 * hh;
       *(v4i *)dst = lo;
       *(v4i *)(dst + 16) = hi;
-      if (hh == 0) ks[row] = valid ? sc : 0.f;
+      if (hh == 0) a.ks[at] = valid ? sc : 0.f;
     }
   };
   if (part == 1) {
     // the slab holds the chains' last round
     if (two_rounds) {
-      quant_round(1);
+      quant_round(std::integral_constant<int, 1>{});
       __syncthreads();
       PUT(0)
       __syncthreads();
     }
-    quant_round(0);
+    quant_round(std::integral_constant<int, 0>{});
   } else {
     PUT(0)
     __syncthreads();
-    quant_round(0);
+    quant_round(std::integral_constant<int, 0>{});
     if (two_rounds) {
       __syncthreads();
       PUT(1)
       __syncthreads();
-      quant_round(1);
+      quant_round(std::integral_constant<int, 1>{});
     }
   }
 #undef PUT
