@@ -114,8 +114,8 @@ int check_offs(const int32_t *offs, int B) {
   return IXH_OK;
 }
 
-void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<int32_t> &order,
-                std::vector<int32_t> &groups) {
+void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<int32_t> &order, int slots,
+                bool share, std::vector<int32_t> &groups) {
   constexpr int kSlots = 16, kSeqs = 8;
   groups.clear();
   std::vector<int> open[kSlots], count;  // groups with w free slots; their sequences
@@ -123,12 +123,13 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
     const int n = offs[b + 1] - offs[b];
     const int nb = std::max(2, (n + 63) / 64 * 2);
     int w = nb;
-    while (w < kSlots && open[w].empty()) w++;  // the fullest group it fits into
+    while (w < slots && open[w].empty()) w++;  // the fullest group it fits into
     int g;
-    if (w < kSlots) {
+    if (w < slots) {
       g = open[w].back();
       open[w].pop_back();
     } else {
+      w = slots;
       g = (int)count.size();
       groups.insert(groups.end(), kQkvGroup, 0);
       for (int s = 0; s < kSlots; s++) groups[(size_t)kQkvGroup * g + 4 * s] = -1;
@@ -136,7 +137,7 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
       count.push_back(0);
     }
     int32_t *e = &groups[(size_t)kQkvGroup * g];
-    const int first = kSlots - w;
+    const int first = slots - w;
     for (int k = 0; k < nb; k++) {
       int32_t *s = e + 4 * (first + k);
       s[0] = 16 * b + k;
@@ -145,7 +146,7 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
       s[3] = padoff[b];
     }
     e[64 + count[g]++] = 16 * n + first;
-    if (w - nb > 0 && count[g] < kSeqs) open[w - nb].push_back(g);
+    if (share && w - nb > 0 && count[g] < kSeqs) open[w - nb].push_back(g);
   }
 }
 

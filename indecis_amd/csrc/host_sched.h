@@ -75,10 +75,12 @@ void split_points(const int32_t *offs, int B, int P, std::vector<int> &cut);
 // row, its length and its first key slot; 64 + w: 16 times the length of the
 // group's w-th sequence plus its first slot (-1: none). A sequence (at most 512
 // tokens) takes the consecutive slots of its blocks padded to 64 rows, an
-// empty one two; slots are taken in order. order: the sequences, longest first.
+// empty one two; slots are taken in order, of `slots` (16; 8, where no sequence
+// is over 256 tokens). share: several sequences a group. order: the
+// sequences, longest first.
 constexpr int kQkvGroup = 72;
-void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<int32_t> &order,
-                std::vector<int32_t> &groups);
+void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<int32_t> &order, int slots,
+                bool share, std::vector<int32_t> &groups);
 
 // What a pass writes (null: not wanted). states [N][H] final states
 // (EncodeTokens); pooled [B][H] (EncodeSeqs); zp [B][rp] pooled-row head

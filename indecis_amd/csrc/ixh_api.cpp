@@ -636,7 +636,22 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
 
   int rc;
   std::vector<int32_t> groups;
-  if (kblock) qkv_groups(offs, padoff.data(), order, groups);
+  // its workgroups: sequences share them once one a sequence, head and part
+  // would not all be resident (two a CU); of 8 row blocks where no sequence has
+  // more, up to four rounds of that, else of 16. us a launch with 8 and 16
+  // blocks, sequences of 200 tokens, hidden 768 (384): 4 sequences 13.4 and
+  // 20.0, 16 19.0 and 20.8 (9.9 and 14.8), 32 29.7 and 29.8, 64 (26 and 29),
+  // 164 125 and 119.
+  const int cus = device_cus();
+  bool two_blocks = T > 256;
+  if (kblock) {
+    const bool share = 3 * nh * B > 2 * cus;
+    qkv_groups(offs, padoff.data(), order, two_blocks ? 16 : 8, share, groups);
+    if (!two_blocks && 3 * nh * (int64_t)(groups.size() / kQkvGroup) > 8 * cus) {
+      two_blocks = true;
+      qkv_groups(offs, padoff.data(), order, 16, share, groups);
+    }
+  }
   const size_t ntab = 2 * (size_t)(B + 1) + blocks.size() + B + groups.size();
   if ((rc = w->tabs.ensure(4 * ntab)) || (rc = w->pos.ensure(4 * (size_t)N)) ||
       (rc = w->x.ensure(4 * (size_t)N * H)) || (rc = w->xn.ensure(4 * (size_t)N * H)) ||
@@ -877,7 +892,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
       // scales are its only outputs
       RUN("gemm_qkv", 2 * dN * 3 * dH * dH,
           gemm_bytes(dH, 3 * dH, 0, false) + dN * (3 * dH + 8 * nh) + 4.0 * B * dH,
-          launch_qkv_attn(g, aa, d_order, d_groups, (int)groups.size() / kQkvGroup, tune.qkv_heads, st));
+          launch_qkv_attn(g, aa, d_order, d_groups, (int)groups.size() / kQkvGroup, two_blocks, tune.qkv_heads, st));
     } else {
       RUN("gemm_qkv", 2 * dN * 3 * dH * dH,
           gemm_bytes(dH, 3 * dH, 2 * dH, false) + dN * (4 + dH + 4 * nh), launch_gemm(EPI_ROPE, g, st));

@@ -307,11 +307,11 @@ constexpr int kKeyPad = 64;       // key slots of a sequence are padded to this
 // EPI_ROPE GEMM (A, sa, B, sb, zc, c128, Kp, rope tables, pos, qq, sq,
 // attn_scale; C unused), a as for launch_attn_prologue (qkv unused);
 // order[B]: the sequences, longest first; groups[kQkvGroup ngroups]: the workgroups'
-// waves as qkv_groups makes them (K-blocked input); heads: per workgroup, 1 or
+// waves as qkv_groups makes them (K-blocked input), two_blocks: of 16 slots; heads: per workgroup, 1 or
 // 2 (2 only for an even head count where the device grants the LDS).
 constexpr int kQkvSeqMax = 512;
 void launch_qkv_attn(const GemmArgs &g, const AttnArgs &a, const int32_t *order, const int32_t *groups, int ngroups,
-                     int heads, hipStream_t s);
+                     bool two_blocks, int heads, hipStream_t s);
 // QKV projection, Attn8.Prepare and attention in one kernel (short_attn.hip),
 // for batches of short sequences (see there) and Kp one of 768, 384, 256: g as for launch_qkv_attn with the K-blocked input, a as for
 // launch_attn_main (of the prologue's outputs nothing is written); false

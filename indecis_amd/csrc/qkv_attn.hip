@@ -77,9 +77,11 @@ __device__ __forceinline__ void wait_vmcnt_upto(int n) {
   else wait_vmcnt<3>();
 }
 
-template <int NH, bool KB>
+// BLK: row blocks a wave (1: K-blocked input, no group uses second blocks)
+template <int NH, bool KB, int BLK>
 __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnArgs a, const int32_t *work, int nwork) {
   static_assert(!KB || NH == 1, "K-blocked input: one head a workgroup");
+  static_assert(KB || BLK == 2, "the ring: a sequence of up to 512 rows");
   using S = Shape<NH>;
   constexpr int NW = S::NW, RING = S::RING, STAGE = S::STAGE;
   extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
@@ -104,9 +106,9 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     int npad, nb, nbc;         // rows and blocks stored (even), blocks computed (one past n is all zeros)
     int slot0, sw;             // first key slot (K and V outputs); place in stat_s
     __device__ bool on() const { return rb < nbc; }
-  } e[2];
+  } e[BLK];
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
+  for (int i = 0; i < BLK; i++) {
     Block &x = e[i];
     x.slot = wv + 8 * i;
     if constexpr (KB) {
@@ -135,7 +137,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   // the ring path's sequence
   const int b = e[0].b, base = e[0].base, n = e[0].n, nb = e[0].nb, nbc = e[0].nbc;
   // whether second blocks are in use (slots are taken in order)
-  const bool two_rounds = KB ? work[kQkvGroup * si + 4 * 8] >= 0 : n > 256;
+  const bool two_rounds = BLK == 2 && (KB ? work[kQkvGroup * si + 4 * 8] >= 0 : n > 256);
   // the sequence whose K mean this wave sums: its first slot, its rows
   const int own = KB ? work[kQkvGroup * si + 64 + wv_u] : wv == 0 ? 16 * n : -1;
   const int col0 = part * a.H + h * D;   // this half's head: first output column
@@ -150,7 +152,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   static_assert(SEQ_MAX <= 512, "one row scale a thread");
   // KB: lanes 0-31 the rows of the wave's first block, 32-63 of its second
   // (an empty sequence at the batch's end has no row of its own)
-  const float sa_v = KB ? g.sa[min(fh ? e[1].base + min(32 * e[1].rb + fr, e[1].last)
+  const float sa_v = KB ? g.sa[min(BLK == 2 && fh ? e[BLK - 1].base + min(32 * e[BLK - 1].rb + fr, e[BLK - 1].last)
                                       : e[0].base + min(32 * e[0].rb + fr, e[0].last), a.N - 1)]
                         : tid < 32 * nb ? g.sa[base + min(tid, n - 1)] : 0.f;
   float zc[2], sb[2];
@@ -201,10 +203,10 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   };
 
   // (the K-blocked loop starts its sums from the MFMAs' zero operand)
-  v16i acc[2][2];
+  v16i acc[BLK][2];
   if constexpr (!KB) {
 #pragma unroll
-  for (int i = 0; i < 2; i++)
+  for (int i = 0; i < BLK; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++)
 #pragma unroll
@@ -225,32 +227,32 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     // stored), a K-block further on every ak_rows rows: the lane's byte
     // offsets in the VGPRs, the K-block's in an SGPR (no address
     // arithmetic a load)
-    constexpr int PF = 4;  // K-blocks in flight (nkb is a multiple of 4)
+    constexpr int PF = BLK == 2 ? 4 : 8;  // K-blocks in flight (nkb is a multiple of 4)
     const auto ars = buf_rsrc(g.Ak, (uint32_t)nkb * g.ak_rows * 32);
-    uint32_t avo[2];
+    uint32_t avo[BLK];
 #pragma unroll
-    for (int i = 0; i < 2; i++) avo[i] = (uint32_t)(e[i].base + min(32 * e[i].rb + fr, e[i].last)) * 32 + 16 * fh;
+    for (int i = 0; i < BLK; i++) avo[i] = (uint32_t)(e[i].base + min(32 * e[i].rb + fr, e[i].last)) * 32 + 16 * fh;
     const uint32_t akstep = (uint32_t)g.ak_rows * 32;
-    const bool two = e[1].on();  // this wave's second row block
+    const bool two = BLK == 2 && e[BLK - 1].on();  // this wave's second row block
     // Both row blocks' fragments are loaded every K-block, past the last
     // K-block the last one again, whether or not the wave has a second
     // block (then row n-1: one 32-byte piece): with a load count that does
     // not depend on the wave or the step, the compiler waits for exactly
     // the fragment it needs, not for every load in flight.
-    v4i fa[PF][2];
+    v4i fa[PF][BLK];
     auto loadA = [&](int kb, v4i *dst) {
       const uint32_t so = __builtin_amdgcn_readfirstlane((uint32_t)min(kb, nkb - 1) * akstep);
       dst[0] = __builtin_amdgcn_raw_buffer_load_b128(ars, avo[0], so, 0);
-      dst[1] = __builtin_amdgcn_raw_buffer_load_b128(ars, avo[1], so, 0);
+      if constexpr (BLK == 2) dst[BLK - 1] = __builtin_amdgcn_raw_buffer_load_b128(ars, avo[BLK - 1], so, 0);
     };
 #pragma unroll
     for (int u = 0; u < PF; u++) loadA(u, fa[u]);
-    wait_vmcnt<2 * PF>();  // this wave's weight chunks (older than its 2 PF A loads)
+    wait_vmcnt<BLK * PF>();  // this wave's weight chunks (older than its A loads)
     __builtin_amdgcn_s_barrier();  // every wave's weight chunks are in LDS
-    // PF K-blocks from k0; the first round's first K-block starts the sums
-    auto round = [&](int k0, auto first) {
+    // NU K-blocks from k0; the first round's first K-block starts the sums
+    auto round = [&](int k0, auto first, auto nu) {
 #pragma unroll
-      for (int u = 0; u < PF; u++) {
+      for (int u = 0; u < decltype(nu)::value; u++) {
         const int kb = k0 + u;
         const bool z = decltype(first)::value && u == 0;
         v4i fb[2];
@@ -260,14 +262,18 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
         for (int j = 0; j < 2; j++) acc[0][j] = mfma32(fa[u][0], fb[j], z ? v16i{} : acc[0][j]);
         if (two) {
 #pragma unroll
-          for (int j = 0; j < 2; j++) acc[1][j] = mfma32(fa[u][1], fb[j], z ? v16i{} : acc[1][j]);
+          for (int j = 0; j < 2; j++)
+            acc[BLK - 1][j] = mfma32(fa[u][BLK - 1], fb[j], z ? v16i{} : acc[BLK - 1][j]);
         }
         loadA(kb + PF, fa[u]);
       }
     };
     if (e[0].on() || two) {
-      round(0, std::true_type{});
-      for (int k0 = PF; k0 < nkb; k0 += PF) round(k0, std::false_type{});
+      constexpr std::integral_constant<int, PF> whole;
+      round(0, std::true_type{}, whole);
+      int k0 = PF;
+      for (; k0 + PF <= nkb; k0 += PF) round(k0, std::false_type{}, whole);
+      if (BLK == 1 && k0 < nkb) round(k0, std::false_type{}, std::integral_constant<int, 4>{});
     }
   } else {
   const int nk = g.Kp / BK;
@@ -291,7 +297,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
         fb[j] = *(const v4i *)(st + A_BYTES + row * BK + 16 * ((2 * s + fh) ^ swz(row)));
       }
 #pragma unroll
-      for (int i = 0; i < 2; i++) {
+      for (int i = 0; i < BLK; i++) {
         if (wv_u + 8 * i < nbc) {
           const int row = 32 * (wv_u + 8 * i) + fr;
           const v4i fa = *(const v4i *)(st + row * BK + 16 * ((2 * s + fh) ^ swz(row)));
@@ -302,7 +308,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     }
   }
   }  // !KB
-  if constexpr (KB) sa_s[32 * (wv + 8 * fh) + fr] = sa_v;
+  if constexpr (KB) sa_s[32 * (wv + 8 * fh) + fr] = sa_v;  // (BLK 1: the upper half's is not read)
   else if (tid < 32 * nb) sa_s[tid] = sa_v;
   __syncthreads();  // the ring is no longer read; the row scales are in LDS
 
@@ -313,7 +319,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   // into this wave's 8 KB of the free ring by 8 direct-to-LDS loads: the
   // first block's issued before the dequantisation of both blocks, the
   // second's once the first block's are read
-  float v[2][2][16];
+  float v[BLK][2][16];
   const bool rope = part < 2;
   const float *tab = (const float *)(smem + wave * 8192);
   auto tables = [&](int i) {
@@ -327,7 +333,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   };
   if (rope && e[0].on()) tables(0);
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
+  for (int i = 0; i < BLK; i++) {
     // a block past n (stored as padding keys) is not computed: its values
     // reach only rows past n, which every store below writes as zeros
     if (!e[i].on()) continue;
@@ -351,7 +357,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
   }
   if (rope) {
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
+    for (int i = 0; i < BLK; i++) {
       if (!e[i].on()) continue;
       if (i == 1) {
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt 0: this wave's reads of the first tables returned
@@ -376,7 +382,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     // row n-1 again (its A row and row scale), so they leave the maxima as
     // they are; a block past n that was not computed is left out
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
+    for (int i = 0; i < BLK; i++) {
 #pragma unroll
       for (int j = 0; j < 2; j++) {
         float vm = 0.f;
@@ -396,15 +402,15 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     __syncthreads();
     // the maxima over each block's sequence (KB: its slots from sw on), every
     // slot's read before the first is used
-    constexpr int NS = KB ? 16 : 8;
-    float vi[2][2];
+    constexpr int NS = KB ? 8 * BLK : 8;
+    float vi[BLK][2];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
       float m[NS];
 #pragma unroll
       for (int w = 0; w < NS; w++) m[w] = stat_s[(KB ? 0 : 8 * hf) + w][32 * j + fr];
 #pragma unroll
-      for (int i = 0; i < 2; i++) {
+      for (int i = 0; i < BLK; i++) {
         const int w0 = KB ? e[i].sw : 0, w1 = KB ? e[i].sw + e[i].nbc : NS;
         float vs = 0.f;
 #pragma unroll
@@ -419,7 +425,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     }
     int8_t *vt_s = smem + wave * (D * VT_LD);  // [64 dims][32 keys] of this wave's block
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
+    for (int i = 0; i < BLK; i++) {
       const int rb = e[i].rb, nb = e[i].nb, nbc = e[i].nbc, n = e[i].n;
       int8_t *vt = a.vt + (size_t)h * D * a.Npad + e[i].slot0;
       if (rb < nb) {
@@ -472,7 +478,7 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     const int ks0 = own < 0 ? -1 : own & 15, kn = own < 0 ? 0 : own >> 4;
     float ksum = 0.f;
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
+    for (int t = 0; t < BLK; t++) {
       if (t == 0 || two_rounds) {  // block-uniform
         PUT(t)
         __syncthreads();
@@ -561,24 +567,26 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
       if (hh == 0) a.ks[at] = valid ? sc : 0.f;
     }
   };
+  constexpr std::integral_constant<int, 0> first;
+  constexpr std::integral_constant<int, BLK - 1> second;
   if (part == 1) {
     // the slab holds the chains' last round
     if (two_rounds) {
-      quant_round(std::integral_constant<int, 1>{});
+      quant_round(second);
       __syncthreads();
       PUT(0)
       __syncthreads();
     }
-    quant_round(std::integral_constant<int, 0>{});
+    quant_round(first);
   } else {
     PUT(0)
     __syncthreads();
-    quant_round(std::integral_constant<int, 0>{});
+    quant_round(first);
     if (two_rounds) {
       __syncthreads();
-      PUT(1)
+      PUT(BLK - 1)
       __syncthreads();
-      quant_round(std::integral_constant<int, 1>{});
+      quant_round(second);
     }
   }
 #undef PUT
@@ -590,21 +598,21 @@ namespace {
 
 // hipFuncSetAttribute once per variant: 1 set, -1 refused (that variant is
 // then not used), 0 not tried yet.
-template <int NH, bool KB>
+template <int NH, bool KB, int BLK>
 bool smem_ready() {
   static int state = 0;
   if (state == 0)
-    state = hipFuncSetAttribute((const void *)qkv_attn_kernel<NH, KB>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    state = hipFuncSetAttribute((const void *)qkv_attn_kernel<NH, KB, BLK>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 Shape<NH>::SMEM) == hipSuccess
                 ? 1
                 : -1;
   return state > 0;
 }
 
-template <int NH, bool KB>
+template <int NH, bool KB, int BLK>
 void launch_nh(const GemmArgs &g, const AttnArgs &a, const int32_t *work, int nwork, hipStream_t s) {
   const int grid = NXCD * 3 * (a.nh / NH) * ((nwork + NXCD - 1) / NXCD);
-  qkv_attn_kernel<NH, KB><<<grid, 512 * NH, Shape<NH>::SMEM, s>>>(g, a, work, nwork);
+  qkv_attn_kernel<NH, KB, BLK><<<grid, 512 * NH, Shape<NH>::SMEM, s>>>(g, a, work, nwork);
 }
 
 }  // namespace
@@ -618,17 +626,22 @@ bool qkv_kblock_supported(int Kp) { return Kp % 128 == 0 && Kp * 64 <= Shape<1>:
 // longer overlap another workgroup's K loop: slower on cfg4 (339 against
 // 315 us a launch).
 void launch_qkv_attn(const GemmArgs &g, const AttnArgs &a, const int32_t *order, const int32_t *groups, int ngroups,
-                     int heads, hipStream_t s) {
+                     bool two_blocks, int heads, hipStream_t s) {
   if (a.B <= 0) return;
   const bool pair = heads == 2 && a.nh % 2 == 0 && !g.Ak;
-  if (pair && smem_ready<2, false>()) {
-    launch_nh<2, false>(g, a, order, a.B, s);
+  if (pair && smem_ready<2, false, 2>()) {
+    launch_nh<2, false, 2>(g, a, order, a.B, s);
   } else if (g.Ak) {
-    (void)smem_ready<1, true>();
-    launch_nh<1, true>(g, a, groups, ngroups, s);
+    if (two_blocks) {
+      (void)smem_ready<1, true, 2>();
+      launch_nh<1, true, 2>(g, a, groups, ngroups, s);
+    } else {
+      (void)smem_ready<1, true, 1>();
+      launch_nh<1, true, 1>(g, a, groups, ngroups, s);
+    }
   } else {
-    (void)smem_ready<1, false>();
-    launch_nh<1, false>(g, a, order, a.B, s);
+    (void)smem_ready<1, false, 2>();
+    launch_nh<1, false, 2>(g, a, order, a.B, s);
   }
 }
 

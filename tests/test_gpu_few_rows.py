@@ -118,11 +118,19 @@ def test_shared_qkv_workgroups_exact(shape, lanes, plant):
         w.wqkv_q[0, cfg.hidden + 5, :] = 127
     gpu, ora = Model(w, lanes=lanes), orc.OracleModel(w, lanes=lanes)
     rng = np.random.default_rng(107)
+    # (shared from 512 workgroups on: 3 * heads a sequence; groups of 16 blocks
+    # with a sequence over 256 tokens or past 2,048 workgroups)
     batches = [(129, 64, 1, 128, 0, 65, 192, 2, 256, 0), (193, 63, 130, 127, 33, 257, 31, 32, 512, 0, 0),
-               tuple(int(n) for n in rng.integers(0, 300, 40 if shape == "small" else 12)) + (0,)]
+               tuple(int(n) for n in rng.integers(0, 300, 60 if shape == "small" else 30)) + (0,),
+               tuple(int(n) for n in rng.integers(0, 257, 60 if shape == "small" else 20)) + (0, 256)]
     for lens in batches:
         seqs = seqs_of(rng, cfg.vocab, *lens)
         got, want = gpu.encode_tokens(seqs), ora.encode_tokens(seqs)[0]
         assert f32_bits_equal(got, want), (lens, mismatch_report(got, want))
         assert f32_bits_equal(gpu.encode_seqs(seqs), ora.encode_seqs(seqs)), lens
+    if shape == "small":
+        gpu.set_option("parts", 1)
+        seqs = seqs_of(rng, cfg.vocab, *(int(n) for n in rng.integers(129, 257, 200)))
+        got, want = gpu.encode_tokens(seqs), ora.encode_tokens(seqs)[0]
+        assert f32_bits_equal(got, want), mismatch_report(got, want)
     gpu.close()
