@@ -933,10 +933,17 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
       lr.qk_rows = N;
       RUN("gemm_wo", 2 * dN * dH * dH, res_bytes(dH, false),
           launch_res_split(product(L.o, w->ctx.as<float>(), H, cmax, nh, w->x.as<float>(), H, H), st));
-      RUN("ln_quant", 0, ln_bytes, launch_rownorm(lr, st));
       float *const gm = w->gmax.as<float>();
-      RUN("gemm_wi", 2 * dN * 2 * dI * dH, gemm_bytes(dH, 2 * dI, dI, false),
-          launch_wi_split(product(L.i, nullptr, H, gm, I / 32, w->g.as<float>(), I, 2 * I), st));
+      SplitArgs wi = product(L.i, w->x.as<float>(), H, gm, I / 32, w->g.as<float>(), I, 2 * I);
+      if (ln_wi_split_supported(I, N, cus)) {
+        wi.gamma = lr.gamma;
+        wi.eps = lr.eps;
+        wi.lanes = lr.lanes;
+        RUN("ln_wi", 2 * dN * 2 * dI * dH, dN * (4 * dH + 4 * dI) + 2 * dI * dH, launch_ln_wi_split(wi, st));
+      } else {
+        RUN("ln_quant", 0, ln_bytes, launch_rownorm(lr, st));
+        RUN("gemm_wi", 2 * dN * 2 * dI * dH, gemm_bytes(dH, 2 * dI, dI, false), launch_wi_split(wi, st));
+      }
       RUN("gemm_womlp", 2 * dN * dH * dI, res_bytes(dI, false),
           launch_res_split(product(L.omlp, w->g.as<float>(), I, gm, I / 32, w->x.as<float>(), H, H), st));
       if (l + 1 < c.layers) {

@@ -312,4 +312,70 @@ __device__ __forceinline__ float4 deq4(int4 t, bool small, const int32_t *c128, 
                      deq(t.w + c.w, z.w, sb.w, sa));
 }
 
+// LayerNormRow's chains (vec_simd.go:285-327) over rows of H floats in LDS, LD
+// apart: chain ch, a thread, is lane partial ch % V of row ch / V (V 0: one
+// float64 chain a row). The threads past the last chain repeat it. REREAD: the
+// second pass reads its values again instead of keeping the first's (H / V
+// registers).
+template <int V>
+__device__ constexpr int ln_chain_threads(int rows) {
+  return ((V > 0 ? V : 1) * rows + 63) / 64 * 64;
+}
+template <int H, int V, bool REREAD>
+__device__ __forceinline__ void ln_chains(const float *xs, int LD, int t, int lane, int rows, double eps,
+                                          float *mean_s, float *rstd_s) {
+  constexpr int W = V > 0 ? V : 1;
+  const int ch = min(t, W * rows - 1), cr = ch / W;
+  const float *xr = xs + cr * LD + ch % W;
+  float mean = 0.f;
+#pragma unroll
+  for (int pass = 0; pass < 2; pass++) {
+    double sum = 0.0;
+    if constexpr (REREAD) asm volatile("" ::: "memory");
+    if constexpr (V > 0) {
+      constexpr int NE = H / W, NB = NE % 16 == 0 ? 16 : 8;  // values a lane, a batch of them
+      static_assert(NE % NB == 0, "whole batches");
+      float p = 0.f, b[NB], n[NB];
+#pragma unroll
+      for (int e = 0; e < NB; e++) b[e] = xr[V * e];
+#pragma unroll
+      for (int e0 = 0; e0 < NE; e0 += NB) {
+        if (e0 + NB < NE) {
+#pragma unroll
+          for (int e = 0; e < NB; e++) n[e] = xr[V * (e0 + NB + e)];
+        }
+#pragma unroll
+        for (int e = 0; e < NB; e++) {
+          if (pass == 0) {
+            p = p + b[e];
+          } else {
+            const float d = b[e] - mean;
+            p = __builtin_fmaf(d, d, p);
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < NB; e++) b[e] = n[e];
+      }
+      const int base = lane & ~(W - 1);
+#pragma unroll
+      for (int q = 0; q < V; q++) sum += (double)__shfl(p, base + q);
+    } else {
+      for (int e = 0; e < H; e++) {
+        if (pass == 0) {
+          sum += (double)xr[e];
+        } else {
+          const double d = (double)(xr[e] - mean);
+          sum += d * d;
+        }
+      }
+    }
+    if (pass == 0) {
+      mean = (float)(sum / (double)H);
+    } else if (t < W * rows && t % W == 0) {
+      mean_s[cr] = mean;
+      rstd_s[cr] = (float)(1.0 / __builtin_sqrt(sum / (double)H + eps));
+    }
+  }
+}
+
 }  // namespace ixh

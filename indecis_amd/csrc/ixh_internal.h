@@ -189,10 +189,17 @@ struct SplitArgs {
   float *rmax;           // [M][P] max |A| (res, in) or |g| (wi, out: P = n/64) of the row's parts
   int P;
   int M;
+  const float *gamma;    // ln_wi: A is x, its LayerNorm's weights,
+  double eps;
+  int lanes;             // epsilon and lane width
 };
 // (H, I) one of (768, 1152), (384, 1152), (256, 512), unpadded
 bool split_rows_supported(int H, int I, int KpH, int KpI);
 void launch_wi_split(const SplitArgs &a, hipStream_t s);
+// The LayerNorm and quantisation of x before it in the same kernel: while its
+// workgroups are at most the CUs.
+bool ln_wi_split_supported(int I, int M, int cus);
+void launch_ln_wi_split(const SplitArgs &a, hipStream_t s);
 void launch_res_split(const SplitArgs &a, hipStream_t s);
 // ---- host helpers (ixh_api.cpp) ---------------------------------------------
 // Sets the calling thread's ixh_last_error message; returns code.

@@ -858,61 +858,7 @@ __global__ __launch_bounds__(256) void ln_rows_kernel(RowArgs a) {
 #pragma unroll
   for (int u = 0; u < C4; u++) *(float4 *)&xs[r * LD + 4 * (c + 32 * u)] = v[u];
   __syncthreads();
-  // chain ch: lane partial ch % V of row ch / V (V 0: one float64 chain a row)
-  constexpr int NCH = V > 0 ? ROWS * V : ROWS;
-  if (tid < (NCH + 63) / 64 * 64) {
-    const int ch = min(tid, NCH - 1), cr = V > 0 ? ch / (V > 0 ? V : 1) : ch;
-    float mean = 0.f;
-#pragma unroll
-    for (int pass = 0; pass < 2; pass++) {
-      double sum = 0.0;
-      if constexpr (V > 0) {
-        const float *xr = xs + cr * LD + ch % V;
-        constexpr int NE = H / V, NB = NE % 16 == 0 ? 16 : 8;  // values a lane, a batch of them
-        static_assert(NE % NB == 0, "whole batches");
-        float p = 0.f, b[NB], n[NB];
-#pragma unroll
-        for (int e = 0; e < NB; e++) b[e] = xr[V * e];
-#pragma unroll
-        for (int e0 = 0; e0 < NE; e0 += NB) {
-          if (e0 + NB < NE) {
-#pragma unroll
-            for (int e = 0; e < NB; e++) n[e] = xr[V * (e0 + NB + e)];
-          }
-#pragma unroll
-          for (int e = 0; e < NB; e++) {
-            if (pass == 0) {
-              p = p + b[e];
-            } else {
-              const float d = b[e] - mean;
-              p = __builtin_fmaf(d, d, p);
-            }
-          }
-#pragma unroll
-          for (int e = 0; e < NB; e++) b[e] = n[e];
-        }
-        const int base = lane & ~(V - 1);
-#pragma unroll
-        for (int q = 0; q < V; q++) sum += (double)__shfl(p, base + q);
-      } else {
-        const float *xr = xs + cr * LD;
-        for (int e = 0; e < H; e++) {
-          if (pass == 0) {
-            sum += (double)xr[e];
-          } else {
-            const double d = (double)(xr[e] - mean);
-            sum += d * d;
-          }
-        }
-      }
-      if (pass == 0) {
-        mean = (float)(sum / (double)H);
-      } else if (tid < NCH && (V == 0 || tid % (V > 0 ? V : 1) == 0)) {
-        mean_s[cr] = mean;
-        rstd_s[cr] = (float)(1.0 / __builtin_sqrt(sum / (double)H + a.eps));
-      }
-    }
-  }
+  if (tid < ln_chain_threads<V>(ROWS)) ln_chains<H, V, false>(xs, LD, tid, lane, ROWS, a.eps, mean_s, rstd_s);
   __syncthreads();
   const float mean = mean_s[r], rstd = rstd_s[r];
   float mx = 0.f;

@@ -25,13 +25,18 @@
 //      gated tile of 32 columns), 4 waves over the depth; also max |g| of
 //      each row's 32 columns.
 //
-// What bounds them: latency at few rows. At 24 rows of hidden 768 (36 and 24 workgroups)
-// a launch takes 4.9 us (Wi), 5.1 us (Wo) and 6.4 us (WoMLP), the LayerNorm
-// between them (ln_rows_kernel, rownorm.hip) 4.8: against 25 us (Wo + LayerNorm) and 50 us (the MLP block) on the
-// whole-row kernels, and 2.05 -> 0.93 ms a pass of 22 layers. A wave's
+//  ln_wi_split_kernel  wi_split with mlp_norm before it in the same workgroup,
+//      for the fewest rows.
+//
+// What bounds them: latency at few rows. At 24 rows of hidden 768 (36 and 24
+// workgroups) a launch takes 4.9 us (Wi; 8.0 with its LayerNorm), 5.1 us (Wo)
+// and 6.4 us (WoMLP), a LayerNorm of its own (ln_rows_kernel, rownorm.hip) 4.8:
+// against 25 us (Wo + LayerNorm) and 50 us (the MLP block) on the whole-row
+// kernels, and 2.05 -> 0.93 ms a pass of 22 layers. A wave's
 // global loads are all issued before its first MFMA. With more rows, the
 // float32 rows read from L2 and the last-level cache by every tile's
-// workgroup: at 4,096 rows WoMLP took 69 us, Wo 47, Wi 26.
+// workgroup: at 4,096 rows WoMLP took 69 us, Wo 47, Wi 26 before
+// the arrangement for many rows (kManyBlocks).
 //
 // The products are transposed as in mlp_block.hip (weights the A operand,
 // rows the B operand): a lane holds one row and 16 consecutive channels,
@@ -132,6 +137,107 @@ __global__ __launch_bounds__(256) void wi_split_kernel(SplitArgs a) {
   }
 }
 
+// wi_split_kernel with the LayerNorm before it (mlp_norm and its quantizeA) in
+// the same workgroup: each recomputes it for its 32 rows, 32 threads a row, so
+// that no launch and no int8 row stand between x and the product. The weight
+// loads of the 4 product waves are in flight during the chains of 4 others. Its
+// time is the chains' latency; us of the two kernels and of this: hidden 768 9.9
+// and 8.0 at 24 rows, 10.8 and 9.3 at 192; 384 9.5 and 6.6 at 15 rows; 256 9.5
+// and 7.1 at 480.
+template <int KT, int V>
+__global__ __launch_bounds__(1024) void ln_wi_split_kernel(SplitArgs a) {
+  constexpr int KS = 4, KW = KT / KS, H = 32 * KT, LD = H + 8, C4 = H / 128;
+  constexpr int HALF = 528, KB = 2 * HALF;  // bytes of half a K step (32 rows x 16 and a bank group's 16), a K step
+  static_assert(KT % KS == 0 && 2 * KS * 4 * 64 * 16 <= 32 * LD * 4, "depth over the waves, the sums over the rows");
+  __shared__ __attribute__((aligned(16))) float xs[32 * LD];
+  __shared__ __attribute__((aligned(16))) int8_t panel[KT * KB];
+  __shared__ __attribute__((aligned(16))) float gamma_s[H];
+  __shared__ float mean_s[32], rstd_s[32], sa_s[32], mx_s[KS][64];
+  int4 *const part = (int4 *)xs;  // [2][KS * 4 * 64], once the rows are quantised
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int t, blk;
+  if (!tile_of(a.n / 64, (a.M + 31) / 32, &t, &blk)) return;
+  const int m0 = 32 * blk, r = tid >> 5, c = tid & 31;
+  const float *xp = a.A + (size_t)min(m0 + r, a.M - 1) * a.lda + 4 * c;  // rows past M: row M-1, never stored
+  float4 v[C4];
+#pragma unroll
+  for (int u = 0; u < C4; u++) v[u] = *(const float4 *)(xp + 128 * u);
+  if (tid < H / 4) *(float4 *)&gamma_s[4 * tid] = *(const float4 *)(a.gamma + 4 * tid);
+#pragma unroll
+  for (int u = 0; u < C4; u++) *(float4 *)&xs[r * LD + 4 * (c + 32 * u)] = v[u];
+  const int fr = lane & 31, fh = lane >> 5, ks = wave & (KS - 1);
+  const int ch = 64 * t + 16 * fh + 4 * ks;  // this lane's GELU-input channels (the multiplier's: + 32)
+  v4i w[KW][2];
+  float4 sba, sbb;
+  if (wave < KS) {
+    const int8_t *wp = a.Bk + ((size_t)(ks * KW) * a.Np + 64 * t + perm32(fr)) * 32 + 16 * fh;
+#pragma unroll
+    for (int k = 0; k < KW; k++) {
+      w[k][0] = *(const v4i *)(wp + (size_t)k * a.Np * 32);
+      w[k][1] = *(const v4i *)(wp + (size_t)k * a.Np * 32 + 1024);
+    }
+    sba = *(const float4 *)(a.sb + ch);
+    sbb = *(const float4 *)(a.sb + ch + 32);
+  }
+  lds_barrier();
+  const int ct = tid - 64 * KS;
+  if (ct >= 0 && ct < ln_chain_threads<V>(32)) ln_chains<H, V, true>(xs, LD, ct, lane, 32, a.eps, mean_s, rstd_s);
+  lds_barrier();
+  const float mean = mean_s[r], rstd = rstd_s[r];
+  float mx = 0.f;
+#pragma unroll
+  for (int u = 0; u < C4; u++) {
+    const float4 x = *(const float4 *)&xs[r * LD + 4 * (c + 32 * u)], g = *(const float4 *)&gamma_s[4 * (c + 32 * u)];
+    v[u] = make_float4(((x.x - mean) * rstd) * g.x, ((x.y - mean) * rstd) * g.y, ((x.z - mean) * rstd) * g.z,
+                       ((x.w - mean) * rstd) * g.w);
+    mx = amax(amax(amax(amax(mx, v[u].x), v[u].y), v[u].z), v[u].w);
+  }
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, o));
+  float s = 0.f, inv = 0.f;
+  if (mx != 0.f) {  // quantizeA: s = max/127, inv = 1/s (int8.go:175-183)
+    s = mx / 127.0f;
+    inv = 1.0f / s;
+  }
+  if (c == 0) sa_s[r] = s;
+#pragma unroll
+  for (int u = 0; u < C4; u++) {
+    const int col = 4 * (c + 32 * u);
+    *(int *)(panel + (col >> 5) * KB + ((col >> 4) & 1) * HALF + r * 16 + (col & 15)) = pack4(v[u], inv);
+  }
+  lds_barrier();
+  v16i acc[2] = {};
+  if (wave < KS) {
+#pragma unroll
+    for (int k = 0; k < KW; k++) {
+      const v4i x = *(const v4i *)(panel + (ks * KW + k) * KB + fh * HALF + 16 * fr);
+      acc[0] = mfma32(w[k][0], x, acc[0]);
+      acc[1] = mfma32(w[k][1], x, acc[1]);
+    }
+    put_sums<KS>(part, ks, lane, acc[0]);
+    put_sums<KS>(part + KS * 4 * 64, ks, lane, acc[1]);
+  }
+  lds_barrier();
+  if (wave < KS) {
+    int4 ta, tb;
+    gather_sums<KS>(part, ks, lane, acc[0], &ta);
+    gather_sums<KS>(part + KS * 4 * 64, ks, lane, acc[1], &tb);
+    const float sa = sa_s[fr];
+    const float4 za = deq4(ta, a.small, a.c128 + ch, a.zc + ch, sba, sa);
+    const float4 zb = deq4(tb, a.small, a.c128 + ch + 32, a.zc + ch + 32, sbb, sa);
+    const float4 g = make_float4(gelu_fma(za.x) * zb.x, gelu_fma(za.y) * zb.y, gelu_fma(za.z) * zb.z, gelu_fma(za.w) * zb.w);
+    if (m0 + fr < a.M) *(float4 *)(a.C + (size_t)(m0 + fr) * a.ldc + 32 * t + 16 * fh + 4 * ks) = g;
+    mx_s[ks][lane] = amax(amax(amax(amax(0.f, g.x), g.y), g.z), g.w);
+  }
+  lds_barrier();
+  if (tid < 32 && m0 + tid < a.M) {
+    float m = 0.f;
+#pragma unroll
+    for (int q = 0; q < KS; q++) m = __builtin_fmaxf(__builtin_fmaxf(m, mx_s[q][tid]), mx_s[q][32 + tid]);
+    a.rmax[(size_t)(m0 + tid) * a.P + t] = m;
+  }
+}
+
 template <int KT, int KS, int CT>
 __global__ __launch_bounds__(64 * KS * CT) void res_split_kernel(SplitArgs a) {
   constexpr int KW = KT / KS, GO = 4 / KS;                 // K steps and accumulator groups of a wave
@@ -210,6 +316,16 @@ void wi_one(const SplitArgs &a, hipStream_t s) {
   wi_split_kernel<KT><<<tile_grid(a.n / 64, (a.M + 31) / 32), 256, 0, s>>>(a);
 }
 template <int KT>
+void ln_wi_one(const SplitArgs &a, hipStream_t s) {
+  const int grid = tile_grid(a.n / 64, (a.M + 31) / 32);
+  switch (a.lanes) {
+  case 0: ln_wi_split_kernel<KT, 0><<<grid, 1024, 0, s>>>(a); break;
+  case 4: ln_wi_split_kernel<KT, 4><<<grid, 1024, 0, s>>>(a); break;
+  case 8: ln_wi_split_kernel<KT, 8><<<grid, 1024, 0, s>>>(a); break;
+  default: ln_wi_split_kernel<KT, 16><<<grid, 1024, 0, s>>>(a); break;
+  }
+}
+template <int KT>
 void res_one(const SplitArgs &a, hipStream_t s) {
   const int nblk = (a.M + 31) / 32;
   if (nblk < kManyBlocks) res_split_kernel<KT, 4, 1><<<tile_grid(a.n / 32, nblk), 256, 0, s>>>(a);
@@ -222,6 +338,17 @@ void launch_wi_split(const SplitArgs &a, hipStream_t s) {
   if (a.K == 768) wi_one<24>(a, s);
   else if (a.K == 384) wi_one<12>(a, s);
   else wi_one<8>(a, s);
+}
+
+// one workgroup fills a CU: as long as no XCD has more than its CUs (hidden 768,
+// 224 rows, 35 workgroups on an XCD of 32 CUs: 14.6 us, the two kernels 10.8)
+bool ln_wi_split_supported(int I, int M, int cus) { return tile_grid(I / 32, (M + 31) / 32) <= cus; }
+
+void launch_ln_wi_split(const SplitArgs &a, hipStream_t s) {
+  if (a.M <= 0) return;
+  if (a.K == 768) ln_wi_one<24>(a, s);
+  else if (a.K == 384) ln_wi_one<12>(a, s);
+  else ln_wi_one<8>(a, s);
 }
 
 void launch_res_split(const SplitArgs &a, hipStream_t s) {

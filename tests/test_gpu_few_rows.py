@@ -25,7 +25,8 @@ def seqs_of(rng, vocab, *lens):
 def test_few_rows_exact(shape, lanes, plant):
     """Row counts around the 32-row blocks (and the 8 rows of a LayerNorm
     workgroup), one sequence or several, a sequence over 512 keys (QKV input
-    row-major), the two arrangements of the residual kernel (from 481 rows
+    row-major), the LayerNorm in the Wi kernel and before it (up to 192 rows,
+    shape small 512), the two arrangements of the residual kernel (from 481 rows
     on) and the two sides of the rules that pick these kernels and the
     32-row MLP kernel; setting a kernel option (here to its default) picks
     the whole-row kernels, and gives the same bits."""
@@ -36,7 +37,7 @@ def test_few_rows_exact(shape, lanes, plant):
     gpu, ora = Model(w, lanes=lanes), orc.OracleModel(w, lanes=lanes)
     rng = np.random.default_rng(97)
     batches = [seqs_of(rng, cfg.vocab, *lens)
-               for lens in ((1,), (7, 1), (31,), (9, 0, 23), (33,), (64, 1, 192), (480,), (481,), (600, 9))]
+               for lens in ((1,), (7, 1), (31,), (9, 0, 23), (33,), (192,), (193,), (64, 1, 192), (480,), (481,), (512,), (513,), (600, 9))]
     gpu.set_option("parts", 1)
     want = [ora.encode_tokens(b)[0] for b in batches]
     for b, e in zip(batches, want):
