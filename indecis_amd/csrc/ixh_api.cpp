@@ -857,6 +857,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   auto res_bytes = [&](double k, bool ln_out) {
     return dN * 4 * k + k * dH + 12 * dH + dN * 8 * dH + (ln_out ? dN * (dH + 4) : 0);
   };
+  ShortLn short_ln;      // the attn_norm that short_attn_kernel computes for this layer
   bool ln_done = false;  // the attn_norm LayerNorm of this layer ran in the previous WoMLP
   for (int l = 0; l < c.layers; l++) {
     const auto &L = m->layers[l];
@@ -886,7 +887,8 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
     if (short_seqs) {
       RUN(global ? "qkv_attn_global" : "qkv_attn_local", 2 * dN * 3 * dH * dH + 4.0 * D * nh * pairs,
           gemm_bytes(dH, 3 * dH, 0, false) + dN * dH * 4,
-          if (!launch_short_attn(g, aa, st)) return refused("qkv_attn"));
+          if (!launch_short_attn(g, aa, short_ln, st)) return refused("qkv_attn"));
+      short_ln = ShortLn{};
     } else if (fused) {
       // QKV GEMM and Attn8.Prepare in one kernel: int8 Q, K, V and their
       // scales are its only outputs
@@ -946,7 +948,10 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
       }
       RUN("gemm_womlp", 2 * dN * dH * dI, res_bytes(dI, false),
           launch_res_split(product(L.omlp, w->g.as<float>(), I, gm, I / 32, w->x.as<float>(), H, H), st));
-      if (l + 1 < c.layers) {
+      if (l + 1 < c.layers && short_seqs && short_attn_ln_supported(T, B * nh)) {
+        short_ln = {w->x.as<float>(), m->layers[l + 1].attn_norm.as<float>(), lr.eps, lr.lanes};
+        ln_done = true;
+      } else if (l + 1 < c.layers) {
         lr.gamma = m->layers[l + 1].attn_norm.as<float>();
         lr.qk = kblock ? w->xqk.as<int8_t>() : nullptr;
         RUN("ln_quant", 0, ln_bytes, launch_rownorm(lr, st));

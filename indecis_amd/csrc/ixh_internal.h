@@ -324,7 +324,16 @@ void launch_qkv_attn(const GemmArgs &g, const AttnArgs &a, const int32_t *order,
 // launch_attn_main (of the prologue's outputs nothing is written); false
 // (nothing launched) otherwise.
 bool short_attn_supported(int Kp, int max_n, int workgroups);
-bool launch_short_attn(const GemmArgs &g, const AttnArgs &a, hipStream_t s);
+// The LayerNorm (and quantisation) of the rows before it in the same kernel,
+// when x is not null: sequences of at most 32 tokens, a workgroup a CU.
+struct ShortLn {
+  const float *x = nullptr;  // [N][H]
+  const float *gamma = nullptr;
+  double eps = 0;
+  int lanes = 0;
+};
+bool short_attn_ln_supported(int max_n, int workgroups);
+bool launch_short_attn(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStream_t s);
 // The fused QKV kernel's K-blocked input ([Kp/32][rows][32]): supported
 // for Kp a multiple of 128 whose weight rows fit in its LDS.
 bool qkv_kblock_supported(int Kp);

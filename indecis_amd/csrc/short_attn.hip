@@ -53,9 +53,25 @@ struct Shape {
   static constexpr int SMEM = QKV + 2 * R * BLD + D * VLD + RT * RT * 64 * 16;
 };
 
-template <int KT, int RT>
-__global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a) {
+// The LayerNorm variant's LDS past Shape<1>'s: the int8 rows as MFMA operands
+// (half a K step is 32 rows x 16 bytes, padded by a bank group's 16), gamma.
+template <int KT>
+struct LnShape {
+  static constexpr int H = 32 * KT, LD = H + 8, HALF = 528, KB = 2 * HALF;
+  static constexpr int SMEM = Shape<1>::SMEM + KT * KB + 4 * H;
+  static_assert(4 * 32 * LD <= Shape<1>::QKV, "the float32 rows under the partial sums");
+};
+
+// LNV: -1, or (one row block) the lane width of the LayerNorm and quantisation
+// of the sequence's rows done first by each head's workgroup, 32 threads a row,
+// the weight loads in flight meanwhile. us a layer, the LayerNorm kernel and this
+// one, then both in one: hidden 768, 24 rows 13.6 and 11.7; 384, 15 rows 12.7
+// and 9.5; 256, 64 sequences of 15 12.4 and 9.8.
+template <int KT, int RT, int LNV>
+__global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a, ShortLn ln) {
   using S = Shape<RT>;
+  constexpr bool LN = LNV >= 0;
+  static_assert(!LN || RT == 1, "one row block");
   constexpr int KS = S::KS, GO = 4 / KS, KW = KT / KS, R = S::R, VLD = S::VLD, NG = S::NG;
   constexpr int PF = KW <= 6 ? KW : 4;  // K steps in flight
   static_assert(KT % KS == 0 && KW % PF == 0, "depth");
@@ -67,6 +83,10 @@ __global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a)
   __shared__ __attribute__((aligned(16))) float mean_s[D], vs_s[D], sq_s[R], ks_s[R];
   __shared__ float vmax_s[4][D], mx_s[RT][NG][64], om_s[2][R];
   __shared__ int vsum_s[D], psum_s[R];
+  __shared__ float lmean_s[LN ? 32 : 1], lrstd_s[LN ? 32 : 1], sa_s[LN ? 32 : 1];
+  using SL = LnShape<KT>;
+  float *const xs = (float *)smem, *const gamma_s = (float *)(smem + S::SMEM + KT * SL::KB);
+  int8_t *const panel = smem + S::SMEM;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 31, fh = lane >> 5;
   // item = head * B + sequence; each XCD takes a contiguous run of items, so
@@ -92,10 +112,24 @@ __global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a)
   const auto wrs = buf_rsrc(g.Bk, (uint32_t)KT * g.Np * 32), xrs = buf_rsrc(g.Ak, (uint32_t)KT * g.ak_rows * 32);
   const uint32_t wvo = (uint32_t)(wrow + lw) * 32 + 16 * fh, xvo = (uint32_t)(base + tok) * 32 + 16 * fh;
   const uint32_t wst = (uint32_t)g.Np * 32, xst = (uint32_t)g.ak_rows * 32;
+  if constexpr (LN) {  // the float32 rows, 24 at a time (as many as the threads hold)
+    const int lr = tid >> 5, lc = 4 * (tid & 31);
+    float4 v[SL::H / 128];
+    for (int r = lr; r - lr < n; r += 24) {
+      const float *xp = ln.x + (size_t)(base + min(r, n - 1)) * SL::H + lc;
+#pragma unroll
+      for (int u = 0; u < SL::H / 128; u++) v[u] = *(const float4 *)(xp + 128 * u);
+      if (r < 32) {
+#pragma unroll
+        for (int u = 0; u < SL::H / 128; u++) *(float4 *)&xs[r * SL::LD + lc + 128 * u] = v[u];
+      }
+    }
+    if (tid < SL::H / 4) *(float4 *)&gamma_s[4 * tid] = *(const float4 *)(ln.gamma + 4 * tid);
+  }
   v4i w[PF][2], x[PF];
   auto load = [&](int k, int s) {
     const uint32_t kk = ks * KW + k;
-    x[s] = __builtin_amdgcn_raw_buffer_load_b128(xrs, xvo, __builtin_amdgcn_readfirstlane(kk * xst), 0);
+    if constexpr (!LN) x[s] = __builtin_amdgcn_raw_buffer_load_b128(xrs, xvo, __builtin_amdgcn_readfirstlane(kk * xst), 0);
     w[s][0] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wvo, __builtin_amdgcn_readfirstlane(kk * wst), 0);
     w[s][1] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wvo + 1024, __builtin_amdgcn_readfirstlane(kk * wst), 0);
   };
@@ -108,7 +142,7 @@ __global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a)
   int vc1[2];
   auto constants = [&] {
     if (part < 2) {
-      psa[0][0] = g.sa[base + tok];
+      if constexpr (!LN) psa[0][0] = g.sa[base + tok];
 #pragma unroll
       for (int q = 0; q < GO; q++) {
         const int d0 = 16 * fh + 4 * (GO * ks + q);
@@ -129,10 +163,53 @@ __global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a)
       for (int q = 0; q < GO; q++)
 #pragma unroll
         for (int u = 0; u < 4; u++)  // rows past n: row n-1 again
-          psa[q][u] = g.sa[base + min(32 * rt + 8 * (GO * ks + q) + 4 * fh + u, n - 1)];
+          if constexpr (!LN) psa[q][u] = g.sa[base + min(32 * rt + 8 * (GO * ks + q) + 4 * fh + u, n - 1)];
     }
   };
   if constexpr (RT == 1) constants();
+  if constexpr (LN) {
+    static_assert(KW == PF, "every weight load in flight");
+    lds_barrier();
+    if (tid < ln_chain_threads<LNV>(n)) ln_chains<SL::H, LNV, true>(xs, SL::LD, tid, lane, n, ln.eps, lmean_s, lrstd_s);
+    lds_barrier();
+    const int lc = 4 * (tid & 31);
+    for (int r = tid >> 5; r < n; r += 24) {
+      const float mean = lmean_s[r], rstd = lrstd_s[r];
+      float4 v[SL::H / 128];
+      float mx = 0.f;
+#pragma unroll
+      for (int u = 0; u < SL::H / 128; u++) {
+        const float4 t = *(const float4 *)&xs[r * SL::LD + lc + 128 * u], gm = *(const float4 *)&gamma_s[lc + 128 * u];
+        v[u] = make_float4(((t.x - mean) * rstd) * gm.x, ((t.y - mean) * rstd) * gm.y, ((t.z - mean) * rstd) * gm.z,
+                           ((t.w - mean) * rstd) * gm.w);
+        mx = amax(amax(amax(amax(mx, v[u].x), v[u].y), v[u].z), v[u].w);
+      }
+#pragma unroll
+      for (int o = 1; o < 32; o <<= 1) mx = __builtin_fmaxf(mx, __shfl_xor(mx, o));
+      float sc = 0.f, inv = 0.f;
+      if (mx != 0.f) {  // quantizeA: s = max/127, inv = 1/s (int8.go:175-183)
+        sc = mx / 127.0f;
+        inv = 1.0f / sc;
+      }
+      if (lc == 0) sa_s[r] = sc;
+#pragma unroll
+      for (int u = 0; u < SL::H / 128; u++) {
+        const int col = lc + 128 * u;
+        *(int *)(panel + (col >> 5) * SL::KB + ((col >> 4) & 1) * SL::HALF + r * 16 + (col & 15)) = pack4(v[u], inv);
+      }
+    }
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < PF; k++) x[k] = *(const v4i *)(panel + (ks * KW + k) * SL::KB + fh * SL::HALF + 16 * tok);
+    if (part < 2) {
+      psa[0][0] = sa_s[tok];
+    } else {
+#pragma unroll
+      for (int q = 0; q < GO; q++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) psa[q][u] = sa_s[min(8 * (GO * ks + q) + 4 * fh + u, n - 1)];
+    }
+  }
   const bool small = g.small;
   v16i acc[2] = {};
   auto products = [&](auto vpart) {
@@ -379,22 +456,31 @@ __global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a)
   }
 }
 
-template <int KT, int RT>
-bool launch_one(const GemmArgs &g, const AttnArgs &a, hipStream_t s) {
-  constexpr int shm = Shape<RT>::SMEM;
+template <int KT, int RT, int LNV>
+bool launch_one(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStream_t s) {
+  constexpr int shm = LNV < 0 ? Shape<RT>::SMEM : LnShape<KT>::SMEM;
   // the device's grant of that much LDS: 1 granted, -1 refused, 0 not asked yet
   static std::atomic<int> state{0};
+  const auto kern = short_attn_kernel<KT, RT, LNV>;
   if (state.load() == 0)
-    state = hipFuncSetAttribute((const void *)short_attn_kernel<KT, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, shm) == hipSuccess ? 1 : -1;
+    state = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm) == hipSuccess ? 1 : -1;
   if (state.load() < 0) return false;
-  short_attn_kernel<KT, RT><<<NXCD * ((a.B * a.nh + NXCD - 1) / NXCD), 768, shm, s>>>(g, a);
+  kern<<<NXCD * ((a.B * a.nh + NXCD - 1) / NXCD), 768, shm, s>>>(g, a, ln);
   return true;
 }
 template <int KT>
-bool launch_kt(const GemmArgs &g, const AttnArgs &a, hipStream_t s) {
-  if (a.max_n <= 32) return launch_one<KT, 1>(g, a, s);
-  if (a.max_n <= 64) return launch_one<KT, 2>(g, a, s);
-  return launch_one<KT, 4>(g, a, s);
+bool launch_kt(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStream_t s) {
+  if (ln.x) {
+    switch (ln.lanes) {
+    case 0: return launch_one<KT, 1, 0>(g, a, ln, s);
+    case 4: return launch_one<KT, 1, 4>(g, a, ln, s);
+    case 8: return launch_one<KT, 1, 8>(g, a, ln, s);
+    default: return launch_one<KT, 1, 16>(g, a, ln, s);
+    }
+  }
+  if (a.max_n <= 32) return launch_one<KT, 1, -1>(g, a, ln, s);
+  if (a.max_n <= 64) return launch_one<KT, 2, -1>(g, a, ln, s);
+  return launch_one<KT, 4, -1>(g, a, ln, s);
 }
 
 }  // namespace
@@ -409,12 +495,16 @@ bool short_attn_supported(int Kp, int max_n, int workgroups) {
   return max_n <= 32 || (max_n <= 64 && workgroups <= 2 * device_cus()) || (max_n <= 128 && workgroups <= device_cus());
 }
 
-bool launch_short_attn(const GemmArgs &g, const AttnArgs &a, hipStream_t s) {
+// a workgroup fills a CU (154 KB of LDS): one round of them
+bool short_attn_ln_supported(int max_n, int workgroups) { return max_n <= 32 && workgroups <= device_cus(); }
+
+bool launch_short_attn(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStream_t s) {
   if (a.B <= 0) return true;
-  if (!short_attn_supported(g.Kp, a.max_n, a.B * a.nh) || !g.Ak) return false;
-  if (g.Kp == 768) return launch_kt<24>(g, a, s);
-  if (g.Kp == 384) return launch_kt<12>(g, a, s);
-  return launch_kt<8>(g, a, s);
+  if (!short_attn_supported(g.Kp, a.max_n, a.B * a.nh) || !(g.Ak || ln.x)) return false;
+  if (ln.x && !short_attn_ln_supported(a.max_n, a.B * a.nh)) return false;
+  if (g.Kp == 768) return launch_kt<24>(g, a, ln, s);
+  if (g.Kp == 384) return launch_kt<12>(g, a, ln, s);
+  return launch_kt<8>(g, a, ln, s);
 }
 
 }  // namespace ixh

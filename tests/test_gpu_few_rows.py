@@ -62,7 +62,8 @@ def test_short_sequences_exact(shape, lanes, window, plant):
     window that cuts sequences and one that does not, empty sequences, QKV
     rows past the dequantisation bound, and batches one workgroup either side
     of the rules that pick it (two rounds of the 256 CUs up to 64 tokens, one
-    up to 128), against the oracle."""
+    up to 128) and with the LayerNorm before it in the same kernel (at most 32
+    tokens, 24 rows at a time, one round), against the oracle."""
     cfg = SHAPES[shape](layers=2, local_attention=window)
     w = Weights.random(cfg, seed=101)
     if plant:
@@ -73,6 +74,7 @@ def test_short_sequences_exact(shape, lanes, window, plant):
     batches = [(1,), (15, 2), (31, 0, 1), (32, 32, 17), (33, 5), (40, 0, 63, 1), (64, 33), (65, 31), (97, 8), (127,),
                (128, 1, 90), (129, 3)]
     two, one = 512 // cfg.heads, 256 // cfg.heads
+    batches += [(24,), (25, 24, 3), (30,) + (2,) * (one - 1), (30,) + (2,) * one]
     batches += [(33,) + (2,) * (two - 1), (33,) + (2,) * two, (65,) + (2,) * (one - 1), (65,) + (2,) * one]
     for lens in batches:
         seqs = seqs_of(rng, cfg.vocab, *lens)
