@@ -593,7 +593,9 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 ? 4 : 2) void attn_main_kerne
   const float kap = (64.0f + 3.5f * fabsf(m)) * 0x1p-24f;
   float eb = __builtin_fmaf(-m, 1.44269504088896341f, 7.99435343685885793f) - 1.4427f * kap;
   float hi = 1.0f + 2.125f * kap;  // (1 - kap) hi >= 1 + kap
-  if (qact && !(fabsf(m) <= 32768.0f)) {  // y = 1, its upper bound 300
+  // (also a query scale whose product with log2 e overflows: such a scale
+  // times the scores can still be finite). y = 1, its upper bound 300
+  if (qact && !(fabsf(m) <= 32768.0f && es < __builtin_huge_valf())) {
     es = 0.0f;
     eb = 0.0f;
     hi = 300.0f;

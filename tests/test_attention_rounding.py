@@ -60,3 +60,26 @@ def test_attend8_score_magnitudes(scale, lanes):
         q[n // 2] = 0
         got, want = linalg.attend8(q, k, v, window, 0.125, lanes), orc.attend8(q, k, v, window, 0.125, lanes)
         assert f32_bits_equal(got, want), (n, window, mismatch_report(got, want))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lanes", [8, 0])
+@pytest.mark.parametrize("qmax", [3.2e38, 2.9e38])
+def test_attend8_query_scale_overflow(qmax, lanes):
+    """Queries near the largest float with a scale of 100: the query scale
+    max|q|/127*100 is finite (2.5e38 and 2.3e38), its product with log2 e is
+    not (it is, for the second), and the scores are a few units (one key:
+    zero), against the oracle, bit for bit."""
+    from indecis_amd import linalg
+    from oracle import oracle as orc
+    rng = np.random.default_rng(lanes)
+    for n, window in ((1, -1), (2, -1), (33, 4), (300, -1), (700, 64)):
+        q, k = np.zeros((n, 64), np.float32), (3e-37 * rng.standard_normal((n, 64))).astype(np.float32)
+        q[:, 0] = qmax
+        q[:, 1] = np.float32(qmax) / np.float32(127) * rng.integers(1, 3, n).astype(np.float32)
+        k[:, 0] = 0
+        k[:, 1] *= np.float32(0.05)
+        v = rng.standard_normal((n, 64)).astype(np.float32)
+        got, want = linalg.attend8(q, k, v, window, 100.0, lanes), orc.attend8(q, k, v, window, 100.0, lanes)
+        assert np.isfinite(want).all()
+        assert f32_bits_equal(got, want), (n, window, mismatch_report(got, want))
