@@ -388,7 +388,9 @@ int ixh_attend8(int device, float *o, const float *q, const float *k,
  * 255*exp(s - max) with the device's base-2 exponential and fall back to
  * the reference's exp32 formulas where the value is within a tolerance of
  * a rounding boundary. For every float v in [-inf, -0] and +0 this counts
- * the v where that shortcut would round differently from the reference:
+ * the v where that shortcut would round differently from the reference and,
+ * where P is above 0 (v >= -6.4), those where it is further from 255*exp(v)
+ * than the 10 * 2^-24 of it that the attention kernels' error bound takes:
  * bad[0] for the vector formula (ExpShift's SIMD body), bad[1] for the
  * scalar exp32; both must be 0. max_err[0..1]: the largest distance of the
  * shortcut from 255*exp(v) of each formula; *undecided: how many v take the

@@ -578,19 +578,24 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 ? 4 : 2) void attn_main_kerne
   // formula elsewhere.
   //
   // The error, with u = 2^-24 and the scores that matter (P > 0: s - m >
-  // -6.3, so |s| <= |m| + 6.3): the reference's own roundings of s and of s -
-  // m move the exponent by log2 e (|s| + |s - m|) u, the products and the
-  // constants here by (|s| log2 e + 8 + |m| log2 e + 8) u, the exponent's
-  // rounding in exp255_fast 8 u: together (51.3 + 4.33 |m|) u, times ln 2 in
-  // y; exp255_fast against the reference formulas 8 u (the relative form of
-  // kExp255Tol), the hardware exponential twice and the scaling by hi 6 u:
-  // (50 + 3 |m|) u, taken as kap = (64 + 3.5 |m|) u. Past |m| = 2^15 every
+  // -6.3, so |s| <= |m| + 6.3). In the exponent, against the one that
+  // exp255_fast forms of the reference's s - m: the reference's roundings of s
+  // and of s - m log2 e (|s| + |s - m|) u, that of es log2 e |s| u, the two of
+  // eb (the fma, then kap's subtraction) 2 (log2 e |m| + 8) u, that of either
+  // exponent 8 u; the constants are the same in both. Together (59.3 + 4 log2 e
+  // |m|) u, times ln 2 in y: (41.1 + 4 |m|) u. exp255_fast against the reference
+  // formulas 10 u (kExp255Rel), the hardware exponential twice and the scaling
+  // by hi 6 u. The sum, (57.1 + 4 |m|) u, is taken as kap = (64 + 4.25 |m|) u;
+  // kap <= 0.0084, so its squares stay inside the 0.125 kap that hi has over
+  // (1 + kap) / (1 - kap). A lower score (s - m < -6.3, 255 exp below 0.469) stays
+  // under a half: per unit of |s| past |m| + 6.3 its error gains 3 u while its
+  // logarithm falls by 1. Past |m| = 2^15 every
   // group takes the other way. 11 VALU slots a score instead of 13 (the
   // exponential takes 4) and fewer scores formed twice: global layers of
   // 8,192 tokens 2,900 -> 2,650 us a launch, of 4,096 162 -> 146, of 256 64.5
   // -> 60.3; local layers 97 -> 93.5 and 50.2 -> 49.
   float es = sqv * 1.44269504088896341f;
-  const float kap = (64.0f + 3.5f * fabsf(m)) * 0x1p-24f;
+  const float kap = (64.0f + 4.25f * fabsf(m)) * 0x1p-24f;
   float eb = __builtin_fmaf(-m, 1.44269504088896341f, 7.99435343685885793f) - 1.4427f * kap;
   float hi = 1.0f + 2.125f * kap;  // (1 - kap) hi >= 1 + kap
   // (also a query scale whose product with log2 e overflows: such a scale
@@ -794,7 +799,8 @@ __global__ __launch_bounds__(256 * KSPL, KSPL == 1 ? 4 : 2) void attn_main_kerne
 // Every float v = bits -> float over [lo, hi) (v <= 0 expected): counts
 // the v where exp255_fast decides the rounding (away from a half-integer by
 // more than kExp255Tol) and RNE differs from the reference's
-// RNE(f32(255*exp(v))), for exp32_simd (res[0]) and exp32_scalar (res[1]);
+// RNE(f32(255*exp(v))), and the v >= -6.4 where exp255_fast is further than
+// kExp255Rel from f32(255*exp(v)), for exp32_simd (res[0]) and exp32_scalar (res[1]);
 // res[2], res[3]: largest |exp255_fast - 255*exp| of each formula, as
 // float bits; res[4]: number of undecided v.
 __global__ __launch_bounds__(256) void check_exp255_kernel(uint32_t lo, uint32_t hi,
@@ -810,6 +816,10 @@ __global__ __launch_bounds__(256) void check_exp255_kernel(uint32_t lo, uint32_t
     const float yv = exp32_simd(v) * 255.0f, ys = exp32_scalar(v) * 255.0f;
     err_v = amax(err_v, y - yv);
     err_s = amax(err_s, y - ys);
+    if (v >= -6.4f) {  // where P > 0: the relative distance too
+      bad_v += fabsf(y - yv) > kExp255Rel * yv;
+      bad_s += fabsf(y - ys) > kExp255Rel * ys;
+    }
     if (decided) {
       bad_v += rne(yv) != p;
       bad_s += rne(ys) != p;

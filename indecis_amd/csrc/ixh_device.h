@@ -120,6 +120,9 @@ __device__ __forceinline__ float4 buf_load_f4(__amdgpu_buffer_rsrc_t r, uint32_t
 // |exp255_fast - 255*exp32| over those floats is 7.63e-5 (5 ulp at 255);
 // the tolerance is 1.6 times that.
 constexpr float kExp255Tol = 1.0f / 8192;
+// Relative to 255*exp32, for v >= -6.4 (below, P is 0): verified there float
+// by float too. (6.1 2^-24 with an exact 2^x; v_exp_f32 adds up to 2.)
+constexpr float kExp255Rel = 10.0f * 0x1p-24f;
 __device__ __forceinline__ float exp255_fast(float v) {
   return __builtin_amdgcn_exp2f(__builtin_fmaf(v, 1.44269504088896341f, 7.99435343685885793f));
 }

@@ -1,11 +1,15 @@
 """The bound behind the attention kernel's rounding of P (attention_i8.hip):
 the exponent it forms in one fused step against the reference's roundings,
 on the CPU; and, on the GPU, scores of every magnitude against the oracle."""
+import os
+import re
+
 import numpy as np
 import pytest
 
 from helpers import f32_bits_equal, mismatch_report
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 L2E, L255, U = np.float32(1.44269504088896341), np.float32(7.99435343685885793), 2.0 ** -24
 
 
@@ -14,12 +18,36 @@ def fma(a, b, c):
     return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)).astype(np.float32)
 
 
+def kap_terms():
+    """(c, d) of the kernel's kap = (c + d |m|) u."""
+    src = open(os.path.join(ROOT, "indecis_amd", "csrc", "attention_i8.hip")).read()
+    return [float(t) for t in re.search(r"kap = \(([0-9.]+)f \+ ([0-9.]+)f \* fabsf\(m\)\) \* 0x1p-24f", src).groups()]
+
+
+def test_kap_covers_every_rounding():
+    """kap against the roundings counted one by one, each at its largest: in
+    the exponent s and s - m (the reference's), es, the two of eb, the exponent
+    itself on either side; then exp255_fast against the reference formulas
+    (10 u, verified float by float on the device), two hardware exponentials
+    of 2 u and the scaling by hi. |s| <= |m| + 6.3; the constants' own errors
+    are the same on both sides."""
+    c, d = kap_terms()
+    l2e, ln2 = 1.0 / np.log(2.0), np.log(2.0)
+    for m in (0.0, 1.0, 18.0, 100.0, 32768.0):
+        s = m + 6.3
+        exponent = l2e * (s + 6.3) + l2e * s + 2 * (l2e * m + 8) + 2 * 8
+        assert exponent * ln2 + 10 + 4 + 2 <= c + d * m, m
+        kap = (c + d * m) * U  # the two bounds: e^-kap times, and that hi = 1 + 2.125 kap times
+        assert (1 + kap) * np.exp(-kap) <= 1 and (1 - kap) * np.exp(-kap) * (1 + 2.125 * kap) >= 1
+
+
 @pytest.mark.parametrize("top", [0.01, 1.0, 8.0, 300.0, 32768.0])
 def test_exponent_error_bound(top):
     """x = f32(q.k)*ks, sq and the row max m at random, scores s = x*sq
-    within 6.3 of m: the kernel's exponent differs from the one that
-    exp255_fast forms of f32(f32(x*sq) - m) by at most (51.3 + 4.33 |m|) u,
-    and 255*exp(s - m) lies between its two bounds."""
+    within 6.3 of m: the kernel's exponent, kap's share of it added back,
+    differs from the one that exp255_fast forms of f32(f32(x*sq) - m) by at
+    most (59.3 + 4 log2 e |m|) u, and 255*exp(s - m) lies between its two
+    bounds."""
     rng = np.random.default_rng(5)
     n = 400000
     m = (rng.uniform(-top, top, n)).astype(np.float32)
@@ -32,11 +60,14 @@ def test_exponent_error_bound(top):
     ref = fma(d, np.full_like(d, L2E), np.full_like(d, L255))
     es = (sq * L2E).astype(np.float32)
     base = fma(-m, np.full_like(m, L2E), np.full_like(m, L255))
-    err = np.abs(fma(x, es, base).astype(np.float64) - ref)
     am = np.abs(m).astype(np.float64)
-    assert np.all(err <= (51.3 + 4.33 * am) * U), (err / ((51.3 + 4.33 * am) * U)).max()
-    kap = ((np.float32(64) + np.float32(3.5) * np.abs(m)) * np.float32(U)).astype(np.float32)
-    y = np.exp2(fma(x, es, (base - np.float32(1.4427) * kap).astype(np.float32)).astype(np.float64))
+    k0, k1 = kap_terms()
+    kap = ((np.float32(k0) + np.float32(k1) * np.abs(m)) * np.float32(U)).astype(np.float32)
+    low = (np.float32(1.4427) * kap).astype(np.float32)
+    arg = fma(x, es, (base - low).astype(np.float32)).astype(np.float64)
+    err, bound = np.abs(arg + low - ref), (59.3 + 4 * 1.442696 * am) * U
+    assert np.all(err <= bound), (err / bound).max()
+    y = np.exp2(arg)
     hi = (np.float32(1) + np.float32(2.125) * kap).astype(np.float64)
     true = 255.0 * np.exp(d.astype(np.float64))
     # 12 u: the share of the hardware exponential and of the reference formulas
