@@ -185,9 +185,9 @@ int ixh_model_set_rope(ixh_model *m, int is_global, const float *cos_t,
  * reference, whose only knob is the worker count, linalg.SetWorkers).
  * Results never depend on them (the tests check every choice against the
  * oracle); they only move time. Each call reads the handle's values once.
- * Setting a kernel option (any but PARTS and PASS_TOKENS, to any value)
- * fixes the options' kernels for every batch size; until then batches of
- * few rows take kernels of their own. */
+ * Batches of few rows and of short sequences take kernels of their own while
+ * FEW_ROWS is 1 and every kernel option (all but PARTS and PASS_TOKENS) has
+ * its default; otherwise the options' kernels run at every batch size. */
 enum {
   IXH_OPT_PARTS = 0,       /* streams a large batch is split over: 0 auto (default), 1..4 */
   IXH_OPT_PASS_TOKENS = 1, /* most tokens of one pass, 1..131072 (default): larger
@@ -213,6 +213,9 @@ enum {
                               (written so by the MLP kernel and the embedding LayerNorm) and
                               keeps the head's weight rows in LDS (needs FUSE_MLP); 0:
                               row-major rows through an LDS ring */
+  IXH_OPT_FEW_ROWS = 10,   /* 1 (default): the kernels of few rows and short sequences, while
+                              every kernel option has its default; 0: the options' kernels
+                              at every batch size */
 };
 int ixh_model_set_option(ixh_model *m, int option, int64_t value);
 int ixh_model_get_option(ixh_model *m, int option, int64_t *value);

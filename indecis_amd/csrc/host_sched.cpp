@@ -30,12 +30,10 @@ int set_tuning(Tuning &t, int option, int64_t v, bool model_opts) {
   case IXH_OPT_GEMM:
     if (v < 0 || v > 2) return bad();
     t.gemm = (int)v;
-    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_GEMM_TILE:
     if (v < 0 || v > 2) return bad();
     t.gemm_tile = (int)v;
-    t.fixed = true;
     return IXH_OK;
   default: break;
   }
@@ -52,32 +50,30 @@ int set_tuning(Tuning &t, int option, int64_t v, bool model_opts) {
   case IXH_OPT_QKV_FUSED:
     if (v != 0 && v != 1) return bad();
     t.qkv_fused = (int)v;
-    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_QKV_HEADS:
     if (v != 1 && v != 2) return bad();
     t.qkv_heads = (int)v;
-    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_LN_SEG:
     if (v != 0 && v != 1) return bad();
     t.ln_seg = (int)v;
-    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_FUSE_RES:
     if (v < 0 || v > 4) return bad();
     t.fuse_res = (int)v;
-    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_FUSE_MLP:
     if (v < 0 || v > 2) return bad();
     t.fuse_mlp = (int)v;
-    t.fixed = true;
     return IXH_OK;
   case IXH_OPT_QKV_KBLOCK:
     if (v != 0 && v != 1) return bad();
     t.qkv_kblock = (int)v;
-    t.fixed = true;
+    return IXH_OK;
+  case IXH_OPT_FEW_ROWS:
+    if (v != 0 && v != 1) return bad();
+    t.few_rows = (int)v;
     return IXH_OK;
   default: return fail(IXH_EINVAL, "indecis: unknown option %d", option);
   }
@@ -95,6 +91,7 @@ int get_tuning(const Tuning &t, int option, int64_t *v) {
   case IXH_OPT_FUSE_RES: *v = t.fuse_res; return IXH_OK;
   case IXH_OPT_FUSE_MLP: *v = t.fuse_mlp; return IXH_OK;
   case IXH_OPT_QKV_KBLOCK: *v = t.qkv_kblock; return IXH_OK;
+  case IXH_OPT_FEW_ROWS: *v = t.few_rows; return IXH_OK;
   default: return fail(IXH_EINVAL, "indecis: unknown option %d", option);
   }
 }

@@ -35,9 +35,16 @@ struct Tuning {
   int fuse_mlp = 2;       // the MLP block (Wi, GeGLU, quantizeA, WoMLP, next LN) as one kernel:
                           // 2 mlp_block (64 rows, transposed), 1 mlp_res (32 rows), 0 separate
   int qkv_kblock = 1;     // the fused QKV kernel reads its input rows K-blocked (1) or row-major (0)
-  // a kernel option was set: the options' kernels at every batch size
-  // (unset, batches of few rows take kernels of their own)
-  bool fixed = false;
+  int few_rows = 1;       // kernels of their own for few rows and short sequences (1) or not (0)
+
+  // The options' kernels at every batch size: few_rows 0, or a kernel option
+  // away from its default (back at it, the handle chooses as a new one does).
+  bool fixed() const {
+    const Tuning d;
+    return !few_rows || qkv_fused != d.qkv_fused || qkv_heads != d.qkv_heads || gemm != d.gemm ||
+           gemm_tile != d.gemm_tile || ln_seg != d.ln_seg || fuse_res != d.fuse_res || fuse_mlp != d.fuse_mlp ||
+           qkv_kblock != d.qkv_kblock;
+  }
 };
 
 // Upper bound of Tuning::pass_tokens.

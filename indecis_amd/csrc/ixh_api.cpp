@@ -616,14 +616,14 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   const bool mlp_common = m->layers[0].i.qk.p && m->layers[0].omlp.qk.p && gelu_fma_cols(I, c.lanes) == I;
   bool mats_small = true;  // the 64-row kernel dequantises as f32(acc) * sb * sa
   for (int l = 0; l < c.layers; l++) mats_small = mats_small && m->layers[l].i.small && m->layers[l].omlp.small;
-  const bool mlp32 = !tune.fixed && N <= kMlp32RowsMax && mlp_common && fuse_res &&
+  const bool mlp32 = !tune.fixed() && N <= kMlp32RowsMax && mlp_common && fuse_res &&
                      mlp_res_supported(H, I, KpH, KpI, m->layers[0].i.np);
   const bool mlp_block = !mlp32 && mlp_common && tune.fuse_mlp == 2 && mats_small &&
                          mlp_block_supported(H, I, KpH, KpI, m->layers[0].i.np);
   const bool fuse_mlp = mlp_block || (mlp_common && fuse_res && tune.fuse_mlp != 0 &&
                                       mlp_res_supported(H, I, KpH, KpI, m->layers[0].i.np));
   // few rows: Wo and the MLP cut by output channel (split_rows.hip)
-  const bool split = !tune.fixed && N <= split_rows_max(H) && split_rows_supported(H, I, KpH, KpI) &&
+  const bool split = !tune.fixed() && N <= split_rows_max(H) && split_rows_supported(H, I, KpH, KpI) &&
                      m->layers[0].o.qk.p && mlp_common;
   // the fused QKV kernel's input rows K-blocked (the weight rows then stay
   // in LDS): written so by the embedding LayerNorm and by the MLP kernel of
@@ -632,7 +632,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
                       m->layers[0].qkv.qk.p;
 
   // short sequences: QKV, Attn8.Prepare and attention in one kernel
-  const bool short_seqs = !tune.fixed && kblock && short_attn_supported(KpH, T, B * nh);
+  const bool short_seqs = !tune.fixed() && kblock && short_attn_supported(KpH, T, B * nh);
 
   int rc;
   std::vector<int32_t> groups;
@@ -752,7 +752,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
     ra.qk_rows = N;
   }
   ra.seg = tune.ln_seg;
-  ra.few = !tune.fixed && N <= kFewRowsMax;
+  ra.few = !tune.fixed() && N <= kFewRowsMax;
   RUN("emb_ln_quant", 0, dN * (4 + row_bytes + 4 * dH + dH + 4), launch_rownorm(ra, st));
 
   auto gemm = [&](int epi, const Mat &M, int Kp, float *C, int ldc, int n_valid) {
@@ -818,7 +818,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   ln.ldq = KpH;
   ln.sa = w->sa.as<float>();
   ln.seg = tune.ln_seg;
-  ln.few = !tune.fixed;
+  ln.few = !tune.fixed();
   const double ln_bytes = dN * (4 * dH + dH + 4);
 
   float *const cmax = stream_ctx || split ? w->cmax.as<float>() : nullptr;
@@ -1062,7 +1062,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
     r.eps = c.norm_eps;
     r.lanes = c.lanes;
     r.seg = tune.ln_seg;
-    r.few = !tune.fixed;
+    r.few = !tune.fixed();
     r.out = xn;
     RUN("final_norm", 0, dN * 8 * dH, launch_rownorm(r, st));
   }

@@ -260,8 +260,10 @@ class Model:
 
     def set_option(self, name, value):
         """A kernel or pass choice (ixh_model_set_option): parts,
-        pass_tokens, qkv_fused, qkv_heads, gemm, gemm_tile, ln_seg.
-        Results never depend on it."""
+        pass_tokens, qkv_fused, qkv_heads, gemm, gemm_tile, ln_seg, fuse_res,
+        fuse_mlp, qkv_kblock, few_rows. Results never depend on it. While any
+        but parts and pass_tokens is away from its default, few rows and short
+        sequences do without kernels of their own."""
         _lib.check(self._L.ixh_model_set_option(self._h, _lib.OPTIONS[name], int(value)))
 
     def option(self, name):

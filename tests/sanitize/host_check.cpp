@@ -281,6 +281,7 @@ static void check_options() {
       {IXH_OPT_FUSE_RES, 0, 4, false, &ixh::Tuning::fuse_res},
       {IXH_OPT_FUSE_MLP, 0, 2, false, &ixh::Tuning::fuse_mlp},
       {IXH_OPT_QKV_KBLOCK, 0, 1, false, &ixh::Tuning::qkv_kblock},
+      {IXH_OPT_FEW_ROWS, 0, 1, false, &ixh::Tuning::few_rows},
   };
   for (const Opt &o : opts) {
     for (int64_t v : {(int64_t)o.lo - 1, (int64_t)o.lo, (int64_t)o.lo + 1, (int64_t)o.hi - 1, (int64_t)o.hi,
@@ -299,7 +300,19 @@ static void check_options() {
       }
     }
   }
+  // a kernel option away from its default fixes the options' kernels; read,
+  // changed and set back, the handle chooses as a new one
   ixh::Tuning t;
+  CHECK(!t.fixed(), "a new handle's kernels fixed");
+  for (const Opt &o : opts) {
+    int64_t old = -1, other;
+    CHECK(ixh::get_tuning(t, o.id, &old) == 0, "get option %d", o.id);
+    CHECK(ixh::set_tuning(t, o.id, old, true) == 0 && !t.fixed(), "option %d at its default fixes the kernels", o.id);
+    other = old == o.lo ? o.hi : o.lo;
+    CHECK(ixh::set_tuning(t, o.id, other, true) == 0, "set option %d", o.id);
+    CHECK(t.fixed() == (o.id != IXH_OPT_PARTS && o.id != IXH_OPT_PASS_TOKENS), "option %d: fixed %d", o.id, t.fixed());
+    CHECK(ixh::set_tuning(t, o.id, old, true) == 0 && !t.fixed(), "option %d set back: still fixed", o.id);
+  }
   int64_t v = 0;
   CHECK(ixh::set_tuning(t, 999, 0, true) == IXH_EINVAL, "unknown option accepted");
   CHECK(ixh::get_tuning(t, 999, &v) == IXH_EINVAL, "unknown option read");

@@ -21,8 +21,10 @@ _models = {}
 
 @contextlib.contextmanager
 def options(gpu, **kw):
-    """Sets model options for a block, then restores them (the models are
-    shared between tests)."""
+    """Sets model options for a block (kernel options at every batch size), then
+    restores them (the models are shared between tests)."""
+    if set(kw) - {"parts", "pass_tokens"}:
+        kw = {"few_rows": 0, **kw}
     old = {k: gpu.option(k) for k in kw}
     try:
         for k, v in kw.items():

@@ -28,8 +28,8 @@ def test_few_rows_exact(shape, lanes, plant):
     row-major), the LayerNorm in the Wi kernel and before it (up to 192 rows,
     shape small 512), the two arrangements of the residual kernel (from 481 rows
     on) and the two sides of the rules that pick these kernels and the
-    32-row MLP kernel; setting a kernel option (here to its default) picks
-    the whole-row kernels, and gives the same bits."""
+    32-row MLP kernel; option few_rows 0 picks the whole-row kernels, and gives
+    the same bits."""
     cfg = SHAPES[shape](layers=2)
     w = Weights.random(cfg, seed=97)
     if plant:
@@ -46,7 +46,7 @@ def test_few_rows_exact(shape, lanes, plant):
     most = {"small": 2048, "base": 3072, "bekko": 4096}[shape]
     edges = [seqs_of(rng, cfg.vocab, *[64] * (n // 64), n % 64) for n in (most, most + 1, 8192, 8193)]
     few = [gpu.encode_tokens(b) for b in batches + edges]
-    gpu.set_option("fuse_mlp", 2)
+    gpu.set_option("few_rows", 0)
     for b, e in zip(batches + edges, few):
         got = gpu.encode_tokens(b)
         assert f32_bits_equal(got, e), ([len(s) for s in b], mismatch_report(got, e))
@@ -136,4 +136,29 @@ def test_shared_qkv_workgroups_exact(shape, lanes, plant):
         seqs = seqs_of(rng, cfg.vocab, *(int(n) for n in rng.integers(129, 257, 200)))
         got, want = gpu.encode_tokens(seqs), ora.encode_tokens(seqs)[0]
         assert f32_bits_equal(got, want), mismatch_report(got, want)
+    gpu.close()
+
+
+def test_options_set_back():
+    """An option read, changed and set back leaves a handle with the kernels of
+    few rows that it had, and so does few_rows."""
+    cfg = small_cfg(layers=2)
+    gpu = Model(Weights.random(cfg, seed=109))
+    seqs = seqs_of(np.random.default_rng(109), cfg.vocab, 24)
+
+    def classes():
+        gpu.set_profiling(True)
+        gpu.encode_seqs(seqs)
+        got = set(gpu.profile())
+        gpu.set_profiling(False)
+        return got
+
+    few = classes()
+    assert "ln_wi" in few
+    for name, other in (("fuse_mlp", 1), ("gemm_tile", 1), ("few_rows", 0)):
+        old = gpu.option(name)
+        gpu.set_option(name, other)
+        assert "ln_wi" not in classes(), name
+        gpu.set_option(name, old)
+        assert classes() == few, name
     gpu.close()
