@@ -2,7 +2,7 @@
 // a CPU build can run it under sanitizers: the kernel options of a handle
 // (Tuning), the checks of a batch's offsets, the planning of encoder passes
 // and stream parts, where a pass's outputs start, the serving batcher's
-// request queue (batch.go:1-82) and the free list of per-call workspaces.
+// request queue (batch.go:1-82) and the lists of idle per-call workspaces.
 #pragma once
 #include <stdint.h>
 
@@ -137,6 +137,47 @@ class FreeList {
  private:
   std::mutex mu_;
   std::vector<T *> items_;
+};
+
+// Idle items kept for the next caller: at most kItems of them, max_bytes
+// together. put() allocates nothing; what it does not keep stays the caller's
+// to destroy.
+template <class T>
+class KeepPool {
+ public:
+  static constexpr int kItems = 4;
+  explicit KeepPool(size_t max_bytes) : max_(max_bytes) {}
+  // the item put last, null when none is idle
+  T *take() {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (n_ == 0) return nullptr;
+    total_ -= bytes_[--n_];
+    return items_[n_];
+  }
+  bool put(T *p, size_t bytes) {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (n_ == kItems || bytes > max_ - total_) return false;
+    items_[n_] = p;
+    bytes_[n_++] = bytes;
+    total_ += bytes;
+    return true;
+  }
+  // every idle item, for their destruction; their number
+  int drain(T **out) {
+    std::lock_guard<std::mutex> lk(mu_);
+    const int n = n_;
+    for (int i = 0; i < n; i++) out[i] = items_[i];
+    n_ = 0;
+    total_ = 0;
+    return n;
+  }
+
+ private:
+  std::mutex mu_;
+  const size_t max_;
+  size_t total_ = 0, bytes_[kItems] = {};
+  T *items_[kItems] = {};
+  int n_ = 0;
 };
 
 // WithBatching / batcher (batch.go:1-82, model.go:136-160): worker threads

@@ -55,7 +55,11 @@ int fail(int code, const char *fmt, ...) {
 
 inline size_t round_up(size_t v, size_t m) { return (v + m - 1) / m * m; }
 
-// Device buffer that grows and never shrinks.
+// Frees the current device's idle linear workspaces; whether there were any.
+bool trim_idle();
+
+// Device buffer that grows and never shrinks. An allocation that fails is
+// tried once more after the idle workspaces are freed.
 struct DevBuf {
   void *p = nullptr;
   size_t n = 0;
@@ -68,7 +72,12 @@ struct DevBuf {
     p = nullptr;
     n = 0;
     size_t want = round_up(std::max<size_t>(bytes, 256), 256);
-    HIPCK(hipMalloc(&p, want));
+    if (hipMalloc(&p, want) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+      (void)trim_idle();
+      HIPCK(hipMalloc(&p, want));
+    }
     n = want;
     return IXH_OK;
   }
@@ -292,8 +301,8 @@ struct ixh_model {
 };
 
 // Stream and device buffers of one linear call (ixh_matmul8,
-// ixh_matmul8_outliers, ixh_linear8), kept with the handle between calls:
-// created per call, a call of 784 x 3,072 rows took 823 us, with them 590.
+// ixh_matmul8_outliers, ixh_linear8), kept between calls: created per call, a
+// call of 784 x 3,072 rows took 823 us, with them 642.
 struct LinWs {
   hipStream_t stream = nullptr;
   DevBuf a, rest, q, sa, c, colmax, cols, w, bias;
@@ -305,15 +314,45 @@ struct LinWs {
   }
 };
 
-struct ixh_packed_b8 {
-  // what a handle keeps: at most kKeep workspaces of at most kKeepBytes each
-  static constexpr int kKeep = 2;
-  static constexpr size_t kKeepBytes = (size_t)256 << 20;
-  FreeList<LinWs> pool;
-  std::atomic<int> kept{0};
-  ~ixh_packed_b8() {
-    for (LinWs *w : pool.drain()) delete w;
+// A device's idle linear workspaces, shared by its PackedB8 handles (a
+// program's layers run one after another): at most 256 MiB together.
+struct LinPool {
+  KeepPool<LinWs> idle{(size_t)256 << 20};
+  bool trim() {
+    LinWs *w[KeepPool<LinWs>::kItems];
+    const int n = idle.drain(w);
+    for (int i = 0; i < n; i++) delete w[i];
+    return n > 0;
   }
+  ~LinPool() { trim(); }
+};
+
+namespace {
+// by device ordinal; a pool lives as long as a handle of its device
+std::mutex g_lin_mu;
+std::weak_ptr<LinPool> g_lin[64];
+
+std::shared_ptr<LinPool> lin_pool(int dev) {
+  std::lock_guard<std::mutex> lk(g_lin_mu);
+  std::shared_ptr<LinPool> p = g_lin[dev].lock();
+  if (!p) g_lin[dev] = p = std::make_shared<LinPool>();
+  return p;
+}
+
+bool trim_idle() {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+  std::shared_ptr<LinPool> p;
+  {
+    std::lock_guard<std::mutex> lk(g_lin_mu);
+    p = g_lin[dev].lock();
+  }
+  return p && p->trim();
+}
+}  // namespace
+
+struct ixh_packed_b8 {
+  std::shared_ptr<LinPool> pool;
   int device = 0;
   Mat mat;
   std::vector<int8_t> rows;  // host copy, for the GeGLU interleave
@@ -1718,7 +1757,8 @@ int ixh_packb8_create(int device, const int8_t *q, const float *scale, int k, in
   int src = scratch_ptr(device, &nd);  // set-up: resolve the device's scratch copy now
   if (src) return src;
   auto *b = new ixh_packed_b8();
-  b->device = device;
+  b->device = device;  // (below 64: scratch_ptr)
+  b->pool = lin_pool(device);
   b->rows = to_rows(q, k, n, layout);
   b->scale.assign(scale, scale + n);
   int rc = upload_mat(b->mat, b->rows, scale, k, n, nullptr);
@@ -1808,16 +1848,13 @@ std::vector<int> choose_outliers(const std::vector<float> &colmax, float ratio) 
   return out;
 }
 
-// A workspace of the handle for one call, its stream idle when it is given
-// back (a call that fails waits for what it queued); null: no stream.
+// A workspace of the handle's device for one call, its stream idle when it is
+// given back (a call that fails waits for what it queued); null: no stream.
 struct LinGuard {
-  ixh_packed_b8 *b;
+  LinPool &pool;
   LinWs *w;
-  explicit LinGuard(ixh_packed_b8 *handle) : b(handle), w(handle->pool.take()) {
-    if (w) {
-      b->kept--;
-      return;
-    }
+  explicit LinGuard(ixh_packed_b8 *handle) : pool(*handle->pool), w(pool.idle.take()) {
+    if (w) return;
     w = new LinWs();
     if (hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking) != hipSuccess) {
       (void)hipGetLastError();
@@ -1828,12 +1865,7 @@ struct LinGuard {
   ~LinGuard() {
     if (!w) return;
     (void)hipStreamSynchronize(w->stream);
-    if (w->bytes() <= ixh_packed_b8::kKeepBytes && b->kept++ < ixh_packed_b8::kKeep) {
-      b->pool.put(w);
-    } else {
-      if (w->bytes() <= ixh_packed_b8::kKeepBytes) b->kept--;
-      delete w;
-    }
+    if (!pool.idle.put(w, w->bytes())) delete w;
   }
 };
 

@@ -16,7 +16,7 @@
 //     pass planning and stream parts over random ragged batches (empty
 //     sequences, pass boundaries, the token cap of wide models), with each
 //     pass's outputs written through Outputs::at into exact-size buffers;
-//     the workspace free list on 8 threads; the serving batcher's queue
+//     the lists of idle workspaces on 8 threads; the serving batcher's queue
 //     driven by 8 client threads with a stub encode (merged batches, errors
 //     handed to every request of a batch, close).
 // Usage: host_check <tokenizer.json> <scratch dir>. Exit status 0 when
@@ -458,6 +458,48 @@ static void check_free_list() {
   CHECK(pool.take() == nullptr, "drained list not empty");
 }
 
+// Items of 1 to 5 bytes in a pool of 8: never more than its bytes or items
+// idle, none handed out twice, none lost.
+static void check_keep_pool() {
+  struct Item {
+    std::atomic<int> held{0};
+  };
+  using Pool = ixh::KeepPool<Item>;
+  Pool pool(8);
+  std::atomic<int> alive{0}, twice{0};
+  std::vector<std::thread> th;
+  for (int w = 0; w < 8; w++)
+    th.emplace_back([&, w]() {
+      std::mt19937 rng(w);
+      for (int i = 0; i < 3000; i++) {
+        if (i % 64 == 0) {
+          Item *all[Pool::kItems];
+          const int n = pool.drain(all);
+          for (int k = 0; k < n; k++) delete all[k], alive--;
+        }
+        Item *a = pool.take();
+        if (!a) a = new Item, alive++;
+        if (a->held.exchange(1)) twice++;
+        a->held.store(0);
+        if (!pool.put(a, 1 + rng() % 5)) delete a, alive--;
+      }
+    });
+  for (auto &x : th) x.join();
+  Item *all[Pool::kItems];
+  int n = pool.drain(all);
+  CHECK(twice.load() == 0, "keep pool handed an item out twice (%d)", twice.load());
+  CHECK(n == alive.load(), "keep pool holds %d of %d items", n, alive.load());
+  for (int k = 0; k < n; k++) delete all[k];
+  CHECK(pool.take() == nullptr, "drained pool not empty");
+  Item it[6];
+  CHECK(!pool.put(&it[0], 9), "an item over the pool's bytes kept");
+  CHECK(pool.put(&it[0], 5) && pool.put(&it[1], 3) && !pool.put(&it[2], 1) && pool.put(&it[3], 0), "pool of 8 bytes");
+  CHECK(pool.take() == &it[3] && pool.take() == &it[1] && pool.put(&it[2], 2), "the item put last, its bytes freed");
+  CHECK(pool.put(&it[4], 0) && pool.put(&it[5], 0) && !pool.put(&it[1], 0), "pool of four items");
+  n = pool.drain(all);
+  CHECK(n == 4 && pool.put(&it[0], 8), "drained pool keeps nothing");
+}
+
 // The batcher's queue with a stub encode: a sequence's row is (length,
 // sum of ids, first id, request tag); a batch with an id of -7 fails.
 static void check_batcher() {
@@ -566,6 +608,7 @@ int main(int argc, char **argv) {
   check_options();
   check_passes();
   check_free_list();
+  check_keep_pool();
   check_batcher();
   if (failures) {
     fprintf(stderr, "host_check: %d checks failed\n", failures);
