@@ -79,3 +79,18 @@ def test_linear_workspaces_bounded():
     for b in layers + [other]:
         b.close()
     assert before - free() <= 32 << 20
+
+
+def test_linear_most_rows():
+    """More row blocks of 16 than a grid's y dimension has (65,535), the last
+    rows holding the massive values that make a channel an outlier."""
+    k, n, rows = 16, 8, 65535 * 16 + 21
+    rng = np.random.default_rng(11)
+    q, s = linalg.pack_b8(rng.standard_normal((n, k), dtype=np.float32))
+    cs = q.astype(np.int32).sum(axis=1).astype(np.int32)
+    x = rng.standard_normal((rows, k), dtype=np.float32)
+    x[-1, 3], x[-20, 7] = 500, -400
+    b = linalg.PackedB8(q, s)
+    got, want = linalg.linear8(x, b, None, True, 6.0), orc.linear8(x, q, s, cs, None, True, 6.0)
+    assert f32_bits_equal(got, want), mismatch_report(got, want)
+    b.close()
