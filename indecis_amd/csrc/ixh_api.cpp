@@ -602,8 +602,8 @@ struct Pending {
   std::vector<std::shared_ptr<DevBuf>> hold;
 };
 
-// The forward pass. ids/out are device pointers here. With `defer` the
-// launches are only issued: the caller synchronises the stream, then calls
+// The forward pass. ids/out are device pointers here. With `defer` the pass
+// is one of several parts and the launches are only issued: the caller synchronises the stream, then calls
 // defer->prof->flush().
 int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w, hipStream_t st,
             const int32_t *d_ids, const int32_t *offs, int B, const Outputs &out,
@@ -671,7 +671,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
                       m->layers[0].qkv.qk.p;
 
   // short sequences: QKV, Attn8.Prepare and attention in one kernel
-  const bool short_seqs = !tune.fixed() && kblock && short_attn_supported(KpH, T, B * nh);
+  const bool short_seqs = !tune.fixed() && kblock && short_attn_picked(KpH, T, B * nh, defer != nullptr);
 
   int rc;
   std::vector<int32_t> groups;

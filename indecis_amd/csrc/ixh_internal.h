@@ -319,11 +319,14 @@ constexpr int kKeyPad = 64;       // key slots of a sequence are padded to this
 constexpr int kQkvSeqMax = 512;
 void launch_qkv_attn(const GemmArgs &g, const AttnArgs &a, const int32_t *order, const int32_t *groups, int ngroups,
                      bool two_blocks, int heads, hipStream_t s);
-// QKV projection, Attn8.Prepare and attention in one kernel (short_attn.hip),
-// for batches of short sequences (see there) and Kp one of 768, 384, 256: g as for launch_qkv_attn with the K-blocked input, a as for
-// launch_attn_main (of the prologue's outputs nothing is written); false
-// (nothing launched) otherwise.
-bool short_attn_supported(int Kp, int max_n, int workgroups);
+// QKV projection, Attn8.Prepare and attention in one kernel (short_attn.hip):
+// sequences of at most 128 tokens, Kp one of 768, 384, 256; g as for
+// launch_qkv_attn with the K-blocked input, a as for launch_attn_main (of the
+// prologue's outputs nothing is written); false (nothing launched) otherwise.
+bool short_attn_supported(int Kp, int max_n);
+// Whether it is the faster one, by the workgroups (a sequence and head each);
+// beside: another part of the batch runs at the same time.
+bool short_attn_picked(int Kp, int max_n, int workgroups, bool beside);
 // The LayerNorm (and quantisation) of the rows before it in the same kernel,
 // when x is not null: sequences of at most 32 tokens, a workgroup a CU.
 struct ShortLn {

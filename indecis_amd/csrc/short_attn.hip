@@ -485,22 +485,43 @@ bool launch_kt(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStrea
 
 }  // namespace
 
-// us a layer of hidden 768, this kernel and the two it replaces: at most 32
-// tokens, one sequence 8.7 and 15.8, 200 sequences 48 and 66: always; at most
-// 64, one 13.0 and 17.2, 40 (two rounds of the CUs, which a workgroup fills)
-// 25 and 36, 200 144 and 71: two rounds; at most 128, one 21.2 and 21.5, 12
-// 21.1 and 25.7, 20 21.7 and 31: one round.
-bool short_attn_supported(int Kp, int max_n, int workgroups) {
-  if (Kp != 768 && Kp != 384 && Kp != 256) return false;
-  return max_n <= 32 || (max_n <= 64 && workgroups <= 2 * device_cus()) || (max_n <= 128 && workgroups <= device_cus());
+// us a layer of the whole pass, on this kernel and on the two it replaces, by
+// rounds of the CUs (a workgroup fills one). At most 32 tokens: hidden 768, 16
+// tokens, 1 sequence 32.7 and 41.1, 64 (3 rounds) 59.7 and 65.2, 106 of 4-32
+// (5) 88.5 and 91.2, 128 (6) 92.0 and 90.2, 512 (24) 230 and 185; 384, 200 (5)
+// 84.7 and 84.3, 512 (12) 133 and 120; 256, 384 (6) 65.8 and 67.8, 512 (8) 77.6
+// and 74.3. At most 64, 64 tokens: 768, 1 42.5 and 45.9, 21 (1) 63.4 and 71.9,
+// 32 (1.5) 80.9 and 78.5, 42 of 33-64 (2) 81.6 and 85.9, 64 (3) 107 and 102;
+// 384, 32 (0.75) 49.4 and 54.2, 85 (2) 80.6 and 81.4, 128 (3) 92.1 and 91.4 (200 121
+// and 111); 256, 64 (1) 41.1 and 46.0, 128 (2) 52.1 and 52.5, 200 80.1 and
+// 72.2. At most 128, 128 tokens: 768, 1 51.7 and 49.4, 8 (0.4) 63.1 and 61.2, 12
+// (0.6) 73.4 and 75.3, 21 (1) 90.6 and 97.2, 32 112 and 102; 384, 1 41.7 and 39.6,
+// 42 of 65-128 (1) 78.5 and 81.9; 256, 1 39.2 and 37.7, 64 (1) 53.4 and 55.8.
+// With another part's kernels beside this pass's (two parts a batch, the figure
+// of a part): at most 32 tokens, 32: 384, 3 rounds 121 and 125, 3.75 117 and 110;
+// 256, 3 81.2 and 88.1, 4 99.4 and 96.4; 64: 384, 1 94.8 and 100, 1.2 104 and 106,
+// 1.5 116 and 114; 256, 1.2 73.1 and 75.3, 1.6 85.3 and 81.8; 128: 768, 0.75 114
+// and 117, 1 145 and 151; 384, 0.4 84.4 and 85.4, 0.6 100 and 108; 256, 0.25 81.8 and
+// 84.5, 1 88.9 and 90.3.
+bool short_attn_picked(int Kp, int max_n, int workgroups, bool beside) {
+  if (!short_attn_supported(Kp, max_n)) return false;
+  const int wg = workgroups, cus = device_cus();
+  if (max_n <= 32) return wg <= (beside ? 3 : Kp == 256 ? 6 : 5) * cus;
+  if (max_n <= 64) {
+    if (beside) return 4 * wg <= 5 * cus;
+    return wg <= cus || (wg <= 2 * cus && (Kp < 768 || 4 * wg > 7 * cus));
+  }
+  return wg <= cus && (beside || 2 * wg > cus);
 }
+
+bool short_attn_supported(int Kp, int max_n) { return (Kp == 768 || Kp == 384 || Kp == 256) && max_n <= 128; }
 
 // a workgroup fills a CU (154 KB of LDS): one round of them
 bool short_attn_ln_supported(int max_n, int workgroups) { return max_n <= 32 && workgroups <= device_cus(); }
 
 bool launch_short_attn(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStream_t s) {
   if (a.B <= 0) return true;
-  if (!short_attn_supported(g.Kp, a.max_n, a.B * a.nh) || !(g.Ak || ln.x)) return false;
+  if (!short_attn_supported(g.Kp, a.max_n) || !(g.Ak || ln.x)) return false;
   if (ln.x && !short_attn_ln_supported(a.max_n, a.B * a.nh)) return false;
   if (g.Kp == 768) return launch_kt<24>(g, a, ln, s);
   if (g.Kp == 384) return launch_kt<12>(g, a, ln, s);

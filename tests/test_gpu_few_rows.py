@@ -60,10 +60,10 @@ def test_short_sequences_exact(shape, lanes, window, plant):
     """QKV, Attn8.Prepare and attention in one kernel (short_attn.hip): the
     longest sequence at the edges of its 1, 2 and 4 row blocks, with a local
     window that cuts sequences and one that does not, empty sequences, QKV
-    rows past the dequantisation bound, and batches one workgroup either side
-    of the rules that pick it (two rounds of the 256 CUs up to 64 tokens, one
-    up to 128) and with the LayerNorm before it in the same kernel (at most 32
-    tokens, 24 rows at a time, one round), against the oracle."""
+    rows past the dequantisation bound, and with the LayerNorm before it in the
+    same kernel (at most 32 tokens, 24 rows at a time, one round of the 256
+    CUs), against the oracle; and batches one workgroup either side of the rules
+    that pick it, by the kernels that ran."""
     cfg = SHAPES[shape](layers=2, local_attention=window)
     w = Weights.random(cfg, seed=101)
     if plant:
@@ -73,13 +73,45 @@ def test_short_sequences_exact(shape, lanes, window, plant):
     rng = np.random.default_rng(101)
     batches = [(1,), (15, 2), (31, 0, 1), (32, 32, 17), (33, 5), (40, 0, 63, 1), (64, 33), (65, 31), (97, 8), (127,),
                (128, 1, 90), (129, 3)]
-    two, one = 512 // cfg.heads, 256 // cfg.heads
+    one = 256 // cfg.heads
     batches += [(24,), (25, 24, 3), (30,) + (2,) * (one - 1), (30,) + (2,) * one]
-    batches += [(33,) + (2,) * (two - 1), (33,) + (2,) * two, (65,) + (2,) * (one - 1), (65,) + (2,) * one]
-    for lens in batches:
+    picked = [None] * len(batches)
+    # longest sequence, most (or, negative, one less than the fewest) sixteenths of a round
+    edges = [(32, 96 if shape == "small" else 80), (64, 32), (65, -8), (128, 16)]
+    edges += [(33, 16), (64, -28)] if shape == "base" else []
+    for n, most in edges:
+        seqs = abs(most) * 16 // cfg.heads
+        batches += [(n,) + (2,) * (seqs - 1), (n,) + (2,) * seqs]
+        picked += [most > 0, most < 0]
+    gpu.set_profiling(True)
+    for lens, short in zip(batches, picked):
         seqs = seqs_of(rng, cfg.vocab, *lens)
         got, want = gpu.encode_tokens(seqs), ora.encode_tokens(seqs)[0]
         assert f32_bits_equal(got, want), (lens[:4], mismatch_report(got, want))
+        ran = set(gpu.profile())
+        gpu.set_profiling(True)  # clears the sums
+        if short is not None:
+            assert ("gemm_qkv" not in ran) == short, (lens[0], len(lens))
+    gpu.close()
+
+
+def test_short_sequences_in_parts():
+    """A batch run as two parts: short_attn.hip up to three rounds a part of at
+    most 32 tokens, with the same bits as the other kernels."""
+    cfg = small_cfg(layers=2)
+    gpu = Model(Weights.random(cfg, seed=102))
+    rng = np.random.default_rng(102)
+    gpu.set_option("parts", 2)
+    for seqs, short in ((384, True), (386, False)):
+        batch = seqs_of(rng, cfg.vocab, *[32] * seqs)
+        gpu.set_profiling(True)
+        got = gpu.encode_tokens(batch)
+        assert ("gemm_qkv" not in gpu.profile()) == short, seqs
+        gpu.set_profiling(False)
+        gpu.set_option("few_rows", 0)
+        want = gpu.encode_tokens(batch)
+        gpu.set_option("few_rows", 1)
+        assert f32_bits_equal(got, want), (seqs, mismatch_report(got, want))
     gpu.close()
 
 
