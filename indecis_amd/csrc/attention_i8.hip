@@ -872,15 +872,19 @@ void launch_attn_main(const AttnArgs &a, hipStream_t s) {
   // 8 runs of (nblocks * nh + 7) / 8 items, one an XCD (see the kernel)
   const int items = a.nblocks * a.nh, cus = device_cus();
   const dim3 grid(8 * ((items + 7) / 8));
-  // Waves that share a query block's keys. us a launch with 1, 2 and 4,
-  // global: 24 workgroups of 256 keys 12.8, 10.8, 11.6; 192 of 2,048 66, 48.5,
-  // 44.9; of 4,096 134, 95, 86; 384 of 4,096 152, 126, 159; 768 of 8,192 401,
-  // 374, 441. Local: 24 10.7, 10.0, 11.2; 192 11.6, 10.6, 11.5; 384 13.9, 18.0,
-  // 20.4. With one, a grid of less than three workgroups a CU leaves SIMDs with
-  // one wave, or with none.
+  // Waves that share a query block's keys: 2 up to two workgroups a CU (up to
+  // one in local layers), 4 up to one over more than 512 keys. us a layer of the
+  // whole pass with 1, 2 and 4. Global, hidden 768: 96 workgroups of 512 keys 82.4,
+  // 78.9, 79.1; 192 of 2,048 169, 153, 149; 384 of 256 105.7, 105.2, 110.5, of
+  // 4,096 280, 259, 292; 504 of 384 122.3, 120.8, 129; 612 139, 144, 155; 576 of
+  // 6,144 432, 439, 493; 768 of 8,192 603, 605, 680; hidden 256: 248 of 256 59.4,
+  // 57.7, 58.0; 512 of 1,024 147, 141, 152, of 8,192 501, 450, 508; 768 648, 654,
+  // 733. Local: 96 of 512 75.0, 72.9; 240 of 256 91.7, 89.7; 288 104, 108. With
+  // one, a grid of less than three workgroups a CU leaves SIMDs with one wave, or
+  // with none; from two on their shared work costs more than that.
   if (a.window < 0) {
     if (items <= cus && a.max_n > 512) attn_main_kernel<true, 4><<<grid, 1024, 0, s>>>(a);
-    else if (items <= 3 * cus) attn_main_kernel<true, 2><<<grid, 512, 0, s>>>(a);
+    else if (items <= 2 * cus) attn_main_kernel<true, 2><<<grid, 512, 0, s>>>(a);
     else attn_main_kernel<true, 1><<<grid, 256, 0, s>>>(a);
   } else {
     if (items <= cus) attn_main_kernel<false, 2><<<grid, 512, 0, s>>>(a);

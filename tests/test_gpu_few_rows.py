@@ -120,7 +120,7 @@ def test_shared_keys_exact(shape, window):
     """Attention with 1, 2 and 4 waves on a query block's keys
     (attention_i8.hip), by the number of query blocks and the longest
     sequence: one sequence around the chunks of 256 keys and past 512 keys,
-    and batches either side of 256 and of 768 workgroups, against the oracle
+    and batches either side of 256 and of 512 workgroups, against the oracle
     (the largest against one-sequence calls)."""
     cfg = SHAPES[shape](layers=2, local_attention=window)
     w = Weights.random(cfg, seed=103)
@@ -131,7 +131,7 @@ def test_shared_keys_exact(shape, window):
         got, want = gpu.encode_tokens(seqs), ora.encode_tokens(seqs)[0]
         assert f32_bits_equal(got, want), (lens, mismatch_report(got, want))
     gpu.set_option("parts", 1)
-    for items in (256, 768):
+    for items in (256, 512):
         for blocks in (items // cfg.heads, items // cfg.heads + 1):
             seqs = seqs_of(rng, cfg.vocab, *[150, 129] * (blocks // 4), *[140] * ((blocks % 4) // 2), *[9] * (blocks % 2))
             got = gpu.encode_seqs(seqs)
