@@ -246,12 +246,8 @@ void launch_kt(const GemmArgs &a, hipStream_t s) {
   int G = std::min(units, 2 * device_cus());
   G = std::max(NXCD, G / NXCD * NXCD);
   const size_t shm = (size_t)BM * 32 * KT;
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute((const void *)gemm_as_kernel<MB, KT, EPI>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    attr = true;
-  }
+  static PerDevice lds;
+  (void)lds_granted(lds, (const void *)gemm_as_kernel<MB, KT, EPI>, (int)shm);
   gemm_as_kernel<MB, KT, EPI><<<G, 256, shm, s>>>(a, units, nchunk);
 }
 

@@ -333,13 +333,9 @@ void launch_cfg(int epi, const GemmArgs &a, hipStream_t s) {
   const size_t shm = C::SMEM;
   // up to 72 KB of LDS per workgroup (gfx950 has 160 KB per CU): allow more
   // than the default 64 KB of dynamic LDS, once per kernel instance
-  static bool attr_set[8] = {};
+  static PerDevice lds[8];
   auto launch = [&](auto kern) {
-    if (!attr_set[epi]) {
-      (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)shm);
-      attr_set[epi] = true;
-    }
+    (void)lds_granted(lds[epi], (const void *)kern, (int)shm);
     kern<<<grid, block, shm, s>>>(a);
   };
   switch (epi) {

@@ -426,12 +426,8 @@ __global__ __launch_bounds__(256, 2) void gemm_res_kernel(ResArgs a) {
 template <int KT, int NB, int V, bool LN, bool STREAM>
 void launch_one(const ResArgs &a, hipStream_t s) {
   const size_t shm = smem_bytes(KT, NB, STREAM);
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute((const void *)gemm_res_kernel<KT, NB, V, LN, STREAM>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    attr = true;
-  }
+  static PerDevice lds;
+  (void)lds_granted(lds, (const void *)gemm_res_kernel<KT, NB, V, LN, STREAM>, (int)shm);
   gemm_res_kernel<KT, NB, V, LN, STREAM><<<(a.M + BM - 1) / BM, 256, shm, s>>>(a);
 }
 

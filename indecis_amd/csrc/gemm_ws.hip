@@ -271,12 +271,8 @@ void launch_kt(const GemmArgs &a, hipStream_t s) {
   int G = std::min(units, device_cus());
   G = std::max(NXCD, G / NXCD * NXCD);
   const size_t shm = (size_t)BM * 32 * KT + HAND_BYTES;
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute((const void *)gemm_ws_kernel<KT, EPI>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    attr = true;
-  }
+  static PerDevice lds;
+  (void)lds_granted(lds, (const void *)gemm_ws_kernel<KT, EPI>, (int)shm);
   gemm_ws_kernel<KT, EPI><<<G, 512, shm, s>>>(a, units, nchunk);
 }
 

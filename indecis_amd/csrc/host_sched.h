@@ -6,6 +6,7 @@
 #pragma once
 #include <stdint.h>
 
+#include <atomic>
 #include <condition_variable>
 #include <deque>
 #include <functional>
@@ -178,6 +179,24 @@ class KeepPool {
   size_t total_ = 0, bytes_[kItems] = {};
   T *items_[kItems] = {};
   int n_ = 0;
+};
+
+// A yes or no of each device: asked of the current device until it has
+// answered once (by several threads at a time, maybe), then kept. A device past
+// kDevices is asked every time.
+class PerDevice {
+ public:
+  static constexpr int kDevices = 64;
+  template <class Ask>
+  bool get(int dev, Ask ask) {
+    if (dev < 0 || dev >= kDevices) return ask();
+    int v = state_[dev].load();
+    if (v == 0) state_[dev] = v = ask() ? 1 : -1;
+    return v > 0;
+  }
+
+ private:
+  std::atomic<int> state_[kDevices] = {};
 };
 
 // WithBatching / batcher (batch.go:1-82, model.go:136-160): worker threads

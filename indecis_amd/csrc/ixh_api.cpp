@@ -1368,6 +1368,15 @@ int device_cus() {
   }
   return n;
 }
+bool lds_granted(PerDevice &answers, const void *kern, int bytes) {
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess) dev = -1;
+  return answers.get(dev, [&] {
+    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  });
+}
 void model_config(const ixh_model *m, ixh_config *out) { *out = m->cfg; }
 }  // namespace ixh
 

@@ -17,6 +17,9 @@ namespace ixh {
 // Compute units of the current device (cached per device; 256 if the query
 // fails), for grids of resident workgroups.
 int device_cus();
+// Whether the current device grants the kernel `bytes` of dynamic LDS (past
+// 64 KB it has to be asked), from the kernel's own record of the answers.
+bool lds_granted(PerDevice &answers, const void *kern, int bytes);
 
 // ---- int8 GEMM ----------------------------------------------------------
 // C = epilogue(A . B^T): A int8 [M][lda] (signed activations, zero

@@ -648,12 +648,8 @@ __global__ __launch_bounds__(512, 1) void mlp_block_kernel(MlpArgs a) {
 template <int H, int I, int V, bool LN>
 void launch_one(const MlpArgs &a, hipStream_t s) {
   constexpr size_t shm = Shape<H, I>::SMEM;
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute((const void *)mlp_block_kernel<H, I, V, LN>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    attr = true;
-  }
+  static PerDevice lds;
+  (void)lds_granted(lds, (const void *)mlp_block_kernel<H, I, V, LN>, (int)shm);
   mlp_block_kernel<H, I, V, LN><<<(a.M + BM - 1) / BM, 512, shm, s>>>(a);
 }
 

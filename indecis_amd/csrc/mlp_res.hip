@@ -499,12 +499,8 @@ __global__ __launch_bounds__(512, 1) void mlp_res_kernel(MlpArgs a) {
 template <int H, int I, int V, bool LN, bool WO>
 void launch_one(const MlpArgs &a, hipStream_t s) {
   constexpr size_t shm = Shape<H, I>::SMEM;
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute((const void *)mlp_res_kernel<H, I, V, LN, WO>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    attr = true;
-  }
+  static PerDevice lds;
+  (void)lds_granted(lds, (const void *)mlp_res_kernel<H, I, V, LN, WO>, (int)shm);
   mlp_res_kernel<H, I, V, LN, WO><<<(a.M + BM - 1) / BM, 512, shm, s>>>(a);
 }
 

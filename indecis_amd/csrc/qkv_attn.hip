@@ -596,17 +596,11 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
 
 namespace {
 
-// hipFuncSetAttribute once per variant: 1 set, -1 refused (that variant is
-// then not used), 0 not tried yet.
+// Whether the device grants the variant its LDS (refused: it is not used).
 template <int NH, bool KB, int BLK>
 bool smem_ready() {
-  static int state = 0;
-  if (state == 0)
-    state = hipFuncSetAttribute((const void *)qkv_attn_kernel<NH, KB, BLK>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                Shape<NH>::SMEM) == hipSuccess
-                ? 1
-                : -1;
-  return state > 0;
+  static PerDevice lds;
+  return lds_granted(lds, (const void *)qkv_attn_kernel<NH, KB, BLK>, Shape<NH>::SMEM);
 }
 
 template <int NH, bool KB, int BLK>

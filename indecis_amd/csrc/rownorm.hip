@@ -1003,13 +1003,8 @@ void launch_pool(const float *xn, const int32_t *offs, int B, int N, int H, int 
     return;
   }
   constexpr int shm = PL_S * PL_STAGE;  // 128 KB
-  static bool attr[64] = {};
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  if (!attr[dev & 63]) {
-    (void)hipFuncSetAttribute((const void *)pool_ring_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-    attr[dev & 63] = true;
-  }
+  static PerDevice lds;
+  (void)lds_granted(lds, (const void *)pool_ring_kernel, shm);
   pool_ring_kernel<<<dim3((H + 63) / 64, B), 256, shm, s>>>(xn, offs, H, cls, out);
 }
 

@@ -22,7 +22,6 @@
 // later step has what it reduces over in a lane's registers. The scores of a
 // query block are dealt to NG waves by accumulator groups, each wave
 // computing the block's S^T tiles itself.
-#include <atomic>
 #include <type_traits>
 
 #include "ixh_device.h"
@@ -459,12 +458,9 @@ __global__ __launch_bounds__(768) void short_attn_kernel(GemmArgs g, AttnArgs a,
 template <int KT, int RT, int LNV>
 bool launch_one(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStream_t s) {
   constexpr int shm = LNV < 0 ? Shape<RT>::SMEM : LnShape<KT>::SMEM;
-  // the device's grant of that much LDS: 1 granted, -1 refused, 0 not asked yet
-  static std::atomic<int> state{0};
+  static PerDevice lds;
   const auto kern = short_attn_kernel<KT, RT, LNV>;
-  if (state.load() == 0)
-    state = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, shm) == hipSuccess ? 1 : -1;
-  if (state.load() < 0) return false;
+  if (!lds_granted(lds, (const void *)kern, shm)) return false;
   kern<<<NXCD * ((a.B * a.nh + NXCD - 1) / NXCD), 768, shm, s>>>(g, a, ln);
   return true;
 }

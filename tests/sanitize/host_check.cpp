@@ -16,7 +16,7 @@
 //     pass planning and stream parts over random ragged batches (empty
 //     sequences, pass boundaries, the token cap of wide models), with each
 //     pass's outputs written through Outputs::at into exact-size buffers;
-//     the lists of idle workspaces on 8 threads; the serving batcher's queue
+//     the lists of idle workspaces and the answers by device on 8 threads; the serving batcher's queue
 //     driven by 8 client threads with a stub encode (merged batches, errors
 //     handed to every request of a batch, close).
 // Usage: host_check <tokenizer.json> <scratch dir>. Exit status 0 when
@@ -500,6 +500,28 @@ static void check_keep_pool() {
   CHECK(n == 4 && pool.put(&it[0], 8), "drained pool keeps nothing");
 }
 
+// Each device gives its own answer, kept once it is there.
+static void check_per_device() {
+  ixh::PerDevice d;
+  std::atomic<int> asked[3] = {};
+  auto ask = [&](int dev) { return d.get(dev, [&, dev] { asked[dev % 3]++; return dev % 2 == 0; }); };
+  for (int round = 0; round < 3; round++)
+    for (int dev : {0, 1, 2}) CHECK(ask(dev) == (dev % 2 == 0), "device %d: another device's answer", dev);
+  for (int dev : {0, 1, 2}) CHECK(asked[dev] == 1, "device %d asked %d times", dev, asked[dev].load());
+  for (int dev : {-1, ixh::PerDevice::kDevices})
+    for (int round = 0; round < 2; round++)
+      CHECK(d.get(dev, [&] { return round == 1; }) == (round == 1), "device %d: an answer kept", dev);
+  std::atomic<int> wrong{0};
+  std::vector<std::thread> th;
+  for (int w = 0; w < 8; w++)
+    th.emplace_back([&, w] {
+      for (int dev = 3; dev < ixh::PerDevice::kDevices; dev++)
+        if (ask(dev) != (dev % 2 == 0)) wrong++;
+    });
+  for (auto &x : th) x.join();
+  CHECK(wrong.load() == 0, "%d wrong answers on 8 threads", wrong.load());
+}
+
 // The batcher's queue with a stub encode: a sequence's row is (length,
 // sum of ids, first id, request tag); a batch with an id of -7 fails.
 static void check_batcher() {
@@ -609,6 +631,7 @@ int main(int argc, char **argv) {
   check_passes();
   check_free_list();
   check_keep_pool();
+  check_per_device();
   check_batcher();
   if (failures) {
     fprintf(stderr, "host_check: %d checks failed\n", failures);
