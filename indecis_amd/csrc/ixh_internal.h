@@ -341,7 +341,9 @@ struct ShortLn {
 bool short_attn_ln_supported(int max_n, int workgroups);
 bool launch_short_attn(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStream_t s);
 // The fused QKV kernel's K-blocked input ([Kp/32][rows][32]): supported
-// for Kp a multiple of 128 whose weight rows fit in its LDS.
+// for Kp a multiple of 128 from kQkvKblockMin on whose weight rows fit in its
+// LDS.
+constexpr int kQkvKblockMin = 256;
 bool qkv_kblock_supported(int Kp);
 
 }  // namespace ixh

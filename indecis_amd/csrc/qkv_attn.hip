@@ -227,7 +227,9 @@ __global__ __launch_bounds__(512 * NH, 4) void qkv_attn_kernel(GemmArgs g, AttnA
     // stored), a K-block further on every ak_rows rows: the lane's byte
     // offsets in the VGPRs, the K-block's in an SGPR (no address
     // arithmetic a load)
-    constexpr int PF = BLK == 2 ? 4 : 8;  // K-blocks in flight (nkb is a multiple of 4)
+    // K-blocks in flight, all of them in the first round; nkb is a multiple of 4
+    constexpr int PF = BLK == 2 ? 4 : 8;
+    static_assert(32 * PF <= kQkvKblockMin, "the first round's K-blocks");
     const auto ars = buf_rsrc(g.Ak, (uint32_t)nkb * g.ak_rows * 32);
     uint32_t avo[BLK];
 #pragma unroll
@@ -611,7 +613,7 @@ void launch_nh(const GemmArgs &g, const AttnArgs &a, const int32_t *work, int nw
 
 }  // namespace
 
-bool qkv_kblock_supported(int Kp) { return Kp % 128 == 0 && Kp * 64 <= Shape<1>::SMEM; }
+bool qkv_kblock_supported(int Kp) { return Kp >= kQkvKblockMin && Kp % 128 == 0 && Kp * 64 <= Shape<1>::SMEM; }
 
 // One head a workgroup; two (1,024 threads) on request when the
 // head count is even and the device grants the LDS. Two heads halve the
