@@ -16,6 +16,7 @@
 //     pass planning and stream parts over random ragged batches (empty
 //     sequences, pass boundaries, the token cap of wide models), with each
 //     pass's outputs written through Outputs::at into exact-size buffers;
+//     the fused QKV kernel's groups over random lengths, empties and orders;
 //     the lists of idle workspaces and the answers by device on 8 threads; the serving batcher's queue
 //     driven by 8 client threads with a stub encode (merged batches, errors
 //     handed to every request of a batch, close).
@@ -424,6 +425,57 @@ static void check_passes() {
   }
 }
 
+// qkv_groups over random batches: every row block of every sequence (padded to
+// 64 rows, two of an empty one) in exactly one slot, a sequence's blocks in
+// consecutive slots of one group, slots taken in order, the groups' list of
+// sequences the one the slots hold; unshared, one sequence a group.
+static void check_groups() {
+  std::mt19937 rng(17);
+  for (int round = 0; round < 400; round++) {
+    const bool share = round & 1;
+    const int slots = round & 2 ? 16 : 8, top = slots == 8 ? 256 : 512;
+    const int B = 1 + (int)(rng() % (round < 40 ? 3 : 70));
+    std::vector<int32_t> offs(B + 1, 0), padoff(B + 1, 0), order(B);
+    for (int b = 0; b < B; b++) {
+      const int kind = (int)(rng() % 8);
+      const int n = kind == 0 ? 0 : kind == 1 ? top : kind == 2 ? 64 * (int)(rng() % (top / 64 + 1)) : (int)(rng() % (top + 1));
+      offs[b + 1] = offs[b] + n;
+      padoff[b + 1] = padoff[b] + (n + 63) / 64 * 64;
+      order[b] = b;
+    }
+    // longest first, as the pass orders them; every fourth batch in any order
+    if (round % 4 < 3)
+      std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return offs[x + 1] - offs[x] > offs[y + 1] - offs[y]; });
+    else
+      std::shuffle(order.begin(), order.end(), rng);
+    std::vector<int32_t> g(5, 99);
+    ixh::qkv_groups(offs.data(), padoff.data(), order, slots, share, g);
+    CHECK(g.size() % ixh::kQkvGroup == 0, "groups: %zu integers", g.size());
+    std::vector<int> seen(B, 0);
+    for (size_t i = 0; i < g.size() / ixh::kQkvGroup; i++) {
+      const int32_t *e = &g[i * ixh::kQkvGroup];
+      int used = 0, seqs = 0;
+      while (used < 16 && e[4 * used] >= 0) {
+        const int b = e[4 * used] / 16, n = b < B ? offs[b + 1] - offs[b] : 0, nb = std::max(2, (n + 63) / 64 * 2);
+        CHECK(b < B && used + nb <= slots, "group %zu slot %d: sequence %d of %d blocks", i, used, b, nb);
+        if (b >= B || used + nb > 16) return;
+        for (int k = 0; k < nb; k++) {
+          const int32_t *s = e + 4 * (used + k);
+          CHECK(s[0] == 16 * b + k && s[1] == offs[b] && s[2] == n && s[3] == padoff[b], "group %zu slot %d", i, used + k);
+        }
+        CHECK(seqs < 8 && e[64 + seqs] == 16 * n + used, "group %zu: sequence %d of it", i, seqs);
+        seen[b]++;
+        seqs++;
+        used += nb;
+      }
+      for (int s = used; s < 16; s++) CHECK(e[4 * s] == -1, "group %zu: slot %d after a free one", i, s);
+      for (int s = seqs; s < 8; s++) CHECK(e[64 + s] == -1, "group %zu: a sequence without slots", i);
+      CHECK(seqs >= 1 && (share || seqs == 1), "group %zu holds %d sequences", i, seqs);
+    }
+    for (int b = 0; b < B; b++) CHECK(seen[b] == 1, "sequence %d in %d groups", b, seen[b]);
+  }
+}
+
 static void check_free_list() {
   struct Item {
     std::atomic<int> held{0};
@@ -629,6 +681,7 @@ int main(int argc, char **argv) {
   check_normalize();
   check_options();
   check_passes();
+  check_groups();
   check_free_list();
   check_keep_pool();
   check_per_device();

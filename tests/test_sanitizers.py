@@ -1,8 +1,8 @@
 """The library's host-only C++ (tokenizer.cpp with its worker threads,
 safetensors.cpp fed truncated and corrupted files, embed.cpp, and
-host_sched.cpp: options, pass planning, the idle workspaces' lists and the
-serving batcher's queue under concurrent clients) built with
-g++ under AddressSanitizer + UndefinedBehaviorSanitizer and under
+host_sched.cpp: options, pass planning, the fused QKV kernel's groups, the
+idle workspaces' lists and the serving batcher's queue under concurrent
+clients) built with g++ under AddressSanitizer + UndefinedBehaviorSanitizer and under
 ThreadSanitizer, and run on the CPU by tests/sanitize/host_check.cpp (no
 GPU: the model entry points those files call are stubbed there)."""
 import os
