@@ -675,7 +675,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
 
   int rc;
   std::vector<int32_t> groups;
-  // its workgroups: sequences share them once one a sequence, head and part
+  // the fused QKV kernel's workgroups: sequences share them once one a sequence, head and part
   // would not all be resident (two a CU); of 8 row blocks where no sequence has
   // more, up to four rounds of that, else of 16. us a launch with 8 and 16
   // blocks, sequences of 200 tokens, hidden 768 (384): 4 sequences 13.4 and
@@ -683,7 +683,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   // 164 125 and 119.
   const int cus = device_cus();
   bool two_blocks = T > 256;
-  if (kblock) {
+  if (kblock && !short_seqs) {
     const bool share = 3 * nh * B > 2 * cus;
     qkv_groups(offs, padoff.data(), order, two_blocks ? 16 : 8, share, groups);
     if (!two_blocks && 3 * nh * (int64_t)(groups.size() / kQkvGroup) > 8 * cus) {
