@@ -594,6 +594,11 @@ constexpr int kMlp32RowsMax = 8192;
 // it at every size: 4.6 and 8.2 at 24 rows, 34 and 39 at 32,768, 72 and 78 at
 // 73,728 (hidden 384, 65,536 rows: 33 and 43).
 constexpr int kFewRowsMax = 8192;
+// But at hidden 768 with 4 lanes, whose chains hold 192 values a thread: on it
+// and on the row kernel of those lanes, 10.2 and 12.7 at 4,000 rows, 18.0 and
+// 15.3 at 8,000, 60 and 44 at 30,000, 143 and 86 at 76,800 (hidden 384: 46 and
+// 226, 256: 32 and 32).
+constexpr int kFewRowsMax4Lanes = 5888;
 
 // What a forward pass issued but has not waited for: its profiling records
 // and the RoPE tables its kernels read.
@@ -1101,7 +1106,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
     r.eps = c.norm_eps;
     r.lanes = c.lanes;
     r.seg = tune.ln_seg;
-    r.few = !tune.fixed();
+    r.few = !tune.fixed() && !(H == 768 && c.lanes == 4 && N > kFewRowsMax4Lanes);
     r.out = xn;
     RUN("final_norm", 0, dN * 8 * dH, launch_rownorm(r, st));
   }

@@ -171,6 +171,21 @@ def test_shared_qkv_workgroups_exact(shape, lanes, plant):
     gpu.close()
 
 
+@pytest.mark.parametrize("rows", [5888, 5889])
+def test_final_norm_four_lanes(rows):
+    """The final LayerNorm of 4 lanes at hidden 768 either side of the row count
+    at which its kernel changes, against the options' kernels."""
+    cfg = base_cfg(layers=1)
+    gpu = Model(Weights.random(cfg, seed=111), lanes=4)
+    gpu.set_option("parts", 1)
+    seqs = seqs_of(np.random.default_rng(111), cfg.vocab, *[128] * (rows // 128), rows % 128)
+    got = gpu.encode_tokens(seqs)
+    gpu.set_option("few_rows", 0)
+    want = gpu.encode_tokens(seqs)
+    assert f32_bits_equal(got, want), mismatch_report(got, want)
+    gpu.close()
+
+
 def test_options_set_back():
     """An option read, changed and set back leaves a handle with the kernels of
     few rows that it had, and so does few_rows."""
