@@ -147,6 +147,38 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
   }
 }
 
+// Alone, the tiles' workgroups read the rows too many times over past some
+// rows. Sequences of 128 tokens, a pass with the 64-row MLP kernel (the 32-row
+// one at hidden 768 and 256) over one on these: hidden 768 1.75 (1.49) at 1,024
+// rows, 1.40 (1.20) at 2,048, 1.17 (1.00) at 3,072, 1.10 (0.94) at 4,096; 384
+// 1.37 at 2,048, 1.08 at 4,096, 0.91 at 6,144; 256 1.20 (1.06) at 2,048, 1.10
+// (0.98) at 2,560. Beside another part, whose workgroups fill those CUs too, it
+// loses from the smallest batch that is split (4,096 rows) on, but at 384 in two
+// or three parts: us a pass of 8 layers (6 at 256) in two parts of sequences of
+// 512, on these, with the 32- and with the 64-row kernel: 768 1,147, 1,059 and
+// 1,196 at 4,096 rows, 1,389, 1,110 and 1,237 at 6,144; 256 606, 548 and 585 at
+// 4,096; 384 883 and (64) 916 at 4,096, 904 and 921 at 4,608, 931 and 924 at
+// 5,120, 1,085 and 938 at 8,192 (three parts 1,058 and 1,066 at 4,608, four
+// 1,217 and 1,198).
+bool split_rows_picked(int H, int N, int batch) {
+  if (batch > N) return H == 384 && batch <= 4608 && 3 * (int64_t)N >= batch;
+  return N <= (H == 768 ? 3072 : H == 384 ? 4096 : 2048);
+}
+
+// Alone, up to one round of the 256 CUs, where 64 rows a workgroup leave half of
+// them idle. Hidden 768: 2.51 against 2.89 ms a pass at 6,144 rows, 2.90 against
+// 3.18 at 8,192 (38 against 52 us a launch); past one round a 32-row block costs
+// as much as a 64-row one. 256: a launch 12.9 against 19.1 us at 2,560 rows, 13.5
+// and 19.3 at 4,096, 15.0 and 19.7 at 8,192. Beside another part the CUs are
+// shared: us a pass in two parts as above with the 32- and the 64-row kernel,
+// sequences of 160 and of 512, 768 1,381 and 1,401, 1,474 and 1,469 at 10,240
+// rows, 1,581 and 1,542, 1,594 and 1,581 at 12,288, 1,977 and 1,887, 1,865 and
+// 1,744 at 16,384; 256 631 and 656, 638 and 661 at 14,336, 671 and 683, 662 and
+// 678 (1,024: 939 and 915) at 16,384.
+bool mlp32_picked(int H, int N, int batch) {
+  return N <= 8192 && (batch <= N || batch <= (H == 768 ? 10240 : 14336));
+}
+
 // Rows do not depend on their batch (TestMatMul8RowsIndependent), so the
 // results of several passes are those of one.
 int plan_passes(const Tuning &t, int H, int I, const int32_t *offs, int B, std::vector<int> &cut) {

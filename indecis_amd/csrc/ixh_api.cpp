@@ -572,21 +572,6 @@ int split_parts(const Tuning &t, int N, int B, int H) {
   return 2;
 }
 
-// Most rows of a pass whose Wo and MLP run cut by output channel
-// (split_rows.hip), by hidden size. Past it the tiles' workgroups read the
-// rows too many times over. Sequences of 128 tokens, a pass with the 64-row
-// MLP kernel (the 32-row one at hidden 768 and 256) over one on these: hidden
-// 768 1.75 (1.49) at 1,024 rows, 1.40 (1.20) at 2,048, 1.17 (1.00) at 3,072,
-// 1.10 (0.94) at 4,096; 384 1.37 at 2,048, 1.08 at 4,096, 0.91 at 6,144; 256
-// 1.20 (1.06) at 2,048, 1.10 (0.98) at 2,560.
-int split_rows_max(int H) { return H == 768 ? 3072 : H == 384 ? 4096 : 2048; }
-// Above that, most rows of a pass whose MLP runs 32 rows a workgroup
-// (mlp_res.hip): one round of the 256 CUs, where 64 rows a workgroup leave
-// half of them idle. Hidden 768: 2.51 against 2.89 ms a pass at 6,144 rows,
-// 2.90 against 3.18 at 8,192 (38 against 52 us a launch); past one round a
-// 32-row block costs as much as a 64-row one.
-constexpr int kMlp32RowsMax = 8192;
-
 // Most rows of a pass whose embedding LayerNorm runs with 32 threads a row
 // (ln_rows_kernel, rownorm.hip): us a launch on it and on the segment kernel,
 // hidden 768, 6.7 and 14.3 at 24 rows, 9.8 and 16.6 at 4,096, 25.1 and 24.2 at
@@ -607,11 +592,12 @@ struct Pending {
   std::vector<std::shared_ptr<DevBuf>> hold;
 };
 
-// The forward pass. ids/out are device pointers here. With `defer` the pass
-// is one of several parts and the launches are only issued: the caller synchronises the stream, then calls
+// The forward pass. ids/out are device pointers here. batch: the rows of all
+// the parts that run at once, this one's among them. With `defer` the launches
+// are only issued: the caller synchronises the stream, then calls
 // defer->prof->flush().
 int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w, hipStream_t st,
-            const int32_t *d_ids, const int32_t *offs, int B, const Outputs &out,
+            const int32_t *d_ids, const int32_t *offs, int B, const Outputs &out, int batch,
             Pending *defer = nullptr) {
   // an error left by a call outside this pass (the caller's, or one this
   // library already reported) is not this pass's launch failure
@@ -660,14 +646,14 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   const bool mlp_common = m->layers[0].i.qk.p && m->layers[0].omlp.qk.p && gelu_fma_cols(I, c.lanes) == I;
   bool mats_small = true;  // the 64-row kernel dequantises as f32(acc) * sb * sa
   for (int l = 0; l < c.layers; l++) mats_small = mats_small && m->layers[l].i.small && m->layers[l].omlp.small;
-  const bool mlp32 = !tune.fixed() && N <= kMlp32RowsMax && mlp_common && fuse_res &&
+  const bool mlp32 = !tune.fixed() && mlp32_picked(H, N, batch) && mlp_common && fuse_res &&
                      mlp_res_supported(H, I, KpH, KpI, m->layers[0].i.np);
   const bool mlp_block = !mlp32 && mlp_common && tune.fuse_mlp == 2 && mats_small &&
                          mlp_block_supported(H, I, KpH, KpI, m->layers[0].i.np);
   const bool fuse_mlp = mlp_block || (mlp_common && fuse_res && tune.fuse_mlp != 0 &&
                                       mlp_res_supported(H, I, KpH, KpI, m->layers[0].i.np));
   // few rows: Wo and the MLP cut by output channel (split_rows.hip)
-  const bool split = !tune.fixed() && N <= split_rows_max(H) && split_rows_supported(H, I, KpH, KpI) &&
+  const bool split = !tune.fixed() && split_rows_picked(H, N, batch) && split_rows_supported(H, I, KpH, KpI) &&
                      m->layers[0].o.qk.p && mlp_common;
   // the fused QKV kernel's input rows K-blocked (the weight rows then stay
   // in LDS): written so by the embedding LayerNorm and by the MLP kernel of
@@ -676,7 +662,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
                       m->layers[0].qkv.qk.p;
 
   // short sequences: QKV, Attn8.Prepare and attention in one kernel
-  const bool short_seqs = !tune.fixed() && kblock && short_attn_picked(KpH, T, B * nh, defer != nullptr);
+  const bool short_seqs = !tune.fixed() && kblock && short_attn_picked(KpH, T, B * nh, batch > N);
 
   int rc;
   std::vector<int32_t> groups;
@@ -1147,7 +1133,7 @@ int forward_split(ixh_model *m, const Tuning &tune, const HeadSet *hs, Workspace
                   const int32_t *offs, int B, const Outputs &out) {
   const int N = offs[B];
   const int P = std::min(nextra + 1, B);
-  if (P < 2 || N < kSplitTokens) return forward(m, tune, hs, w, st, d_ids, offs, B, out);
+  if (P < 2 || N < kSplitTokens) return forward(m, tune, hs, w, st, d_ids, offs, B, out, N);
   // part p covers sequences [cut[p], cut[p+1]): the first starting at or
   // past p*N/P
   std::vector<int> cut;
@@ -1174,7 +1160,7 @@ int forward_split(ixh_model *m, const Tuning &tune, const HeadSet *hs, Workspace
     offp[p].resize(b1 - b0 + 1);
     for (int b = b0; b <= b1; b++) offp[p][b - b0] = offs[b] - offs[b0];
     const int r = forward(m, tune, hs, wp, sp, d_ids + offs[b0], offp[p].data(), b1 - b0,
-                          out.at(b0, offs[b0], H, hs->rp, hs->rt), &pend[p]);
+                          out.at(b0, offs[b0], H, hs->rp, hs->rt), N, &pend[p]);
     if (r && !rc) rc = r;
   }
   // st waits for every part whatever happened, so nothing is left queued

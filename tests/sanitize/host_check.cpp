@@ -671,6 +671,26 @@ static void check_batcher() {
   }
 }
 
+// The kernels of few rows: alone up to the row counts where they win, beside
+// another part of a batch by the rows of all parts.
+void check_rows_picked() {
+  const struct {
+    int H, alone, mlp32;
+  } w[] = {{768, 3072, 10240}, {384, 4096, 14336}, {256, 2048, 14336}};
+  for (const auto &c : w) {
+    CHECK(ixh::split_rows_picked(c.H, 1, 1) && ixh::split_rows_picked(c.H, c.alone, c.alone), "split rows %d", c.H);
+    CHECK(!ixh::split_rows_picked(c.H, c.alone + 1, c.alone + 1), "split rows %d: past the bound", c.H);
+    const bool two = c.H == 384;  // the width at which they also win beside a part
+    CHECK(ixh::split_rows_picked(c.H, 2048, 4096) == two, "split rows %d: in two parts", c.H);
+    CHECK(ixh::split_rows_picked(c.H, 1536, 4608) == two, "split rows %d: in three", c.H);
+    CHECK(!ixh::split_rows_picked(c.H, 1535, 4608) && !ixh::split_rows_picked(c.H, 2305, 4609), "split rows %d: beside", c.H);
+    CHECK(ixh::mlp32_picked(c.H, 8192, 8192) && !ixh::mlp32_picked(c.H, 8193, 8193), "32-row MLP %d: alone", c.H);
+    CHECK(ixh::mlp32_picked(c.H, c.mlp32 / 2, c.mlp32) && !ixh::mlp32_picked(c.H, 1, c.mlp32 + 1) &&
+              !ixh::mlp32_picked(c.H, 8193, 8200),
+          "32-row MLP %d: beside", c.H);
+  }
+}
+
 int main(int argc, char **argv) {
   if (argc < 3) {
     fprintf(stderr, "usage: host_check <tokenizer.json> <scratch dir>\n");
@@ -682,6 +702,7 @@ int main(int argc, char **argv) {
   check_options();
   check_passes();
   check_groups();
+  check_rows_picked();
   check_free_list();
   check_keep_pool();
   check_per_device();

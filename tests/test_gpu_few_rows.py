@@ -115,6 +115,30 @@ def test_short_sequences_in_parts():
     gpu.close()
 
 
+@pytest.mark.parametrize("shape", ["base", "bekko", "small"])
+def test_rows_in_parts(shape):
+    """A batch run as two parts, which share the CUs: the products cut by output
+    channel only at hidden 384 and up to 4,608 rows in all, by the kernels that
+    ran; with the same bits as the options' kernels either side of that and of
+    the rule of the 32-row MLP kernel."""
+    cfg = SHAPES[shape](layers=2)
+    gpu = Model(Weights.random(cfg, seed=105))
+    rng = np.random.default_rng(105)
+    gpu.set_option("parts", 2)
+    for rows in (4096, 4608, 4609, 10240, 10241, 14336, 14337):
+        batch = seqs_of(rng, cfg.vocab, *[256] * (rows // 256), rows % 256)
+        gpu.set_profiling(True)
+        got = gpu.encode_seqs(batch)
+        ran = set(gpu.profile())
+        gpu.set_profiling(False)
+        assert ("gemm_womlp" in ran) == (shape == "bekko" and rows <= 4608), (rows, ran)
+        gpu.set_option("few_rows", 0)
+        want = gpu.encode_seqs(batch)
+        gpu.set_option("few_rows", 1)
+        assert f32_bits_equal(got, want), (rows, mismatch_report(got, want))
+    gpu.close()
+
+
 @pytest.mark.parametrize("shape,window", [("small", 128), ("bekko", 30)])
 def test_shared_keys_exact(shape, window):
     """Attention with 1, 2 and 4 waves on a query block's keys
