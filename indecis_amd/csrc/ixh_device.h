@@ -46,6 +46,10 @@ __device__ __forceinline__ float rne(float v) { return __builtin_rintf(v); }
 
 // RNE(x * inv) as int8 (QuantizeRow / quantRowAVX2 / quantColsAVX2).
 __device__ __forceinline__ int q8(float x, float inv) { return (int)rne(x * inv); }
+// four of them as a dword
+__device__ __forceinline__ int pack4(const float4 v, float inv) {
+  return (q8(v.x, inv) & 0xff) | ((q8(v.y, inv) & 0xff) << 8) | ((q8(v.z, inv) & 0xff) << 16) | (q8(v.w, inv) << 24);
+}
 
 // exp32 (linalg/fastmath.go:36-52): separate roundings.
 __device__ __forceinline__ float exp32_scalar(float x) {

@@ -35,10 +35,6 @@ constexpr int D = 64, NXCD = 8;
 constexpr int FLD = 68;  // floats a row of the float32 Q and K
 constexpr int BLD = 80;  // bytes a row of the int8 Q and K
 
-__device__ __forceinline__ int pack4(const float4 v, float inv) {
-  return (q8(v.x, inv) & 0xff) | ((q8(v.y, inv) & 0xff) << 8) | ((q8(v.z, inv) & 0xff) << 16) | (q8(v.w, inv) << 24);
-}
-
 template <int RT>
 struct Shape {
   static constexpr int KS = 4 / RT;            // waves sharing a row block's depth

@@ -56,10 +56,6 @@ constexpr int NXCD = 8;
 // channel 16*(lane/32) + r of the tile (mlp_block.hip)
 __device__ __forceinline__ int perm32(int i) { return 16 * ((i >> 2) & 1) + 4 * (i >> 3) + (i & 3); }
 
-__device__ __forceinline__ int pack4(const float4 v, float inv) {
-  return (q8(v.x, inv) & 0xff) | ((q8(v.y, inv) & 0xff) << 8) | ((q8(v.z, inv) & 0xff) << 16) | (q8(v.w, inv) << 24);
-}
-
 // Row blocks from which the kernels are arranged for many rows (512 rows):
 // measured with 4 waves a tile and the tiles dealt to the XCDs, then 2 waves
 // a tile, 4 tiles a workgroup (res) and the row blocks dealt to the XCDs, us
