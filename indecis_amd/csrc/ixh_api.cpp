@@ -302,7 +302,7 @@ struct ixh_model {
 
 // Stream and device buffers of one linear call (ixh_matmul8,
 // ixh_matmul8_outliers, ixh_linear8), kept between calls: created per call, a
-// call of 784 x 3,072 rows took 823 us, with them 642.
+// call of 784 x 3,072 rows took 823 us, with them 648.
 struct LinWs {
   hipStream_t stream = nullptr;
   DevBuf a, rest, q, sa, c, colmax, cols, w, bias;

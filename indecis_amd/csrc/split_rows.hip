@@ -29,10 +29,10 @@
 //      for the fewest rows.
 //
 // What bounds them: latency at few rows. At 24 rows of hidden 768 (36 and 24
-// workgroups) a launch takes 4.9 us (Wi; 8.0 with its LayerNorm), 5.1 us (Wo)
-// and 6.4 us (WoMLP), a LayerNorm of its own (ln_rows_kernel, rownorm.hip) 4.8:
+// workgroups) a launch takes 4.9 us (Wi; 7.9 with its LayerNorm), 4.5 us (Wo)
+// and 5.9 us (WoMLP), a LayerNorm of its own (ln_rows_kernel, rownorm.hip) 4.8:
 // against 25 us (Wo + LayerNorm) and 50 us (the MLP block) on the whole-row
-// kernels, and 2.05 -> 0.93 ms a pass of 22 layers. A wave's
+// kernels; a pass of 22 layers 2.07 -> 0.74 ms with short_attn.hip. A wave's
 // global loads are all issued before its first MFMA. With more rows, the
 // float32 rows read from L2 and the last-level cache by every tile's
 // workgroup: at 4,096 rows WoMLP took 69 us, Wo 47, Wi 26 before
