@@ -152,31 +152,43 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
 // one at hidden 768 and 256) over one on these: hidden 768 1.75 (1.49) at 1,024
 // rows, 1.40 (1.20) at 2,048, 1.17 (1.00) at 3,072, 1.10 (0.94) at 4,096; 384
 // 1.37 at 2,048, 1.08 at 4,096, 0.91 at 6,144; 256 1.20 (1.06) at 2,048, 1.10
-// (0.98) at 2,560. Beside another part, whose workgroups fill those CUs too, it
-// loses from the smallest batch that is split (4,096 rows) on, but at 384 in two
-// or three parts: us a pass of 8 layers (6 at 256) in two parts of sequences of
-// 512, on these, with the 32- and with the 64-row kernel: 768 1,147, 1,059 and
-// 1,196 at 4,096 rows, 1,389, 1,110 and 1,237 at 6,144; 256 606, 548 and 585 at
-// 4,096; 384 883 and (64) 916 at 4,096, 904 and 921 at 4,608, 931 and 924 at
-// 5,120, 1,085 and 938 at 8,192 (three parts 1,058 and 1,066 at 4,608, four
-// 1,217 and 1,198).
-bool split_rows_picked(int H, int N, int batch) {
-  if (batch > N) return H == 384 && batch <= 4608 && 3 * (int64_t)N >= batch;
-  return N <= (H == 768 ? 3072 : H == 384 ? 4096 : 2048);
+// (0.98) at 2,560.
+// In parts, whose workgroups fill the idle CUs too, it loses from the smallest
+// batch that is split (4,096 rows) on, but at 384 in two or three: us a pass of 8
+// layers (6 at 256) in two parts of sequences of 512, on these, with the 32- and
+// with the 64-row kernel: 768 1,147, 1,059 and 1,196 at 4,096 rows, 1,389, 1,110
+// and 1,237 at 6,144; 256 606, 548 and 585 at 4,096; 384 883 and (64) 916 at
+// 4,096, 904 and 921 at 4,608, 931 and 924 at 5,120, 1,085 and 938 at 8,192
+// (three parts 1,058 and 1,066 at 4,608, four 1,217 and 1,198). A part of few
+// rows, beside one of many, gains as it does alone.
+// Beside the passes of other threads: us a call of 6 layers on these and with
+// the better whole-row kernel, sequences of 256. 768, two threads of 1,536 rows
+// 291 and 324, of 2,048 335 and 330; four of 768 158 and 176, of 1,024 177 and 182,
+// of 1,536 219 and 186; eight (four run at a time) of 512 137 and 169, of 1,024 178
+// and 181, of 1,536 220 and 183. 384, two of 2,048 243 and 283, of 3,072 319 and
+// 319; four of 1,536 142 and 152, of 2,048 162 and 155; eight 147 and 156, 166 and
+// 153. 256, two of 1,536 193 and 198, of 2,048 199 and 191; four of 512 99 and 99,
+// of 768 104 and 104, of 1,024 106 and 102; eight of 512 93 and 93, of 1,024 99 and 96.
+bool split_rows_picked(int H, int N, int64_t batch, bool parts) {
+  if (N > (H == 768 ? 3072 : H == 384 ? 4096 : 2048)) return false;
+  if (batch <= N) return true;
+  if (parts) return N <= 512 || (H == 384 && batch <= 4608 && 3 * (int64_t)N >= batch);
+  return N <= (H == 768 ? 1024 : H == 384 ? 1536 : 512) || batch <= (H == 768 ? 4095 : H == 384 ? 6144 : 3072);
 }
 
 // Alone, up to one round of the 256 CUs, where 64 rows a workgroup leave half of
 // them idle. Hidden 768: 2.51 against 2.89 ms a pass at 6,144 rows, 2.90 against
 // 3.18 at 8,192 (38 against 52 us a launch); past one round a 32-row block costs
 // as much as a 64-row one. 256: a launch 12.9 against 19.1 us at 2,560 rows, 13.5
-// and 19.3 at 4,096, 15.0 and 19.7 at 8,192. Beside another part the CUs are
-// shared: us a pass in two parts as above with the 32- and the 64-row kernel,
-// sequences of 160 and of 512, 768 1,381 and 1,401, 1,474 and 1,469 at 10,240
-// rows, 1,581 and 1,542, 1,594 and 1,581 at 12,288, 1,977 and 1,887, 1,865 and
-// 1,744 at 16,384; 256 631 and 656, 638 and 661 at 14,336, 671 and 683, 662 and
-// 678 (1,024: 939 and 915) at 16,384.
-bool mlp32_picked(int H, int N, int batch) {
-  return N <= 8192 && (batch <= N || batch <= (H == 768 ? 10240 : 14336));
+// and 19.3 at 4,096, 15.0 and 19.7 at 8,192. Beside others the CUs are shared: us
+// a pass in two parts as above with the 32- and the 64-row kernel, sequences of
+// 160 and of 512, 768 1,381 and 1,401, 1,474 and 1,469 at 10,240 rows, 1,581 and
+// 1,542, 1,594 and 1,581 at 12,288, 1,977 and 1,887, 1,865 and 1,744 at 16,384; 256
+// 631 and 656, 638 and 661 at 14,336, 671 and 683, 662 and 678 (1,024: 939 and 915)
+// at 16,384. Threads, as above: 768, eight of 1,536 rows 183 and 201, of 2,048 199
+// and 207, of 3,072 271 and 261; 256, eight of 3,072 126 and 131.
+bool mlp32_picked(int H, int N, int64_t batch) {
+  return N <= (H == 768 ? 2048 : 3072) || (N <= 8192 && (batch <= N || batch <= (H == 768 ? 10240 : 14336)));
 }
 
 // Rows do not depend on their batch (TestMatMul8RowsIndependent), so the

@@ -77,13 +77,13 @@ int plan_passes(const Tuning &t, int H, int I, const int32_t *offs, int B, std::
 // empty). cut has P+1 entries, cut[0] 0 and cut[P] B.
 void split_points(const int32_t *offs, int B, int P, std::vector<int> &cut);
 
-// The kernels of a pass of N rows at width H, beside the other parts of a
-// batch of `batch` rows (N: alone), which keep the CUs busy that a few
-// workgroups leave idle. Whether its Wo and MLP run cut by output channel
-// (split_rows.hip), and if not, whether its MLP runs 32 rows a workgroup
-// (mlp_res.hip) instead of 64.
-bool split_rows_picked(int H, int N, int batch);
-bool mlp32_picked(int H, int N, int batch);
+// The kernels of a pass of N rows at width H while passes and parts of `batch`
+// rows run in all (N: alone), which keep the CUs busy that few workgroups leave
+// idle; parts: it is a part of a batch, whose parts run the same kernels in step.
+// Whether its Wo and MLP run cut by output channel (split_rows.hip), and if
+// not, whether its MLP runs 32 rows a workgroup (mlp_res.hip) instead of 64.
+bool split_rows_picked(int H, int N, int64_t batch, bool parts);
+bool mlp32_picked(int H, int N, int64_t batch);
 
 // The fused QKV kernel's workgroups of 8 waves, kQkvGroup integers each: slot
 // s < 16 (wave w computes slots w and w + 8) is the four at 4 s: its sequence

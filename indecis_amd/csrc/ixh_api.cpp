@@ -288,6 +288,7 @@ struct ixh_model {
   std::shared_ptr<HeadSet> heads;  // null: none set
   std::vector<std::shared_ptr<DevBuf>> rope_graveyard;
   FreeList<Workspace> pool;
+  std::atomic<int64_t> rows_now{0};  // of the passes that run at this moment
   std::atomic<bool> weights_valid{true};
   std::mutex tune_mu;
   Tuning tuning;
@@ -593,11 +594,11 @@ struct Pending {
 };
 
 // The forward pass. ids/out are device pointers here. batch: the rows of all
-// the parts that run at once, this one's among them. With `defer` the launches
+// the passes and parts of the handle that run at once, this one's among them. With `defer` the launches
 // are only issued: the caller synchronises the stream, then calls
 // defer->prof->flush().
 int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w, hipStream_t st,
-            const int32_t *d_ids, const int32_t *offs, int B, const Outputs &out, int batch,
+            const int32_t *d_ids, const int32_t *offs, int B, const Outputs &out, int64_t batch,
             Pending *defer = nullptr) {
   // an error left by a call outside this pass (the caller's, or one this
   // library already reported) is not this pass's launch failure
@@ -652,9 +653,11 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
                          mlp_block_supported(H, I, KpH, KpI, m->layers[0].i.np);
   const bool fuse_mlp = mlp_block || (mlp_common && fuse_res && tune.fuse_mlp != 0 &&
                                       mlp_res_supported(H, I, KpH, KpI, m->layers[0].i.np));
-  // few rows: Wo and the MLP cut by output channel (split_rows.hip)
-  const bool split = !tune.fixed() && split_rows_picked(H, N, batch) && split_rows_supported(H, I, KpH, KpI) &&
-                     m->layers[0].o.qk.p && mlp_common;
+  // few rows: Wo and the MLP cut by output channel (split_rows.hip); its buffers
+  // also where only the passes beside this one keep it from that
+  const bool may_split = !tune.fixed() && split_rows_picked(H, N, N, false) && split_rows_supported(H, I, KpH, KpI) &&
+                         m->layers[0].o.qk.p && mlp_common;
+  const bool split = may_split && split_rows_picked(H, N, batch, defer != nullptr);
   // the fused QKV kernel's input rows K-blocked (the weight rows then stay
   // in LDS): written so by the embedding LayerNorm and by the MLP kernel of
   // each layer
@@ -662,7 +665,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
                       m->layers[0].qkv.qk.p;
 
   // short sequences: QKV, Attn8.Prepare and attention in one kernel
-  const bool short_seqs = !tune.fixed() && kblock && short_attn_picked(KpH, T, B * nh, batch > N);
+  const bool short_seqs = !tune.fixed() && kblock && short_attn_picked(KpH, T, B * nh, defer && batch > N);
 
   int rc;
   std::vector<int32_t> groups;
@@ -673,6 +676,12 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   // 20.0, 16 19.0 and 20.8 (9.9 and 14.8), 32 29.7 and 29.8, 64 (26 and 29),
   // 164 125 and 119.
   const int cus = device_cus();
+  // Beside passes of as many rows, the kernels with a LayerNorm inside, whose
+  // workgroups fill a CU, run on half a round of them at most: us a call of 6
+  // layers, 2 and 4 threads, with it inside and before: hidden 768, 192 rows (216
+  // workgroups in the Wi kernel) 182 and 167, 111 and 98; 16 rows 131 and 136, 76
+  // and 77; 504 of 24 a sequence (252 in attention's) 205 and 189, 133 and 122.
+  const int ln_wgs = batch >= 2 * (int64_t)N ? cus / 2 : cus;
   bool two_blocks = T > 256;
   if (kblock && !short_seqs) {
     const bool share = 3 * nh * B > 2 * cus;
@@ -686,14 +695,14 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
   if ((rc = w->tabs.ensure(4 * ntab)) || (rc = w->pos.ensure(4 * (size_t)N)) ||
       (rc = w->x.ensure(4 * (size_t)N * H)) || (rc = w->xn.ensure(4 * (size_t)N * H)) ||
       (!fused && (rc = w->qkv.ensure(4 * (size_t)N * 3 * H))) || (rc = w->xq.ensure((size_t)N * ldq)) ||
-      ((kblock || split) && (rc = w->xqk.ensure((size_t)N * KpH))) ||
+      ((kblock || may_split) && (rc = w->xqk.ensure((size_t)N * KpH))) ||
       (rc = w->sa.ensure(4 * (size_t)N)) || (rc = w->qq.ensure((size_t)N * H)) ||
       (rc = w->sq.ensure(4 * (size_t)N * nh)) || (rc = w->kp.ensure((size_t)nh * Npad * D)) ||
       (rc = w->ks.ensure(4 * (size_t)nh * Npad)) || (rc = w->vt.ensure((size_t)nh * D * Npad)) ||
       (rc = w->vs.ensure(3 * 4 * (size_t)B * nh * D)) || (rc = w->ctx.ensure(4 * (size_t)N * H)) ||
-      ((!fuse_mlp || split) && (rc = w->g.ensure(4 * (size_t)N * I))) ||
-      ((stream_ctx || split) && (rc = w->cmax.ensure(4 * (size_t)N * nh))) ||
-      ((stream_ctx || split) && (rc = w->gmax.ensure(4 * (size_t)N * (I / 32)))))
+      ((!fuse_mlp || may_split) && (rc = w->g.ensure(4 * (size_t)N * I))) ||
+      ((stream_ctx || may_split) && (rc = w->cmax.ensure(4 * (size_t)N * nh))) ||
+      ((stream_ctx || may_split) && (rc = w->gmax.ensure(4 * (size_t)N * (I / 32)))))
     return rc;
 
   // small host-built tables through pinned memory, one copy
@@ -967,7 +976,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
           launch_res_split(product(L.o, w->ctx.as<float>(), H, cmax, nh, w->x.as<float>(), H, H), st));
       float *const gm = w->gmax.as<float>();
       SplitArgs wi = product(L.i, w->x.as<float>(), H, gm, I / 32, w->g.as<float>(), I, 2 * I);
-      if (ln_wi_split_supported(I, N, cus)) {
+      if (ln_wi_split_supported(I, N, ln_wgs)) {
         wi.gamma = lr.gamma;
         wi.eps = lr.eps;
         wi.lanes = lr.lanes;
@@ -978,7 +987,7 @@ int forward(ixh_model *m, const Tuning &tune, const HeadSet *heads, Workspace *w
       }
       RUN("gemm_womlp", 2 * dN * dH * dI, res_bytes(dI, false),
           launch_res_split(product(L.omlp, w->g.as<float>(), I, gm, I / 32, w->x.as<float>(), H, H), st));
-      if (l + 1 < c.layers && short_seqs && short_attn_ln_supported(T, B * nh)) {
+      if (l + 1 < c.layers && short_seqs && B * nh <= ln_wgs && short_attn_ln_supported(T, B * nh)) {
         short_ln = {w->x.as<float>(), m->layers[l + 1].attn_norm.as<float>(), lr.eps, lr.lanes};
         ln_done = true;
       } else if (l + 1 < c.layers) {
@@ -1133,7 +1142,16 @@ int forward_split(ixh_model *m, const Tuning &tune, const HeadSet *hs, Workspace
                   const int32_t *offs, int B, const Outputs &out) {
   const int N = offs[B];
   const int P = std::min(nextra + 1, B);
-  if (P < 2 || N < kSplitTokens) return forward(m, tune, hs, w, st, d_ids, offs, B, out, N);
+  // this pass's rows among those that run at once, until st has run it (every
+  // return below follows that wait, or a failure)
+  struct Rows {
+    ixh_model *m;
+    const int N;
+    const int64_t now;
+    Rows(ixh_model *m, int N) : m(m), N(N), now(m->rows_now.fetch_add(N) + N) {}
+    ~Rows() { m->rows_now -= N; }
+  } rows(m, N);
+  if (P < 2 || N < kSplitTokens) return forward(m, tune, hs, w, st, d_ids, offs, B, out, rows.now);
   // part p covers sequences [cut[p], cut[p+1]): the first starting at or
   // past p*N/P
   std::vector<int> cut;
@@ -1160,7 +1178,7 @@ int forward_split(ixh_model *m, const Tuning &tune, const HeadSet *hs, Workspace
     offp[p].resize(b1 - b0 + 1);
     for (int b = b0; b <= b1; b++) offp[p][b - b0] = offs[b] - offs[b0];
     const int r = forward(m, tune, hs, wp, sp, d_ids + offs[b0], offp[p].data(), b1 - b0,
-                          out.at(b0, offs[b0], H, hs->rp, hs->rt), N, &pend[p]);
+                          out.at(b0, offs[b0], H, hs->rp, hs->rt), rows.now, &pend[p]);
     if (r && !rc) rc = r;
   }
   // st waits for every part whatever happened, so nothing is left queued

@@ -672,21 +672,31 @@ static void check_batcher() {
 }
 
 // The kernels of few rows: alone up to the row counts where they win, beside
-// another part of a batch by the rows of all parts.
+// other parts or passes by the rows of all.
 void check_rows_picked() {
   const struct {
-    int H, alone, mlp32;
-  } w[] = {{768, 3072, 10240}, {384, 4096, 14336}, {256, 2048, 14336}};
+    int H, alone, few, all, few32, all32;
+  } w[] = {{768, 3072, 1024, 4095, 2048, 10240}, {384, 4096, 1536, 6144, 3072, 14336}, {256, 2048, 512, 3072, 3072, 14336}};
+  const int64_t many = (int64_t)1 << 40;
+  using ixh::mlp32_picked;
+  using ixh::split_rows_picked;
   for (const auto &c : w) {
-    CHECK(ixh::split_rows_picked(c.H, 1, 1) && ixh::split_rows_picked(c.H, c.alone, c.alone), "split rows %d", c.H);
-    CHECK(!ixh::split_rows_picked(c.H, c.alone + 1, c.alone + 1), "split rows %d: past the bound", c.H);
+    for (bool parts : {false, true}) {
+      CHECK(split_rows_picked(c.H, 1, 1, parts) && split_rows_picked(c.H, c.alone, c.alone, parts), "split rows %d", c.H);
+      CHECK(!split_rows_picked(c.H, c.alone + 1, c.alone + 1, parts), "split rows %d: past the bound", c.H);
+      CHECK(!split_rows_picked(c.H, c.alone + 1, c.alone + 2, parts), "split rows %d: past the bound, beside", c.H);
+    }
+    CHECK(split_rows_picked(c.H, c.few, many, false) && !split_rows_picked(c.H, c.few + 1, many, false), "split rows %d: few", c.H);
+    CHECK(split_rows_picked(c.H, c.few + 1, c.all, false) && !split_rows_picked(c.H, c.few + 1, c.all + 1, false),
+          "split rows %d: beside passes", c.H);
     const bool two = c.H == 384;  // the width at which they also win beside a part
-    CHECK(ixh::split_rows_picked(c.H, 2048, 4096) == two, "split rows %d: in two parts", c.H);
-    CHECK(ixh::split_rows_picked(c.H, 1536, 4608) == two, "split rows %d: in three", c.H);
-    CHECK(!ixh::split_rows_picked(c.H, 1535, 4608) && !ixh::split_rows_picked(c.H, 2305, 4609), "split rows %d: beside", c.H);
-    CHECK(ixh::mlp32_picked(c.H, 8192, 8192) && !ixh::mlp32_picked(c.H, 8193, 8193), "32-row MLP %d: alone", c.H);
-    CHECK(ixh::mlp32_picked(c.H, c.mlp32 / 2, c.mlp32) && !ixh::mlp32_picked(c.H, 1, c.mlp32 + 1) &&
-              !ixh::mlp32_picked(c.H, 8193, 8200),
+    CHECK(split_rows_picked(c.H, 2048, 4096, true) == two, "split rows %d: in two parts", c.H);
+    CHECK(split_rows_picked(c.H, 1536, 4608, true) == two, "split rows %d: in three", c.H);
+    CHECK(!split_rows_picked(c.H, 1535, 4608, true) && !split_rows_picked(c.H, 2305, 4609, true), "split rows %d: beside", c.H);
+    CHECK(split_rows_picked(c.H, 512, many, true) && !split_rows_picked(c.H, 513, many, true), "split rows %d: a small part", c.H);
+    CHECK(mlp32_picked(c.H, 8192, 8192) && !mlp32_picked(c.H, 8193, 8193), "32-row MLP %d: alone", c.H);
+    CHECK(mlp32_picked(c.H, c.few32, many) && !mlp32_picked(c.H, c.few32 + 1, many), "32-row MLP %d: few", c.H);
+    CHECK(mlp32_picked(c.H, c.all32 / 2, c.all32) && !mlp32_picked(c.H, c.all32 / 2, c.all32 + 1) && !mlp32_picked(c.H, 8193, 8200),
           "32-row MLP %d: beside", c.H);
   }
 }

@@ -1,6 +1,8 @@
 """GPU parity of the encoder on batches of few rows, whose Wo and MLP
 products run cut by output channel (split_rows.hip), against the CPU
 oracle, bit for bit."""
+import concurrent.futures as cf
+
 import numpy as np
 import pytest
 
@@ -136,6 +138,32 @@ def test_rows_in_parts(shape):
         want = gpu.encode_seqs(batch)
         gpu.set_option("few_rows", 1)
         assert f32_bits_equal(got, want), (rows, mismatch_report(got, want))
+    gpu.close()
+
+
+@pytest.mark.parametrize("shape", ["base", "small"])
+def test_rows_beside_threads(shape):
+    """Threads calling one handle, whose passes share the CUs and so pick other
+    kernels than alone (whole rows for passes of some thousand rows), by the
+    kernels that ran; with the bits of calls one at a time, and the kernels of a
+    call alone afterwards."""
+    cfg = SHAPES[shape](layers=2)
+    gpu = Model(Weights.random(cfg, seed=106))
+    rng = np.random.default_rng(106)
+    gpu.set_option("parts", 1)
+    batches = [seqs_of(rng, cfg.vocab, *lens) for lens in
+               ([256] * 8, [200] * 10, [16, 24] * 12, [64] * 3, [15], [256] * 7 + [255], [33] * 20, [2000])]
+    gpu.set_profiling(True)
+    want = [gpu.encode_seqs(b) for b in batches]
+    assert "mlp_ln" not in gpu.profile()
+    gpu.set_profiling(True)
+    with cf.ThreadPoolExecutor(len(batches)) as ex:
+        for b, e, got in zip(batches, want, ex.map(lambda b: [gpu.encode_seqs(b) for _ in range(12)], batches)):
+            assert all(f32_bits_equal(g, e) for g in got), [len(s) for s in b][:4]
+    assert "mlp_ln" in gpu.profile()
+    gpu.set_profiling(True)
+    gpu.encode_seqs(batches[3])
+    assert "ln_wi" in gpu.profile()
     gpu.close()
 
 
