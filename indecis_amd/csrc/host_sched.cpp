@@ -154,13 +154,14 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
 // 1.37 at 2,048, 1.08 at 4,096, 0.91 at 6,144; 256 1.20 (1.06) at 2,048, 1.10
 // (0.98) at 2,560.
 // In parts, whose workgroups fill the idle CUs too, it loses from the smallest
-// batch that is split (4,096 rows) on, but at 384 in two or three: us a pass of 8
-// layers (6 at 256) in two parts of sequences of 512, on these, with the 32- and
-// with the 64-row kernel: 768 1,147, 1,059 and 1,196 at 4,096 rows, 1,389, 1,110
-// and 1,237 at 6,144; 256 606, 548 and 585 at 4,096; 384 883 and (64) 916 at
-// 4,096, 904 and 921 at 4,608, 931 and 924 at 5,120, 1,085 and 938 at 8,192
-// (three parts 1,058 and 1,066 at 4,608, four 1,217 and 1,198). A part of few
-// rows, beside one of many, gains as it does alone.
+// batch that is split (4,096 rows) on, but at 384: us a pass of 8 layers (6 at
+// 256) in two parts of sequences of 512, on these, with the 32- and with the 64-row
+// kernel: 768 1,147, 1,059 and 1,196 at 4,096 rows, 1,389, 1,110 and 1,237 at
+// 6,144; 256 606, 548 and 585 at 4,096; 384 883 and (64) 916 at 4,096, 904 and 921
+// at 4,608, 931 and 924 at 5,120, 1,085 and 938 at 8,192 (three parts 1,058 and
+// 1,066 at 4,608, four 1,217 and 1,198). One sequence a part, 840 of 4,200 rows in
+// the second: 768 1,235 and 1,166, 256 843 and 806, 384 965 and 992 (of 5,000 1,031
+// and 1,034).
 // Beside the passes of other threads: us a call of 6 layers on these and with
 // the better whole-row kernel, sequences of 256. 768, two threads of 1,536 rows
 // 291 and 324, of 2,048 335 and 330; four of 768 158 and 176, of 1,024 177 and 182,
@@ -172,7 +173,7 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
 bool split_rows_picked(int H, int N, int64_t batch, bool parts) {
   if (N > (H == 768 ? 3072 : H == 384 ? 4096 : 2048)) return false;
   if (batch <= N) return true;
-  if (parts) return N <= 512 || (H == 384 && batch <= 4608 && 3 * (int64_t)N >= batch);
+  if (parts) return H == 384 && batch <= 5000;
   return N <= (H == 768 ? 1024 : H == 384 ? 1536 : 512) || batch <= (H == 768 ? 4095 : H == 384 ? 6144 : 3072);
 }
 

@@ -489,18 +489,24 @@ bool launch_kt(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStrea
 // 72.2. At most 128, 128 tokens: 768, 1 51.7 and 49.4, 8 (0.4) 63.1 and 61.2, 12
 // (0.6) 73.4 and 75.3, 21 (1) 90.6 and 97.2, 32 112 and 102; 384, 1 41.7 and 39.6,
 // 42 of 65-128 (1) 78.5 and 81.9; 256, 1 39.2 and 37.7, 64 (1) 53.4 and 55.8.
-// With another part's kernels beside this pass's (two parts a batch, the figure
-// of a part): at most 32 tokens, 32: 384, 3 rounds 121 and 125, 3.75 117 and 110;
-// 256, 3 81.2 and 88.1, 4 99.4 and 96.4; 64: 384, 1 94.8 and 100, 1.2 104 and 106,
-// 1.5 116 and 114; 256, 1.2 73.1 and 75.3, 1.6 85.3 and 81.8; 128: 768, 0.75 114
-// and 117, 1 145 and 151; 384, 0.4 84.4 and 85.4, 0.6 100 and 108; 256, 0.25 81.8 and
-// 84.5, 1 88.9 and 90.3.
+// With another part's kernels beside this pass's, us a pass of 6 layers in two
+// parts, on the two and on this kernel, by the rounds of a part: at most 32 tokens
+// (16; 32), 256, 3 618 and 564; 653 and 619, 5 748 and 727; 870 and 854, 6 833 and
+// 803; 965 and 977; 384, 2.5 (32) 732 and 728, 3 742 and 704; 749 and 770, 3.5 766 and
+// 793; 807 and 830; 768, 3 (32) 814 and 840, 4 901 and 934. At most 64 (33; 64): 256,
+// 1.5 557 and 530; 589 and 579, 1.75 589 and 561; 616 and 621; 384, 1.25 (64) 726 and
+// 700, 1.5 738 and 719; 723 and 738; 768, 1.5 (64) 796 and 815. At most 128 (128): 256,
+// 0.5 523 and 482, 1 641 and 644; 384, 0.5 689 and 653, 1 778 and 771, 1.25 838 and
+// 900; 768, 0.75 783 and 730, 1 863 and 866, 1.25 886 and 921.
 bool short_attn_picked(int Kp, int max_n, int workgroups, bool beside) {
   if (!short_attn_supported(Kp, max_n)) return false;
   const int wg = workgroups, cus = device_cus();
-  if (max_n <= 32) return wg <= (beside ? 3 : Kp == 256 ? 6 : 5) * cus;
+  if (max_n <= 32) {
+    if (beside) return 2 * wg <= (Kp == 256 ? 10 : Kp == 384 && max_n <= 16 ? 6 : 5) * cus;
+    return wg <= (Kp == 256 ? 6 : 5) * cus;
+  }
   if (max_n <= 64) {
-    if (beside) return 4 * wg <= 5 * cus;
+    if (beside) return 4 * wg <= (Kp == 256 ? 6 : 5) * cus;
     return wg <= cus || (wg <= 2 * cus && (Kp < 768 || 4 * wg > 7 * cus));
   }
   return wg <= cus && (beside || 2 * wg > cus);

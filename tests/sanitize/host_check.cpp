@@ -690,10 +690,8 @@ void check_rows_picked() {
     CHECK(split_rows_picked(c.H, c.few + 1, c.all, false) && !split_rows_picked(c.H, c.few + 1, c.all + 1, false),
           "split rows %d: beside passes", c.H);
     const bool two = c.H == 384;  // the width at which they also win beside a part
-    CHECK(split_rows_picked(c.H, 2048, 4096, true) == two, "split rows %d: in two parts", c.H);
-    CHECK(split_rows_picked(c.H, 1536, 4608, true) == two, "split rows %d: in three", c.H);
-    CHECK(!split_rows_picked(c.H, 1535, 4608, true) && !split_rows_picked(c.H, 2305, 4609, true), "split rows %d: beside", c.H);
-    CHECK(split_rows_picked(c.H, 512, many, true) && !split_rows_picked(c.H, 513, many, true), "split rows %d: a small part", c.H);
+    CHECK(split_rows_picked(c.H, 2048, 4096, true) == two && split_rows_picked(c.H, 1, 5000, true) == two, "split rows %d: parts", c.H);
+    CHECK(!split_rows_picked(c.H, 2500, 5001, true) && !split_rows_picked(c.H, 1, 5001, true), "split rows %d: past the bound, parts", c.H);
     CHECK(mlp32_picked(c.H, 8192, 8192) && !mlp32_picked(c.H, 8193, 8193), "32-row MLP %d: alone", c.H);
     CHECK(mlp32_picked(c.H, c.few32, many) && !mlp32_picked(c.H, c.few32 + 1, many), "32-row MLP %d: few", c.H);
     CHECK(mlp32_picked(c.H, c.all32 / 2, c.all32) && !mlp32_picked(c.H, c.all32 / 2, c.all32 + 1) && !mlp32_picked(c.H, 8193, 8200),

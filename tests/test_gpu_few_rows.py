@@ -97,43 +97,46 @@ def test_short_sequences_exact(shape, lanes, window, plant):
     gpu.close()
 
 
-def test_short_sequences_in_parts():
-    """A batch run as two parts: short_attn.hip up to three rounds a part of at
-    most 32 tokens, with the same bits as the other kernels."""
-    cfg = small_cfg(layers=2)
+@pytest.mark.parametrize("shape,tokens,seqs", [
+    ("small", 32, 640), ("small", 64, 192), ("bekko", 32, 212), ("bekko", 16, 256), ("base", 128, 42)])
+def test_short_sequences_in_parts(shape, tokens, seqs):
+    """A batch run as two parts: short_attn.hip up to `seqs` sequences of these
+    lengths (its rounds of the 256 CUs a part), with the same bits as the other
+    kernels."""
+    cfg = SHAPES[shape](layers=2)
     gpu = Model(Weights.random(cfg, seed=102))
     rng = np.random.default_rng(102)
     gpu.set_option("parts", 2)
-    for seqs, short in ((384, True), (386, False)):
-        batch = seqs_of(rng, cfg.vocab, *[32] * seqs)
+    for n, short in ((seqs, True), (seqs + 2, False)):
+        batch = seqs_of(rng, cfg.vocab, *[tokens] * n)
         gpu.set_profiling(True)
         got = gpu.encode_tokens(batch)
-        assert ("gemm_qkv" not in gpu.profile()) == short, seqs
+        assert ("gemm_qkv" not in gpu.profile()) == short, n
         gpu.set_profiling(False)
         gpu.set_option("few_rows", 0)
         want = gpu.encode_tokens(batch)
         gpu.set_option("few_rows", 1)
-        assert f32_bits_equal(got, want), (seqs, mismatch_report(got, want))
+        assert f32_bits_equal(got, want), (n, mismatch_report(got, want))
     gpu.close()
 
 
 @pytest.mark.parametrize("shape", ["base", "bekko", "small"])
 def test_rows_in_parts(shape):
     """A batch run as two parts, which share the CUs: the products cut by output
-    channel only at hidden 384 and up to 4,608 rows in all, by the kernels that
+    channel only at hidden 384 and up to 5,000 rows in all, by the kernels that
     ran; with the same bits as the options' kernels either side of that and of
     the rule of the 32-row MLP kernel."""
     cfg = SHAPES[shape](layers=2)
     gpu = Model(Weights.random(cfg, seed=105))
     rng = np.random.default_rng(105)
     gpu.set_option("parts", 2)
-    for rows in (4096, 4608, 4609, 10240, 10241, 14336, 14337):
+    for rows in (4096, 5000, 5001, 10240, 10241, 14336, 14337):
         batch = seqs_of(rng, cfg.vocab, *[256] * (rows // 256), rows % 256)
         gpu.set_profiling(True)
         got = gpu.encode_seqs(batch)
         ran = set(gpu.profile())
         gpu.set_profiling(False)
-        assert ("gemm_womlp" in ran) == (shape == "bekko" and rows <= 4608), (rows, ran)
+        assert ("gemm_womlp" in ran) == (shape == "bekko" and rows <= 5000), (rows, ran)
         gpu.set_option("few_rows", 0)
         want = gpu.encode_seqs(batch)
         gpu.set_option("few_rows", 1)
