@@ -161,7 +161,12 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
 // at 4,608, 931 and 924 at 5,120, 1,085 and 938 at 8,192 (three parts 1,058 and
 // 1,066 at 4,608, four 1,217 and 1,198). One sequence a part, 840 of 4,200 rows in
 // the second: 768 1,235 and 1,166, 256 843 and 806, 384 965 and 992 (of 5,000 1,031
-// and 1,034).
+// and 1,034). At 384 the smaller of two parts runs on these past that, beside the
+// larger's whole-row kernels, other resources bound: both, the smaller alone and
+// none of two near halves of sequences of 512, 735, 679 and 745 at 5,120 rows, 860,
+// 732 and 749 at 8,192, (-) 890 and 800 at 10,240; with 0.4 of the rows in it
+// (-) 1,235 and 1,282 at 8,000, with 0.3 1,355 and 1,328 (three sequences, 0.29 of
+// 7,172: 22 layers, 3,510 and 3,800).
 // Beside the passes of other threads: us a call of 6 layers on these and with
 // the better whole-row kernel, sequences of 256. 768, two threads of 1,536 rows
 // 291 and 324, of 2,048 335 and 330; four of 768 158 and 176, of 1,024 177 and 182,
@@ -173,7 +178,7 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
 bool split_rows_picked(int H, int N, int64_t batch, bool parts) {
   if (N > (H == 768 ? 3072 : H == 384 ? 4096 : 2048)) return false;
   if (batch <= N) return true;
-  if (parts) return H == 384 && batch <= 5000;
+  if (parts) return H == 384 && (batch <= 5000 || (batch <= 8192 && 2 * (int64_t)N < batch && 4 * (int64_t)N > batch));
   return N <= (H == 768 ? 1024 : H == 384 ? 1536 : 512) || batch <= (H == 768 ? 4095 : H == 384 ? 6144 : 3072);
 }
 
@@ -186,10 +191,12 @@ bool split_rows_picked(int H, int N, int64_t batch, bool parts) {
 // 160 and of 512, 768 1,381 and 1,401, 1,474 and 1,469 at 10,240 rows, 1,581 and
 // 1,542, 1,594 and 1,581 at 12,288, 1,977 and 1,887, 1,865 and 1,744 at 16,384; 256
 // 631 and 656, 638 and 661 at 14,336, 671 and 683, 662 and 678 (1,024: 939 and 915)
-// at 16,384. Threads, as above: 768, eight of 1,536 rows 183 and 201, of 2,048 199
+// at 16,384. Ragged batches (20-512 to 500-3,000 tokens), the 32-row over the 64-row
+// kernel: 768 0.95-1.03 at 9,000-10,000 rows, 0.99-1.06 at 11,000-12,700; 256 0.95-0.98
+// at 15,000, 0.99-1.05 at 17,500. Threads, as above: 768, eight of 1,536 rows 183 and 201, of 2,048 199
 // and 207, of 3,072 271 and 261; 256, eight of 3,072 126 and 131.
 bool mlp32_picked(int H, int N, int64_t batch) {
-  return N <= (H == 768 ? 2048 : 3072) || (N <= 8192 && (batch <= N || batch <= (H == 768 ? 10240 : 14336)));
+  return N <= (H == 768 ? 2048 : 3072) || (N <= 8192 && (batch <= N || batch <= (H == 768 ? 10240 : 16384)));
 }
 
 // Rows do not depend on their batch (TestMatMul8RowsIndependent), so the

@@ -488,7 +488,11 @@ bool launch_kt(const GemmArgs &g, const AttnArgs &a, const ShortLn &ln, hipStrea
 // and 111); 256, 64 (1) 41.1 and 46.0, 128 (2) 52.1 and 52.5, 200 80.1 and
 // 72.2. At most 128, 128 tokens: 768, 1 51.7 and 49.4, 8 (0.4) 63.1 and 61.2, 12
 // (0.6) 73.4 and 75.3, 21 (1) 90.6 and 97.2, 32 112 and 102; 384, 1 41.7 and 39.6,
-// 42 of 65-128 (1) 78.5 and 81.9; 256, 1 39.2 and 37.7, 64 (1) 53.4 and 55.8.
+// 42 of 65-128 (1) 78.5 and 81.9; 256, 1 39.2 and 37.7, 64 (1) 53.4 and 55.8. This
+// kernel over the two, a pass of 6 layers at 65, 96 and 128 tokens: 768, 0.3 rounds
+// 0.99, 1.01 and 1.02, 0.4 0.99, 1.00 and 1.05, 0.5 0.92, 0.96 and 0.97; 384, 0.2
+// 0.97, 1.02 and 1.01, 0.3 0.94, 0.98 and 1.00, 0.4 0.94, 0.96 and 0.98; 256, 0.1 0.98,
+// 0.96 and 1.00, 0.2 0.97, 0.99 and 0.98, 0.5 0.93, 0.97 and 0.96.
 // With another part's kernels beside this pass's, us a pass of 6 layers in two
 // parts, on the two and on this kernel, by the rounds of a part: at most 32 tokens
 // (16; 32), 256, 3 618 and 564; 653 and 619, 5 748 and 727; 870 and 854, 6 833 and
@@ -509,7 +513,7 @@ bool short_attn_picked(int Kp, int max_n, int workgroups, bool beside) {
     if (beside) return 4 * wg <= (Kp == 256 ? 6 : 5) * cus;
     return wg <= cus || (wg <= 2 * cus && (Kp < 768 || 4 * wg > 7 * cus));
   }
-  return wg <= cus && (beside || 2 * wg > cus);
+  return wg <= cus && (beside || wg > (Kp == 768 ? 2 * cus / 5 : Kp == 384 ? cus / 4 : cus / 8));
 }
 
 bool short_attn_supported(int Kp, int max_n) { return (Kp == 768 || Kp == 384 || Kp == 256) && max_n <= 128; }

@@ -676,7 +676,7 @@ static void check_batcher() {
 void check_rows_picked() {
   const struct {
     int H, alone, few, all, few32, all32;
-  } w[] = {{768, 3072, 1024, 4095, 2048, 10240}, {384, 4096, 1536, 6144, 3072, 14336}, {256, 2048, 512, 3072, 3072, 14336}};
+  } w[] = {{768, 3072, 1024, 4095, 2048, 10240}, {384, 4096, 1536, 6144, 3072, 16384}, {256, 2048, 512, 3072, 3072, 16384}};
   const int64_t many = (int64_t)1 << 40;
   using ixh::mlp32_picked;
   using ixh::split_rows_picked;
@@ -691,7 +691,10 @@ void check_rows_picked() {
           "split rows %d: beside passes", c.H);
     const bool two = c.H == 384;  // the width at which they also win beside a part
     CHECK(split_rows_picked(c.H, 2048, 4096, true) == two && split_rows_picked(c.H, 1, 5000, true) == two, "split rows %d: parts", c.H);
-    CHECK(!split_rows_picked(c.H, 2500, 5001, true) && !split_rows_picked(c.H, 1, 5001, true), "split rows %d: past the bound, parts", c.H);
+    CHECK(!split_rows_picked(c.H, 2501, 5002, true) && !split_rows_picked(c.H, 1250, 5001, true), "split rows %d: past the bound, parts", c.H);
+    CHECK(c.H == 256 || (split_rows_picked(c.H, 2500, 5001, true) == two && split_rows_picked(c.H, 2049, 8192, true) == two),
+          "split rows %d: the smaller part", c.H);
+    CHECK(!split_rows_picked(c.H, 4096, 8192, true) && !split_rows_picked(c.H, 4000, 8193, true), "split rows %d: halves", c.H);
     CHECK(mlp32_picked(c.H, 8192, 8192) && !mlp32_picked(c.H, 8193, 8193), "32-row MLP %d: alone", c.H);
     CHECK(mlp32_picked(c.H, c.few32, many) && !mlp32_picked(c.H, c.few32 + 1, many), "32-row MLP %d: few", c.H);
     CHECK(mlp32_picked(c.H, c.all32 / 2, c.all32) && !mlp32_picked(c.H, c.all32 / 2, c.all32 + 1) && !mlp32_picked(c.H, 8193, 8200),

@@ -79,7 +79,7 @@ def test_short_sequences_exact(shape, lanes, window, plant):
     batches += [(24,), (25, 24, 3), (30,) + (2,) * (one - 1), (30,) + (2,) * one]
     picked = [None] * len(batches)
     # longest sequence, most (or, negative, one less than the fewest) sixteenths of a round
-    edges = [(32, 96 if shape == "small" else 80), (64, 32), (65, -8), (128, 16)]
+    edges = [(32, 96 if shape == "small" else 80), (64, 32), (65, {"base": -6, "bekko": -4, "small": -2}[shape]), (128, 16)]
     edges += [(33, 16), (64, -28)] if shape == "base" else []
     for n, most in edges:
         seqs = abs(most) * 16 // cfg.heads
@@ -123,20 +123,20 @@ def test_short_sequences_in_parts(shape, tokens, seqs):
 @pytest.mark.parametrize("shape", ["base", "bekko", "small"])
 def test_rows_in_parts(shape):
     """A batch run as two parts, which share the CUs: the products cut by output
-    channel only at hidden 384 and up to 5,000 rows in all, by the kernels that
-    ran; with the same bits as the options' kernels either side of that and of
+    channel only at hidden 384, up to 5,000 rows in all or in the smaller part
+    (not of equal ones) up to 8,192, by the kernels that ran; with the same bits as the options' kernels either side of that and of
     the rule of the 32-row MLP kernel."""
     cfg = SHAPES[shape](layers=2)
     gpu = Model(Weights.random(cfg, seed=105))
     rng = np.random.default_rng(105)
     gpu.set_option("parts", 2)
-    for rows in (4096, 5000, 5001, 10240, 10241, 14336, 14337):
+    for rows in (4096, 5000, 5001, 5120, 8191, 10240, 10241, 16384, 16385):
         batch = seqs_of(rng, cfg.vocab, *[256] * (rows // 256), rows % 256)
         gpu.set_profiling(True)
         got = gpu.encode_seqs(batch)
         ran = set(gpu.profile())
         gpu.set_profiling(False)
-        assert ("gemm_womlp" in ran) == (shape == "bekko" and rows <= 5000), (rows, ran)
+        assert ("gemm_womlp" in ran) == (shape == "bekko" and rows in (4096, 5000, 5001, 8191)), (rows, ran)
         gpu.set_option("few_rows", 0)
         want = gpu.encode_seqs(batch)
         gpu.set_option("few_rows", 1)
