@@ -166,7 +166,9 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
 // none of two near halves of sequences of 512, 735, 679 and 745 at 5,120 rows, 860,
 // 732 and 749 at 8,192, (-) 890 and 800 at 10,240; with 0.4 of the rows in it
 // (-) 1,235 and 1,282 at 8,000, with 0.3 1,355 and 1,328 (three sequences, 0.29 of
-// 7,172: 22 layers, 3,510 and 3,800).
+// 7,172: 22 layers, 3,510 and 3,800). At 768 the same up to 2,304 rows in it: 130
+// ragged batches of 4,131-6,453 rows, the smaller part alone over none 0.92-1.06,
+// 0.98 in the mean up to there and 1.03 past it; at 256 it loses always.
 // Beside the passes of other threads: us a call of 6 layers on these and with
 // the better whole-row kernel, sequences of 256. 768, two threads of 1,536 rows
 // 291 and 324, of 2,048 335 and 330; four of 768 158 and 176, of 1,024 177 and 182,
@@ -178,7 +180,10 @@ void qkv_groups(const int32_t *offs, const int32_t *padoff, const std::vector<in
 bool split_rows_picked(int H, int N, int64_t batch, bool parts) {
   if (N > (H == 768 ? 3072 : H == 384 ? 4096 : 2048)) return false;
   if (batch <= N) return true;
-  if (parts) return H == 384 && (batch <= 5000 || (batch <= 8192 && 2 * (int64_t)N < batch && 4 * (int64_t)N > batch));
+  if (parts) {
+    const bool smaller = 2 * (int64_t)N < batch && 4 * (int64_t)N > batch;
+    return H == 384 ? batch <= 5000 || (batch <= 8192 && smaller) : H == 768 && N <= 2304 && smaller;
+  }
   return N <= (H == 768 ? 1024 : H == 384 ? 1536 : 512) || batch <= (H == 768 ? 4095 : H == 384 ? 6144 : 3072);
 }
 

@@ -689,10 +689,14 @@ void check_rows_picked() {
     CHECK(split_rows_picked(c.H, c.few, many, false) && !split_rows_picked(c.H, c.few + 1, many, false), "split rows %d: few", c.H);
     CHECK(split_rows_picked(c.H, c.few + 1, c.all, false) && !split_rows_picked(c.H, c.few + 1, c.all + 1, false),
           "split rows %d: beside passes", c.H);
-    const bool two = c.H == 384;  // the width at which they also win beside a part
+    const bool two = c.H == 384;  // the width at which they also win beside an equal part
     CHECK(split_rows_picked(c.H, 2048, 4096, true) == two && split_rows_picked(c.H, 1, 5000, true) == two, "split rows %d: parts", c.H);
+    CHECK(split_rows_picked(c.H, 1281, 5120, true) == (c.H != 256) && !split_rows_picked(c.H, 1280, 5120, true),
+          "split rows %d: a quarter", c.H);
+    CHECK(split_rows_picked(c.H, 2304, 6000, true) == (c.H != 256) && split_rows_picked(c.H, 2305, 6000, true) == two,
+          "split rows %d: the smaller part's rows", c.H);
     CHECK(!split_rows_picked(c.H, 2501, 5002, true) && !split_rows_picked(c.H, 1250, 5001, true), "split rows %d: past the bound, parts", c.H);
-    CHECK(c.H == 256 || (split_rows_picked(c.H, 2500, 5001, true) == two && split_rows_picked(c.H, 2049, 8192, true) == two),
+    CHECK(c.H == 256 || (split_rows_picked(c.H, 2500, 5001, true) == two && split_rows_picked(c.H, 2400, 8192, true) == two),
           "split rows %d: the smaller part", c.H);
     CHECK(!split_rows_picked(c.H, 4096, 8192, true) && !split_rows_picked(c.H, 4000, 8193, true), "split rows %d: halves", c.H);
     CHECK(mlp32_picked(c.H, 8192, 8192) && !mlp32_picked(c.H, 8193, 8193), "32-row MLP %d: alone", c.H);

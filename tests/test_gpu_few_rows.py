@@ -123,20 +123,21 @@ def test_short_sequences_in_parts(shape, tokens, seqs):
 @pytest.mark.parametrize("shape", ["base", "bekko", "small"])
 def test_rows_in_parts(shape):
     """A batch run as two parts, which share the CUs: the products cut by output
-    channel only at hidden 384, up to 5,000 rows in all or in the smaller part
-    (not of equal ones) up to 8,192, by the kernels that ran; with the same bits as the options' kernels either side of that and of
+    channel at hidden 384 up to 5,000 rows in all or in the smaller part (not of
+    equal ones) up to 8,192, at 768 in a smaller part of up to 2,304, by the kernels
+    that ran; with the same bits as the options' kernels either side of that and of
     the rule of the 32-row MLP kernel."""
     cfg = SHAPES[shape](layers=2)
     gpu = Model(Weights.random(cfg, seed=105))
     rng = np.random.default_rng(105)
     gpu.set_option("parts", 2)
-    for rows in (4096, 5000, 5001, 5120, 8191, 10240, 10241, 16384, 16385):
+    for rows in (4096, 4500, 5000, 5001, 5120, 8191, 10240, 10241, 16384, 16385):
         batch = seqs_of(rng, cfg.vocab, *[256] * (rows // 256), rows % 256)
         gpu.set_profiling(True)
         got = gpu.encode_seqs(batch)
         ran = set(gpu.profile())
         gpu.set_profiling(False)
-        assert ("gemm_womlp" in ran) == (shape == "bekko" and rows in (4096, 5000, 5001, 8191)), (rows, ran)
+        assert ("gemm_womlp" in ran) == (rows in {"bekko": (4096, 4500, 5000, 5001, 8191), "base": (4500,), "small": ()}[shape]), (rows, ran)
         gpu.set_option("few_rows", 0)
         want = gpu.encode_seqs(batch)
         gpu.set_option("few_rows", 1)
